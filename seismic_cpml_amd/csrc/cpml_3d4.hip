@@ -74,7 +74,7 @@ __global__ __launch_bounds__(BX *TY4) void k_stress3d4(Step3D<T> p) {
   const int i = c.i, j = c.j, nx = p.nx, ny = p.ny, nz = p.nz;
   const long ld = p.ld, ps = p.ps;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const long mxo = p.sx.s(i) + (long)p.sx.w * j, mxs = (long)p.sx.w * ny;
+  const long mxo = p.sx.at(i, j, ny), mxs = (long)p.sx.w * ny;
   const long myo = i + p.mld * p.sy.s(j), mys = p.mld * p.sy.w;
   const long mzo = i + p.mld * j, mzs = p.mld * ny;
   // loop ranges of 3D-visco:977-979, 1080-1082, 1141-1144, 1185-1186 (0-based)
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 6 : 1) void k_velocity3d4
   const int i = c.i, j = c.j, nx = p.nx, ny = p.ny, nz = p.nz;
   const long ld = p.ld, ps = p.ps;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const long mxo = p.sx.s(i) + (long)p.sx.w * j, mxs = (long)p.sx.w * ny;
+  const long mxo = p.sx.at(i, j, ny), mxs = (long)p.sx.w * ny;
   const long myo = i + p.mld * p.sy.s(j), mys = p.mld * p.sy.w;
   const long mzo = i + p.mld * j, mzs = p.mld * ny;
   // loop ranges of 3D-visco:1244-1246, 1266-1267, 1287-1289 (0-based)

@@ -1621,7 +1621,7 @@ int cpml_gpu_get_memory(cpml_solver *h, int which, void *out) {
         long src = -1;
         switch (kMemAxis[which]) {
           case 0:
-            if (h->sx.in(i)) src = h->sx.s(i) + (long)h->sx.w * (j + (long)ny * k);
+            if (h->sx.in(i)) src = h->sx.at(i, j, ny) + (long)h->sx.w * ny * k;
             break;
           case 1:
             if (h->sy.in(j)) src = i + h->mld * (h->sy.s(j) + (long)h->sy.w * k);
@@ -1751,7 +1751,7 @@ int cpml_gpu_set_memory(cpml_solver *h, int which, const void *in) {
         long dst = -1;
         switch (kMemAxis[which]) {
           case 0:
-            if (h->sx.in(i)) dst = h->sx.s(i) + (long)h->sx.w * (j + (long)ny * k);
+            if (h->sx.in(i)) dst = h->sx.at(i, j, ny) + (long)h->sx.w * ny * k;
             break;
           case 1:
             if (h->sy.in(j)) dst = i + h->mld * (h->sy.s(j) + (long)h->sy.w * k);
@@ -2097,10 +2097,11 @@ int cpml_gpu_set_time_block(cpml_solver *h, int steps, int strip_width, int chun
   h->tb = steps;
   // default strip: every lane the ring leaves (2D, measured fastest: 52 columns
   // at order 4 and 2 steps gave 79.4 Gcell/s against 75.7 for 48); 3D rounds
-  // it down to a multiple of 8 (56 and 48 measured alike)
+  // it down to whole 64-byte sectors, so no tile stores part of one
   const int widest = 64 - 2 * g;
+  const int sector = 64 / (int)h->esize;
   h->tb_ow = strip_width > 0 ? strip_width
-                             : (h->ndim == 3 ? std::max(8, widest / 8 * 8) : widest);
+                             : (h->ndim == 3 ? std::max(8, widest / sector * sector) : widest);
   if (h->tb_ow > widest) h->tb_ow = widest;
   h->tb_jc = jc;
   h->tb_rec_ow = -1;

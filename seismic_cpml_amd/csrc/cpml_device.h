@@ -55,6 +55,34 @@ __device__ __forceinline__ const __attribute__((address_space(4))) A *kernarg() 
   return q;
 }
 
+// x of the next / previous lane of the wavefront (0 past the ends): DPP wave
+// shifts by one lane, which the compiler folds into the instruction that uses
+// the value.
+template <int CTRL>
+__device__ __forceinline__ int dpp_shift(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_shift(float x) {
+  return __builtin_bit_cast(float, dpp_shift<CTRL>(__builtin_bit_cast(int, x)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift(double x) {
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  i32x2 v = __builtin_bit_cast(i32x2, x);
+  v.x = dpp_shift<CTRL>(v.x);
+  v.y = dpp_shift<CTRL>(v.y);
+  return __builtin_bit_cast(double, v);
+}
+template <typename T>
+__device__ __forceinline__ T lane_next(T x) {
+  return dpp_shift<0x130>(x);  // wave_shl:1
+}
+template <typename T>
+__device__ __forceinline__ T lane_prev(T x) {
+  return dpp_shift<0x138>(x);  // wave_shr:1
+}
+
 // Raw buffer resource over `bytes` bytes at p (gfx9 family word 3).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes,

@@ -254,7 +254,7 @@ __global__ __launch_bounds__(FW *(TY + 2)) void k_fused3d(Fused3D<T> P) {
     // axis, loaded before the next plane's loads so that waiting for them
     // does not wait for those
     const bool inz = Z && inside && p.sz.in(s), inzv = Z && dov && p.sz.in(kv);
-    const unsigned ox = p.sx.s(i) + (unsigned)p.sx.w * (j + (unsigned)ny * s);
+    const unsigned ox = (unsigned)p.sx.at(i, j, ny) + (unsigned)p.sx.w * (unsigned)ny * s;
     const unsigned oy = i + (unsigned)p.mld * (p.sy.s(j) + (unsigned)p.sy.w * s);
     const unsigned oz = i + (unsigned)p.mld * (j + (unsigned)ny * p.sz.s(s));
     const unsigned oxv = ox - (unsigned)p.sx.w * ny, oyv = oy - (unsigned)p.mld * p.sy.w;

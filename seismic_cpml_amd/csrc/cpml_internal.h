@@ -9,8 +9,9 @@
 //    stencils read neighbours without bounds tests.  The x halo is XPAD
 //    elements wide so that interior rows start 256-byte aligned.
 //  * C-PML memory variables: only inside the absorbing slabs.  Along x the
-//    slab is the columns [0, wl) U [nx-wr, nx) stored compactly as s in
-//    [0, wl+wr); along y and z likewise for rows and planes.  Outside the slab
+//    slab is the columns [0, wl) U [nx-wr, nx), per plane the rows of the min
+//    side and then those of the max side (Slab::at); along y and z the rows
+//    and planes of both sides are stored compactly as s in [0, wl+wr).  Outside the slab
 //    the reference's memory variable stays exactly 0 (a = 0) and K = 1, so
 //    the update reduces to the plain derivative there.
 #pragma once
@@ -41,10 +42,17 @@ constexpr double kStreamingBytes = 256.0 * 1024 * 1024;
 struct Slab {
   int wl = 0, wr = 0, w = 0;  // widths at the min and max side, total
   int n = 0;                  // grid extent along the axis
+  int k1 = 1;                 // K and K_half are 1 at every point (K_MAX_PML = 1)
   __host__ __device__ bool in(int i) const {
     return i >= 0 && i < n && (i < wl || i >= n - wr);
   }
   __host__ __device__ int s(int i) const { return i < wl ? i : i - (n - wr) + wl; }
+  // Element of (i, j) in one plane of an x-slab memory array of `rows` rows:
+  // the rows of the min side, then those of the max side, so each side's rows
+  // are contiguous (a tile touches one side, and whole cache lines of it).
+  __host__ __device__ long at(int i, long j, long rows) const {
+    return i < wl ? i + wl * j : wl * rows + (i - (n - wr)) + wr * j;
+  }
 };
 
 // Slab widths from one axis's profiles: a point belongs to the slab when any
@@ -54,7 +62,9 @@ template <typename T>
 inline void slab_from_profile(const T *a, const T *ah, const T *K, const T *Kh, int n, Slab &s) {
   const int half = (n + 1) / 2;
   int wl = 0, wr = 0;
+  s.k1 = 1;
   for (int i = 0; i < n; ++i) {
+    if (K[i] != T(1) || Kh[i] != T(1)) s.k1 = 0;
     const bool nz = a[i] != T(0) || ah[i] != T(0) || K[i] != T(1) || Kh[i] != T(1);
     if (!nz) continue;
     if (i < half) wl = i + 1 > wl ? i + 1 : wl;
@@ -77,7 +87,7 @@ template <typename T>
 struct Step2D {
   T *vx, *vy, *sxx, *syy, *sxy;  // interior origin (halo at negative offsets)
   const T *lam, *mu, *rho;
-  // x-slab memories: [0] dvx_dx [1] dvy_dx [2] dsxx_dx [3] dsxy_dx, index s + wx*j
+  // x-slab memories: [0] dvx_dx [1] dvy_dx [2] dsxx_dx [3] dsxy_dx, index sx.at(i, j, ny)
   T *mx[4];
   // y-slab memories: [0] dvy_dy [1] dvx_dy [2] dsxy_dy [3] dsyy_dy, index i + mld*s
   T *my[4];

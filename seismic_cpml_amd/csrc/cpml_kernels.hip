@@ -159,7 +159,7 @@ __global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p) {
   const auto rzz = g.rsrc(p.szz, p.base), rxy = g.rsrc(p.sxy, p.base);
   const auto rxz = g.rsrc(p.sxz, p.base), ryz = g.rsrc(p.syz, p.base);
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const unsigned mxo = p.sx.s(i) + (unsigned)p.sx.w * j, mxs = (unsigned)p.sx.w * ny;
+  const unsigned mxo = (unsigned)p.sx.at(i, j, ny), mxs = (unsigned)p.sx.w * ny;
   const unsigned myo = i + (unsigned)p.mld * p.sy.s(j), mys = (unsigned)p.mld * p.sy.w;
   const unsigned mzo = i + (unsigned)p.mld * j, mzs = (unsigned)p.mld * ny;
   const bool r_n = i <= nx - 2 && j >= 1;
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
   const auto rcb = g.rsrc(p.cbuoy, p.base);
   const auto rvx = g.rsrc(p.vx, p.base), rvy = g.rsrc(p.vy, p.base), rvz = g.rsrc(p.vz, p.base);
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const unsigned mxo = p.sx.s(i) + (unsigned)p.sx.w * j, mxs = (unsigned)p.sx.w * ny;
+  const unsigned mxo = (unsigned)p.sx.at(i, j, ny), mxs = (unsigned)p.sx.w * ny;
   const unsigned myo = i + (unsigned)p.mld * p.sy.s(j), mys = (unsigned)p.mld * p.sy.w;
   const unsigned mzo = i + (unsigned)p.mld * j, mzs = (unsigned)p.mld * ny;
   const bool r_vx = i >= 1 && j >= 1;

@@ -40,7 +40,7 @@ __device__ __forceinline__ void stress2d_point(const Step2D<T> &p, int i, int j)
   const long ld = p.ld;
   const long c = i + j * ld;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const long mxo = p.sx.s(i) + (long)p.sx.w * j;
+  const long mxo = p.sx.at(i, j, p.ny);
   const long myo = i + p.mld * p.sy.s(j);
   // sigma_xx, sigma_yy at (i+1/2, j), Fortran i=1..NX-1, j=2..NY
   if (i <= p.nx - 2 && j >= 1) {
@@ -76,7 +76,7 @@ __device__ __forceinline__ void velocity2d_point(const Step2D<T> &p, int i, int 
   const long ld = p.ld;
   const long c = i + j * ld;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const long mxo = p.sx.s(i) + (long)p.sx.w * j;
+  const long mxo = p.sx.at(i, j, p.ny);
   const long myo = i + p.mld * p.sy.s(j);
   T vxn = ld_once<NT>(p.vx + c), vyn = ld_once<NT>(p.vy + c);
   // vx at (i, j), Fortran i=2..NX, j=2..NY

@@ -109,7 +109,9 @@ __device__ __forceinline__ void tb2d_item(const TB2D<T> &P, int ts, int jb, int 
   auto xs = [&](T x, int k) { return k == 0 ? x : lane_of(x, a4[k + 4]); };
 
   const bool inx = SX && p.sx.in(i);
-  const int sxi = inx ? p.sx.s(i) : 0;
+  // element of this column in the x-slab arrays: sxi + sxw * row
+  const unsigned sxi = inx ? (unsigned)p.sx.at(i, 0, ny) : 0u;
+  const unsigned sxw = i < p.sx.wl ? p.sx.wl : p.sx.wr;
   T pxa = T(0), pxb = T(0), pxK = T(1), pxah = T(0), pxbh = T(0), pxKh = T(1);
   if (inx) {
     pxa = p.px.a[i], pxb = p.px.b[i], pxK = p.px.K[i];
@@ -185,12 +187,12 @@ __device__ __forceinline__ void tb2d_item(const TB2D<T> &P, int ts, int jb, int 
 #pragma unroll
       for (int q = 0; q < 4; ++q) L.px[q] = L.py[q] = T(0);
       if (SX && inx && row_in(s)) {
-        const long o = sxi + (long)p.sx.w * s;
+        const unsigned o = sxi + sxw * (unsigned)s;
         L.px[0] = p.mx[0][o];
         L.px[1] = p.mx[1][o];
       }
       if (SX && inx && row_in(jq)) {
-        const long o = sxi + (long)p.sx.w * jq;
+        const unsigned o = sxi + sxw * (unsigned)jq;
         L.px[2] = p.mx[2][o];
         L.px[3] = p.mx[3][o];
       }
@@ -317,7 +319,7 @@ __device__ __forceinline__ void tb2d_item(const TB2D<T> &P, int ts, int jb, int 
         P.sxy[c] = sxy;
         {
           if (SX && inx) {
-            const long o = sxi + (long)p.sx.w * pr;
+            const unsigned o = sxi + sxw * (unsigned)pr;
             P.mx[0][o] = npx0;
             P.mx[1][o] = npx1;
           }
@@ -420,7 +422,7 @@ __device__ __forceinline__ void tb2d_item(const TB2D<T> &P, int ts, int jb, int 
           P.vy[c] = vyn;
           {
             if (SX && inx) {
-              const long o = sxi + (long)p.sx.w * j;
+              const unsigned o = sxi + sxw * (unsigned)j;
               P.mx[2][o] = npx2;
               P.mx[3][o] = npx3;
             }

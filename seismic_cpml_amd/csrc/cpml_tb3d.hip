@@ -6,13 +6,13 @@
 // A workgroup is NW wavefronts; wave w holds grid row j0 - NT + w and lane l
 // column i0 - NT + l, and the group marches through the z planes of one
 // chunk.  At plane iteration s it
-//   * issues the loads of the next iteration (v at s + 2, sigma and the
-//     coefficients at s + 1, the level-1 memory variables),
 //   * for each time level m = 1..NT computes sigma^m at plane p = s - 2(m-1)
 //     from the 3-plane column window of v^{m-1}, then v^m at plane p - 1
-//     from the 3-plane window of sigma^m; x neighbours move across lanes,
-//     y neighbours through LDS (written the iteration before: one barrier
-//     per plane, two buffers),
+//     from the 3-plane window of sigma^m, and issues the loads of the next
+//     iteration (v at s + 2, sigma and the coefficients at s + 1, the level-1
+//     memory variables) as level 1 frees their registers; x neighbours move
+//     across lanes, y neighbours through LDS (written the iteration before:
+//     one barrier per plane, two buffers),
 //   * stores level NT (sigma at s - 2(NT-1), v at s - 2NT + 1) for the owned
 //     points and planes, and records the receivers of levels 1..NT-1.
 // Every intermediate level stays in registers and LDS; HBM sees the state
@@ -27,41 +27,27 @@
 // Per point the arithmetic is exactly the two-phase kernels' (same
 // expressions, no FMA contraction), so results are bit-identical to them.
 //
-// Tiles are split by the absorbing slabs their points and ring touch: the
-// x/y slabs (XY) and the z slabs (Z); each class is one launch of the kernel
-// built with just the C-PML code it needs.
+// Tiles are split by the axes along which their points and ring touch an
+// absorbing slab or a grid face; each class is one launch of the kernel built
+// with just the C-PML code and the predicates of those axes.
+#include <algorithm>
+
 #include "cpml_device.h"
 #include "cpml_internal.h"
 
 namespace cpml {
 namespace {
 
-__device__ __forceinline__ float lane_of(float x, int a4) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(a4, __builtin_bit_cast(int, x)));
-}
-__device__ __forceinline__ double lane_of(double x, int a4) {
-  typedef int i32x2 __attribute__((ext_vector_type(2)));
-  i32x2 v = __builtin_bit_cast(i32x2, x);
-  v.x = __builtin_amdgcn_ds_bpermute(a4, v.x);
-  v.y = __builtin_amdgcn_ds_bpermute(a4, v.y);
-  return __builtin_bit_cast(double, v);
-}
-
-template <typename T, int N>
-__device__ __forceinline__ void push(T (&w)[N], T x) {
-#pragma unroll
-  for (int k = 0; k < N - 1; ++k) w[k] = w[k + 1];
-  w[N - 1] = x;
-}
-
-// psi <- b*psi + a*d ; d <- d/K + psi (old psi given, new one in `out`); no
-// update where `on` is false.  `slab`: the point lies in this axis' slab.
+// psi <- b*psi + a*d ; d <- d/K + psi (old psi given, new one in `out`) where
+// `slab`: the point lies in this axis' slab.  k1: K is 1 all along the axis, so
+// d / K == d; K: where to read it otherwise.
 template <typename T>
-__device__ __forceinline__ T pml(bool slab, bool on, T d, T old, T &out, T a, T b, T K) {
+__device__ __forceinline__ T pml(bool slab, bool k1, T d, T old, T &out, T a, T b, const T *K) {
   out = old;
-  if (!slab || !on) return d;
+  if (!slab) return d;
   out = b * old + a * d;
-  return over_k(d, K) + out;
+  if (!k1) d = over_k(d, *K);
+  return d + out;
 }
 
 struct Tile {
@@ -116,430 +102,479 @@ __device__ __forceinline__ Tile tb_tile(const P &Q, int nx, int ny, int nz, int 
   return f;
 }
 
+// Plane slot of a 3-plane window in the iteration of phase PH (the march is
+// unrolled by 3, so slots are compile-time constants and no window moves).
+template <int PH, int K>
+constexpr int slot_of() {
+  return ((PH + K) % 3 + 3) % 3;
+}
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
+
+template <typename T>
+__device__ __forceinline__ T ld_at(const T *base, unsigned byte_off) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + byte_off);
+}
+// State stores are streamed past the caches (the next launch reads them a
+// whole grid later); those of the memory variables, whose rows are shorter
+// than a cache line, merge in the L2.
+template <typename T>
+__device__ __forceinline__ void st_at(T *base, unsigned byte_off, T x) {
+  __builtin_nontemporal_store(x,
+                              reinterpret_cast<T *>(reinterpret_cast<char *>(base) + byte_off));
+}
+template <typename T>
+__device__ __forceinline__ void st_mem(T *base, unsigned byte_off, T x) {
+  *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + byte_off) = x;
+}
+
+// What bounds the march (float, 2 steps, 768^3, milliseconds per launch; boxes
+// differ by a few percent, pairs are from one box):
+//  * stores of part of a cache line.  A copy of 12 arrays read and 9 written
+//    in this tile pattern takes 12.9 ms with rows of 56 owned points (224
+//    bytes, so tiles share lines and the memory must merge them), 8.5 with 48
+//    (whole 64-byte sectors, non-temporal) and 7.6 with whole 128-byte lines;
+//    re-reading the ring costs almost nothing beside that.  Hence strips of
+//    whole sectors by default and non-temporal state stores: 15.1 -> 12.5.
+//  * instruction issue: the first form had 523 scalar instructions of 816 per
+//    plane (execution masks around every predicate and load, buffer resources
+//    rebuilt from the argument block).  Now an axis without slab flag has no
+//    predicates (its tiles and rings lie strictly inside the grid); loads are
+//    unconditional (coordinates clamped to the zero ghost points once per
+//    tile, planes once per iteration; a scalar base and one 32-bit lane
+//    offset); x neighbours move by DPP wave shifts folded into the
+//    subtractions; the march is unrolled by the window length, so windows do
+//    not move: 455 instructions, and 3.9 ms for the slab-free class with all
+//    loads hitting the L2, against 7.8 in earnest.
+//  * register spills in the x-slab class wrote more than the fields (5.9 GB
+//    per launch against 2.3 without): its updates are branches, not
+//    selections, and K is read only where it is not 1.
+// Loads two planes ahead (128 registers, 15 spilled): 16.8 against 15.1.
 template <typename T, int NT, int NW, bool SX, bool SY, bool SZ>
 __global__ __launch_bounds__(64 * NW) void k_tb3d(TB3D<T> P) {
   constexpr bool SLAB = SX || SY || SZ;
-  constexpr int WM = 2 * NT;                   // coefficient planes s - 2NT + 1 .. s
   constexpr int NL = NT > 1 ? NT - 1 : 1;      // memory-variable windows (levels 1..NT-1)
   constexpr int NS = 6 * NT;                   // LDS slots per buffer
-  __shared__ T xl[2][NS][NW][64];
+  // one row of padding at both ends: the row below row 0 of slot 0 and above
+  // the last row of the last slot are read (by ring rows only)
+  __shared__ T xl[2 * NS * NW * 64 + 128];
   const Step3D<T> &p = P.a;
   const int nx = p.nx, ny = p.ny, nz = p.nz;
   const Tile ft = tb_tile<SX, SY, SZ>(P, nx, ny, nz, p.kchunk);
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = ft.i0 - NT + lane, j = ft.j0 - NT + w;
-  const bool col_in = i >= 0 && i < nx, row_in = j >= 0 && j < ny;
-  const bool in_xy = col_in && row_in;
-  const bool own = lane >= NT && lane < NT + P.ow && i < nx && w >= NT && w < NT + P.ty && j < ny;
-  const int wm = w > 0 ? w - 1 : 0, wp = w < NW - 1 ? w + 1 : NW - 1;
-  const int up4 = ((lane + 63) & 63) * 4, dn4 = ((lane + 1) & 63) * 4;
+  const bool col_in = !SX || (i >= 0 && i < nx), row_in = !SY || (j >= 0 && j < ny);
+  const bool own = lane >= NT && lane < NT + P.ow && w >= NT && w < NT + P.ty &&
+                   (!SX || i < nx) && (!SY || j < ny);
   const int kb = ft.kb, ke = ft.ke;
+  // predicates of the update ranges: x per lane, y and z per wavefront
+  const bool xlo = !SX || (i >= 1 && i < nx), xhi = !SX || (i >= 0 && i <= nx - 2);
+  const bool ylo = !SY || (j >= 1 && j < ny), yhi = !SY || (j >= 0 && j <= ny - 2);
+  auto zlo = [&](int k) { return !SZ || (k >= 1 && k < nz); };
+  auto zhi = [&](int k) { return !SZ || (k >= 0 && k <= nz - 2); };
 
-  // buffers rebased at interior plane kl (the lowest plane loaded, >= 0)
-  const unsigned es = sizeof(T);
-  const int kl = max(kb - 2 * NT, 0), kh = min(ke + 2 * NT, nz);
-  const unsigned psb = (unsigned)(p.ps * es);
-  const unsigned bytes = (unsigned)((long)(kh - kl) * p.ps * es);
-  const long origin = (long)(kl + p.R) * p.ps - p.base;
-  const unsigned vo = (unsigned)(((long)(j + p.R) * p.ld + p.xpad + i) * es);
-  auto rs = [&](const T *f) { return make_rsrc(f + origin, bytes); };
+  // Offsets from the ghost corner (-1, -1, kl) of each array: clamped
+  // coordinates read a zero ghost point.
+  const int s0 = kb - (2 * NT - 1), s1 = ke - 1 + (2 * NT - 1);
+  const int kl = max(s0 - 1, -1);
+  const int ic = min(max(i, -1), nx), jc = min(max(j, -1), ny);
+  const unsigned vo = (unsigned)(((long)(jc + 1) * p.ld + (ic + 1)) * (long)sizeof(T));
+  const unsigned psb = (unsigned)(p.ps * (long)sizeof(T));
+  const long corner = (long)kl * p.ps - p.ld - 1;
+  auto pl = [&](int k) -> unsigned {
+    const int kk = SZ ? min(max(k, -1), nz) : k;
+    return (unsigned)(kk - kl) * psb + vo;
+  };
+  const T *const ivx = p.vx + corner, *const ivy = p.vy + corner, *const ivz = p.vz + corner;
+  const T *const ixx = p.sxx + corner, *const iyy = p.syy + corner, *const izz = p.szz + corner;
+  const T *const ixy = p.sxy + corner, *const ixz = p.sxz + corner, *const iyz = p.syz + corner;
+  const T *const icl = p.clam + corner, *const icm = p.cmu + corner, *const icb = p.cbuoy + corner;
   using KArgs = const __attribute__((address_space(4))) TB3D<T> *;
   auto args = [&]() -> KArgs { return kernarg<TB3D<T>>(); };
-  // plane k of a field: 0 outside the grid, and outside the planes [kl, kh)
-  // the buffer covers (which only the pipeline's first planes ask for)
-  auto LDP = [&](const T *f, int k) -> T {
-    if (!in_xy || k < kl || k >= kh) return T(0);
-    return BufOp<T>::ld(rs(f), vo, (unsigned)(k - kl) * psb);
-  };
-  auto STP = [&](T x, T *f, int k) { BufOp<T>::st(x, rs(f), vo, (unsigned)(k - kl) * psb); };
 
   // x/y slab membership and profiles (loop invariant)
   const bool inx = SX && p.sx.in(i), iny = SY && p.sy.in(j);
-  T X[6] = {T(0), T(0), T(1), T(0), T(0), T(1)}, Y[6] = {T(0), T(0), T(1), T(0), T(0), T(1)};
-  if (inx) {
-    X[0] = p.px.a[i], X[1] = p.px.b[i], X[2] = p.px.K[i];
-    X[3] = p.px.ah[i], X[4] = p.px.bh[i], X[5] = p.px.Kh[i];
-  }
-  if (iny) {
-    Y[0] = p.py.a[j], Y[1] = p.py.b[j], Y[2] = p.py.K[j];
-    Y[3] = p.py.ah[j], Y[4] = p.py.bh[j], Y[5] = p.py.Kh[j];
-  }
-  const unsigned sxw = (unsigned)p.sx.w, syw = (unsigned)p.sy.w;
-  const unsigned sxi = inx ? (unsigned)p.sx.s(i) : 0u, syj = iny ? (unsigned)p.sy.s(j) : 0u;
-  auto OX = [&](int k) { return sxi + sxw * ((unsigned)j + (unsigned)ny * (unsigned)k); };
-  auto OY = [&](int k) { return (unsigned)i + (unsigned)p.mld * (syj + syw * (unsigned)k); };
-  auto OZ = [&](int k) {
-    return (unsigned)i + (unsigned)p.mld * ((unsigned)j + (unsigned)ny * (unsigned)p.sz.s(k));
-  };
+  T X[4] = {T(0), T(0), T(0), T(0)}, Y[4] = {T(0), T(0), T(0), T(0)};  // a, b, a_half, b_half
+  if (SX && inx) X[0] = p.px.a[i], X[1] = p.px.b[i], X[2] = p.px.ah[i], X[3] = p.px.bh[i];
+  if (SY && iny) Y[0] = p.py.a[j], Y[1] = p.py.b[j], Y[2] = p.py.ah[j], Y[3] = p.py.bh[j];
+  const bool kx1 = p.sx.k1, ky1 = p.sy.k1, kz1 = p.sz.k1;
+  // byte offsets inside one plane of the memory variables
+  constexpr unsigned es = sizeof(T);
+  const unsigned mxo = inx ? (unsigned)p.sx.at(i, jc, ny) * es : 0u;
+  const unsigned myo = iny ? ((unsigned)ic + (unsigned)p.mld * (unsigned)p.sy.s(j)) * es : 0u;
+  const unsigned mzo = ((unsigned)ic + (unsigned)p.mld * (unsigned)jc) * es;
+  const bool mx_on = SX && inx && row_in, my_on = SY && iny && col_in, mz_on = col_in && row_in;
+  const long mxs = (long)p.sx.w * ny, mys = p.mld * p.sy.w, mzs = p.mld * ny;
 
-  // ---- column windows (index 2 = newest plane)
-  T V[NT][3][3];    // v^m (m = 0..NT-1): vx vy vz, planes q_m - 2 .. q_m (q_0 = s + 1)
-  T S[NT][6][3];    // sigma^m (m = 1..NT): xx yy zz xy xz yz, planes p_m - 2 .. p_m
-  T Cw[3][WM];      // DELTAT*lambda, DELTAT*mu, DELTAT/rho: planes s - 2NT + 1 .. s
+  // ---- column windows by plane (slot_of)
+  T V[NT][3][3];    // v^m (m = 0..NT-1): vx vy vz
+  T S[NT][6][3];    // sigma^m (m = 1..NT): xx yy zz xy xz yz
+  T Cl[3], Cm[3], Cb[3];
   // memory variables of levels 1..NT-1 per slab axis: [0..2] the stress
   // phase's (x: dvx_dx dvy_dx dvz_dx, ...), [3..5] the velocity phase's
   T MX[NL][6][3], MY[NL][6][3], MZ[NL][6][3];
 #pragma unroll
-  for (int m = 0; m < NT; ++m)
+  for (int k = 0; k < 3; ++k) {
+    Cl[k] = Cm[k] = Cb[k] = T(0);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
+    for (int m = 0; m < NT; ++m) {
 #pragma unroll
       for (int f = 0; f < 3; ++f) V[m][f][k] = T(0);
 #pragma unroll
       for (int f = 0; f < 6; ++f) S[m][f][k] = T(0);
     }
 #pragma unroll
-  for (int k = 0; k < WM; ++k) Cw[0][k] = Cw[1][k] = Cw[2][k] = T(0);
+    for (int m = 0; m < NL; ++m)
 #pragma unroll
-  for (int m = 0; m < NL; ++m)
-#pragma unroll
-    for (int f = 0; f < 6; ++f)
-#pragma unroll
-      for (int k = 0; k < 3; ++k) MX[m][f][k] = MY[m][f][k] = MZ[m][f][k] = T(0);
+      for (int f = 0; f < 6; ++f) MX[m][f][k] = MY[m][f][k] = MZ[m][f][k] = T(0);
+  }
 
-  // loads of one iteration s: v (s + 1), sigma (s), coefficients (s), and the
-  // level-1 memory variables (stress phase at s, velocity phase at s - 1)
-  struct Ld {
-    T v[3], so[6], c[3];
-    T mx[6], my[6], mz[6];
+  // values in flight: sigma and DELTAT*lambda, DELTAT*mu of the plane to come,
+  // DELTAT/rho of the plane below it, level-1 memory variables
+  T so[6], ncl, ncm, ncb, nv0[3], lx[6], ly[6], lz[6];
+#pragma unroll
+  for (int f = 0; f < 6; ++f) lx[f] = ly[f] = lz[f] = T(0);
+  auto load_s = [&](int k) {
+    const unsigned o = pl(k);
+    so[0] = ld_at(ixx, o), so[1] = ld_at(iyy, o), so[2] = ld_at(izz, o);
+    so[3] = ld_at(ixy, o), so[4] = ld_at(ixz, o), so[5] = ld_at(iyz, o);
+    ncl = ld_at(icl, o), ncm = ld_at(icm, o);
   };
-  auto load = [&](Ld &L, int s) {
+  auto load_v = [&](int k) {  // v of plane k, buoyancy of plane k - 2
+    const unsigned o = pl(k);
+    nv0[0] = ld_at(ivx, o), nv0[1] = ld_at(ivy, o), nv0[2] = ld_at(ivz, o);
+    ncb = ld_at(icb, pl(k - 2));
+  };
+  // memory variables of the stress (F = 0) or velocity (F = 3) phase, plane k
+  auto load_m = [&](auto first, int k) {
+    constexpr int F = decltype(first)::value;
     const KArgs Q = args();
-    L.v[0] = LDP(Q->a.vx, s + 1);
-    L.v[1] = LDP(Q->a.vy, s + 1);
-    L.v[2] = LDP(Q->a.vz, s + 1);
-    L.so[0] = LDP(Q->a.sxx, s);
-    L.so[1] = LDP(Q->a.syy, s);
-    L.so[2] = LDP(Q->a.szz, s);
-    L.so[3] = LDP(Q->a.sxy, s);
-    L.so[4] = LDP(Q->a.sxz, s);
-    L.so[5] = LDP(Q->a.syz, s);
-    L.c[0] = LDP(Q->a.clam, s);
-    L.c[1] = LDP(Q->a.cmu, s);
-    L.c[2] = LDP(Q->a.cbuoy, s);
-    if (SLAB) {
+    const bool kin = !SZ || (k >= 0 && k < nz);
+    if (SX) {
 #pragma unroll
-      for (int f = 0; f < 6; ++f) L.mx[f] = L.my[f] = L.mz[f] = T(0);
-      const bool ks = s >= 0 && s < nz, kv = s - 1 >= 0 && s - 1 < nz;
-      if (SX && inx && row_in) {
-        if (ks)
+      for (int f = F; f < F + 3; ++f) lx[f] = T(0);
+      if (mx_on && kin)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) L.mx[f] = Q->a.mx[f][OX(s)];
-        if (kv)
+        for (int f = F; f < F + 3; ++f) lx[f] = ld_at(Q->a.mx[f] + mxs * k, mxo);
+    }
+    if (SY) {
 #pragma unroll
-          for (int f = 3; f < 6; ++f) L.mx[f] = Q->a.mx[f][OX(s - 1)];
-      }
-      if (SY && iny && col_in) {
-        if (ks)
+      for (int f = F; f < F + 3; ++f) ly[f] = T(0);
+      if (my_on && kin)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) L.my[f] = Q->a.my[f][OY(s)];
-        if (kv)
+        for (int f = F; f < F + 3; ++f) ly[f] = ld_at(Q->a.my[f] + mys * k, myo);
+    }
+    if (SZ) {
 #pragma unroll
-          for (int f = 3; f < 6; ++f) L.my[f] = Q->a.my[f][OY(s - 1)];
-      }
-      if (SZ && in_xy) {
-        if (ks && p.sz.in(s))
+      for (int f = F; f < F + 3; ++f) lz[f] = T(0);
+      if (mz_on && p.sz.in(k))
 #pragma unroll
-          for (int f = 0; f < 3; ++f) L.mz[f] = Q->a.mz[f][OZ(s)];
-        if (kv && p.sz.in(s - 1))
-#pragma unroll
-          for (int f = 3; f < 6; ++f) L.mz[f] = Q->a.mz[f][OZ(s - 1)];
-      }
+        for (int f = F; f < F + 3; ++f) lz[f] = ld_at(Q->a.mz[f] + mzs * p.sz.s(k), mzo);
     }
   };
 
-  const int s0 = kb - (2 * NT - 1), s1 = ke - 1 + (2 * NT - 1);
-  // prefill: v planes s0 - 1, s0; coefficient planes s0 - 2NT + 1 .. s0 - 1
+  const int own_row = 64 + w * 64 + lane;  // this thread's word of LDS slot 0, buffer 0
+  constexpr int SLOT = NW * 64, BUF = NS * SLOT;
+  // prologue (phase 0): v planes s0 - 1 .. s0 + 1, sigma and coefficients of s0
   {
-    const KArgs Q = args();
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      push(V[0][0], LDP(Q->a.vx, s0 - 1 + k));
-      push(V[0][1], LDP(Q->a.vy, s0 - 1 + k));
-      push(V[0][2], LDP(Q->a.vz, s0 - 1 + k));
-    }
-#pragma unroll
-    for (int k = 0; k < WM - 1; ++k) {
-      const int kk = s0 - WM + 1 + k;
-      push(Cw[0], LDP(Q->a.clam, kk));
-      push(Cw[1], LDP(Q->a.cmu, kk));
-      push(Cw[2], LDP(Q->a.cbuoy, kk));
+    V[0][0][slot_of<0, -1>()] = ld_at(ivx, pl(s0 - 1));
+    V[0][1][slot_of<0, -1>()] = ld_at(ivy, pl(s0 - 1));
+    V[0][2][slot_of<0, -1>()] = ld_at(ivz, pl(s0 - 1));
+    V[0][0][slot_of<0, 0>()] = ld_at(ivx, pl(s0));
+    V[0][1][slot_of<0, 0>()] = ld_at(ivy, pl(s0));
+    V[0][2][slot_of<0, 0>()] = ld_at(ivz, pl(s0));
+    load_s(s0);
+    load_v(s0 + 1);
+    if (SLAB) {
+      load_m(Int<0>{}, s0);
+      load_m(Int<3>{}, s0 - 1);
     }
     // LDS cleared, then the y neighbours of v at plane s0 for the first
-    // iteration (which reads buffer (s0 & 1) ^ 1)
-    for (int q = threadIdx.x; q < 2 * NS * NW * 64; q += 64 * NW) (&xl[0][0][0][0])[q] = T(0);
+    // iteration (which reads buffer 1)
+    for (int q = threadIdx.x; q < 2 * BUF + 128; q += 64 * NW) xl[q] = T(0);
     __syncthreads();
-    const int b0 = (s0 & 1) ^ 1;  // plane s0 is the newest of the prefilled window
-    xl[b0][0][w][lane] = V[0][0][2];
-    xl[b0][1][w][lane] = V[0][1][2];
-    xl[b0][2][w][lane] = V[0][2][2];
+    xl[BUF + own_row] = V[0][0][slot_of<0, 0>()];
+    xl[BUF + own_row + SLOT] = V[0][1][slot_of<0, 0>()];
+    xl[BUF + own_row + 2 * SLOT] = V[0][2][slot_of<0, 0>()];
   }
-  Ld C, N;
-  load(C, s0);
   __syncthreads();
 
-  // receivers of this tile: a cursor per recorded level (planes only increase)
+  // receivers of this tile: a cursor per recorded level (planes only
+  // increase), the plane of the next one held in a register
   const int tix = ft.ty * ((nx + P.ow - 1) / P.ow) + ft.tx;
-  int rc1 = 0;
-  int cur[NL];
+  constexpr int kNever = 0x7fffffff;
+  int rc1 = 0, cur[NL], rk[NL];
 #pragma unroll
-  for (int m = 0; m < NL; ++m) cur[m] = 0;
+  for (int m = 0; m < NL; ++m) cur[m] = 0, rk[m] = kNever;
   if (NT > 1 && P.nrec > 0) {
-    rc1 = P.rec_start[tix + 1];
+    rc1 = __builtin_amdgcn_readfirstlane(P.rec_start[tix + 1]);
+    int c = __builtin_amdgcn_readfirstlane(P.rec_start[tix]);
+    while (c < rc1 && P.rec_k[c] < kb) ++c;
+    const int k0 = c < rc1 ? __builtin_amdgcn_readfirstlane(P.rec_k[c]) : kNever;
 #pragma unroll
-    for (int m = 0; m < NL; ++m) cur[m] = P.rec_start[tix];
+    for (int m = 0; m < NL; ++m) cur[m] = c, rk[m] = k0;
   }
   const int it0 = *p.step;
+  // the source's column: its plane if this wavefront holds its row
+  const int ksrc = (j >= 0 && j == p.jsrc) ? p.ksrc : -1000;
 
-  for (int s = s0; s <= s1; ++s) {
-    const KArgs Q = args();
-    const int bw = s & 1, br = bw ^ 1;  // LDS buffer written / read this iteration
-    if (s < s1) load(N, s + 1);
-    push(V[0][0], C.v[0]);
-    push(V[0][1], C.v[1]);
-    push(V[0][2], C.v[2]);
-    push(Cw[0], C.c[0]);
-    push(Cw[1], C.c[1]);
-    push(Cw[2], C.c[2]);
-    // y neighbours of v at plane s + 1 for the next iteration
-    xl[bw][0][w][lane] = C.v[0];
-    xl[bw][1][w][lane] = C.v[1];
-    xl[bw][2][w][lane] = C.v[2];
-
+  auto plane = [&](auto phase, int s, int bw) {
+    constexpr int PH = decltype(phase)::value;
+    T *const wr = xl + own_row + bw * BUF;          // written this iteration
+    const T *const rd = xl + own_row + (bw ^ 1) * BUF;  // written the iteration before
+    Cl[slot_of<PH, 0>()] = ncl;
+    Cm[slot_of<PH, 0>()] = ncm;
+    Cb[slot_of<PH, -1>()] = ncb;
 #pragma unroll
-    for (int m = 1; m <= NT; ++m) {
-      const int pk = s - 2 * (m - 1);  // stress plane
-      const int qk = pk - 1;           // velocity plane
-      const int mb = m >= 2 ? m - 2 : 0;
-      const int cp = WM - 1 - 2 * (m - 1);  // coefficient window index of plane pk
+    for (int f = 0; f < 3; ++f) V[0][f][slot_of<PH, 1>()] = nv0[f];
+    // y neighbours of v at plane s + 1 for the next iteration
+    wr[0 * SLOT] = V[0][0][slot_of<PH, 1>()];
+    wr[1 * SLOT] = V[0][1][slot_of<PH, 1>()];
+    wr[2 * SLOT] = V[0][2][slot_of<PH, 1>()];
+
+    auto level = [&](auto lev) {
+      constexpr int m = decltype(lev)::value;
+      constexpr int D = 2 * (m - 1);
+      const int pk = s - D;   // stress plane
+      const int qk = pk - 1;  // velocity plane
+      constexpr int mb = m >= 2 ? m - 2 : 0;
+      constexpr int c0 = slot_of<PH, -D>(), cm1 = slot_of<PH, -D - 1>(),
+                    cp1 = slot_of<PH, -D + 1>(), cm2 = slot_of<PH, -D - 2>();
       // LDS slots of this level's inputs: v^{m-1} at pk, sigma^m at qk
-      const int sv = m == 1 ? 0 : 3 + 6 * (m - 2) + 3;
-      const int ss = 3 + 6 * (m - 1);
+      constexpr int sv = m == 1 ? 0 : 3 + 6 * (m - 2) + 3;
+      constexpr int ss = 3 + 6 * (m - 1);
       // ---------------- sigma^m at plane pk (3D:836-943)
       T sn[6];
-      if (m == 1) {
 #pragma unroll
-        for (int f = 0; f < 6; ++f) sn[f] = C.so[f];
-      } else {
-#pragma unroll
-        for (int f = 0; f < 6; ++f) sn[f] = S[mb][f][0];
-      }
+      for (int f = 0; f < 6; ++f) sn[f] = m == 1 ? so[f] : S[mb][f][c0];
       T om[9] = {};  // old memory variables of the stress phase: x 0..2, y 3..5, z 6..8
       if (SLAB) {
 #pragma unroll
         for (int f = 0; f < 3; ++f) {
-          if (SX) om[f] = m == 1 ? C.mx[f] : MX[mb][f][0];
-          if (SY) om[3 + f] = m == 1 ? C.my[f] : MY[mb][f][0];
-          if (SZ) om[6 + f] = m == 1 ? C.mz[f] : MZ[mb][f][0];
+          if (SX) om[f] = m == 1 ? lx[f] : MX[mb][f][c0];
+          if (SY) om[3 + f] = m == 1 ? ly[f] : MY[mb][f][c0];
+          if (SZ) om[6 + f] = m == 1 ? lz[f] : MZ[mb][f][c0];
         }
       }
       T nm[9];
 #pragma unroll
       for (int f = 0; f < 9; ++f) nm[f] = om[f];
       {
-        const T vxc = V[m - 1][0][1], vyc = V[m - 1][1][1], vzc = V[m - 1][2][1];
-        const T vx_xp = lane_of(vxc, dn4), vy_xm = lane_of(vyc, up4), vz_xm = lane_of(vzc, up4);
-        const T vx_yp = xl[br][sv + 0][wp][lane];
-        const T vy_ym = xl[br][sv + 1][wm][lane];
-        const T vz_yp = xl[br][sv + 2][wp][lane];
-        const bool inside = in_xy && pk >= 0 && pk < nz;
-        const bool inz = SZ && inside && p.sz.in(pk);
-        T Zp[6] = {T(0), T(0), T(1), T(0), T(0), T(1)};
-        if (inz) {
-          Zp[0] = p.pz.a[pk], Zp[1] = p.pz.b[pk], Zp[2] = p.pz.K[pk];
-          Zp[3] = p.pz.ah[pk], Zp[4] = p.pz.bh[pk], Zp[5] = p.pz.Kh[pk];
+        const T vxc = V[m - 1][0][c0], vyc = V[m - 1][1][c0], vzc = V[m - 1][2][c0];
+        const T vx_yp = rd[(sv + 0) * SLOT + 64];
+        const T vy_ym = rd[(sv + 1) * SLOT - 64];
+        const T vz_yp = rd[(sv + 2) * SLOT + 64];
+        const T dx_vx = lane_next(vxc) - vxc, dx_vy = vyc - lane_prev(vyc),
+                dx_vz = vzc - lane_prev(vzc);
+        const bool inz = SZ && p.sz.in(pk);
+        T Zp[4] = {T(0), T(0), T(0), T(0)};
+        if (SZ && inz)
+          Zp[0] = p.pz.a[pk], Zp[1] = p.pz.b[pk], Zp[2] = p.pz.ah[pk], Zp[3] = p.pz.bh[pk];
+        const T cl = Cl[c0], cm = Cm[c0];
+        if (ylo && zlo(pk) && xhi) {
+          T dvx_dx = dx_vx * p.odx;
+          T dvy_dy = (vyc - vy_ym) * p.ody;
+          T dvz_dz = (vzc - V[m - 1][2][cm1]) * p.odz;
+          if (SX) dvx_dx = pml(inx, kx1, dvx_dx, om[0], nm[0], X[2], X[3], p.px.Kh + i);
+          if (SY) dvy_dy = pml(iny, ky1, dvy_dy, om[3], nm[3], Y[0], Y[1], p.py.K + j);
+          if (SZ) dvz_dz = pml(inz, kz1, dvz_dz, om[6], nm[6], Zp[0], Zp[1], p.pz.K + pk);
+          const T lp2m = cl + T(2) * cm;
+          sn[0] = lp2m * dvx_dx + cl * (dvy_dy + dvz_dz) + sn[0];
+          sn[1] = cl * (dvx_dx + dvz_dz) + lp2m * dvy_dy + sn[1];
+          sn[2] = cl * (dvx_dx + dvy_dy) + lp2m * dvz_dz + sn[2];
         }
-        if (inside) {
-          const T cl = Cw[0][cp], cm = Cw[1][cp];
-          const bool r_n = i <= nx - 2 && j >= 1 && pk >= 1;
-          {
-            T dvx_dx = (vx_xp - vxc) * p.odx;
-            T dvy_dy = (vyc - vy_ym) * p.ody;
-            T dvz_dz = (vzc - V[m - 1][2][0]) * p.odz;
-            dvx_dx = pml(inx, r_n, dvx_dx, om[0], nm[0], X[3], X[4], X[5]);
-            dvy_dy = pml(iny, r_n, dvy_dy, om[3], nm[3], Y[0], Y[1], Y[2]);
-            dvz_dz = pml(inz, r_n, dvz_dz, om[6], nm[6], Zp[0], Zp[1], Zp[2]);
-            if (r_n) {
-              const T lp2m = cl + T(2) * cm;
-              sn[0] = lp2m * dvx_dx + cl * (dvy_dy + dvz_dz) + sn[0];
-              sn[1] = cl * (dvx_dx + dvz_dz) + lp2m * dvy_dy + sn[1];
-              sn[2] = cl * (dvx_dx + dvy_dy) + lp2m * dvz_dz + sn[2];
-            }
-          }
-          const bool r_xy = i >= 1 && j <= ny - 2;
-          {
-            T dvy_dx = (vyc - vy_xm) * p.odx;
-            T dvx_dy = (vx_yp - vxc) * p.ody;
-            dvy_dx = pml(inx, r_xy, dvy_dx, om[1], nm[1], X[0], X[1], X[2]);
-            dvx_dy = pml(iny, r_xy, dvx_dy, om[4], nm[4], Y[3], Y[4], Y[5]);
-            if (r_xy) sn[3] = cm * (dvy_dx + dvx_dy) + sn[3];
-          }
-          const bool r_xz = i >= 1 && pk <= nz - 2;
-          {
-            T dvz_dx = (vzc - vz_xm) * p.odx;
-            T dvx_dz = (V[m - 1][0][2] - vxc) * p.odz;
-            dvz_dx = pml(inx, r_xz, dvz_dx, om[2], nm[2], X[0], X[1], X[2]);
-            dvx_dz = pml(inz, r_xz, dvx_dz, om[7], nm[7], Zp[3], Zp[4], Zp[5]);
-            if (r_xz) sn[4] = cm * (dvz_dx + dvx_dz) + sn[4];
-          }
-          const bool r_yz = j <= ny - 2 && pk <= nz - 2;
-          {
-            T dvz_dy = (vz_yp - vzc) * p.ody;
-            T dvy_dz = (V[m - 1][1][2] - vyc) * p.odz;
-            dvz_dy = pml(iny, r_yz, dvz_dy, om[5], nm[5], Y[3], Y[4], Y[5]);
-            dvy_dz = pml(inz, r_yz, dvy_dz, om[8], nm[8], Zp[3], Zp[4], Zp[5]);
-            if (r_yz) sn[5] = cm * (dvz_dy + dvy_dz) + sn[5];
-          }
+        const bool zin = !SZ || (pk >= 0 && pk < nz);
+        if (yhi && zin && xlo) {
+          T dvy_dx = dx_vy * p.odx;
+          T dvx_dy = (vx_yp - vxc) * p.ody;
+          if (SX) dvy_dx = pml(inx, kx1, dvy_dx, om[1], nm[1], X[0], X[1], p.px.K + i);
+          if (SY) dvx_dy = pml(iny, ky1, dvx_dy, om[4], nm[4], Y[2], Y[3], p.py.Kh + j);
+          sn[3] = cm * (dvy_dx + dvx_dy) + sn[3];
+        }
+        if (row_in && zhi(pk) && xlo) {
+          T dvz_dx = dx_vz * p.odx;
+          T dvx_dz = (V[m - 1][0][cp1] - vxc) * p.odz;
+          if (SX) dvz_dx = pml(inx, kx1, dvz_dx, om[2], nm[2], X[0], X[1], p.px.K + i);
+          if (SZ) dvx_dz = pml(inz, kz1, dvx_dz, om[7], nm[7], Zp[2], Zp[3], p.pz.Kh + pk);
+          sn[4] = cm * (dvz_dx + dvx_dz) + sn[4];
+        }
+        if (yhi && zhi(pk) && col_in) {
+          T dvz_dy = (vz_yp - vzc) * p.ody;
+          T dvy_dz = (V[m - 1][1][cp1] - vyc) * p.odz;
+          if (SY) dvz_dy = pml(iny, ky1, dvz_dy, om[5], nm[5], Y[2], Y[3], p.py.Kh + j);
+          if (SZ) dvy_dz = pml(inz, kz1, dvy_dz, om[8], nm[8], Zp[2], Zp[3], p.pz.Kh + pk);
+          sn[5] = cm * (dvz_dy + dvy_dz) + sn[5];
         }
       }
 #pragma unroll
-      for (int f = 0; f < 6; ++f) push(S[m - 1][f], sn[f]);
-      if (SLAB && m < NT) {
+      for (int f = 0; f < 6; ++f) S[m - 1][f][c0] = sn[f];
+      if constexpr (SLAB && m < NT) {
 #pragma unroll
         for (int f = 0; f < 3; ++f) {
-          if (SX) push(MX[m - 1][f], nm[f]);
-          if (SY) push(MY[m - 1][f], nm[3 + f]);
-          if (SZ) push(MZ[m - 1][f], nm[6 + f]);
+          if (SX) MX[m - 1][f][c0] = nm[f];
+          if (SY) MY[m - 1][f][c0] = nm[3 + f];
+          if (SZ) MZ[m - 1][f][c0] = nm[6 + f];
         }
       }
-      xl[bw][ss + 0][w][lane] = sn[3];  // sigma_xy, sigma_yz, sigma_yy of plane pk
-      xl[bw][ss + 1][w][lane] = sn[5];
-      xl[bw][ss + 2][w][lane] = sn[1];
-      if (m == NT && own && pk >= kb && pk < ke) {
-        STP(sn[0], Q->sxx, pk);
-        STP(sn[1], Q->syy, pk);
-        STP(sn[2], Q->szz, pk);
-        STP(sn[3], Q->sxy, pk);
-        STP(sn[4], Q->sxz, pk);
-        STP(sn[5], Q->syz, pk);
+      wr[(ss + 0) * SLOT] = sn[3];  // sigma_xy, sigma_yz, sigma_yy of plane pk
+      wr[(ss + 1) * SLOT] = sn[5];
+      wr[(ss + 2) * SLOT] = sn[1];
+      if (m == NT && pk >= kb && pk < ke && own) {
+        const unsigned o = pl(pk);
+        st_at(P.sxx + corner, o, sn[0]);
+        st_at(P.syy + corner, o, sn[1]);
+        st_at(P.szz + corner, o, sn[2]);
+        st_at(P.sxy + corner, o, sn[3]);
+        st_at(P.sxz + corner, o, sn[4]);
+        st_at(P.syz + corner, o, sn[5]);
+        const KArgs Q = args();
         if (SX && inx)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) Q->mx[f][OX(pk)] = nm[f];
+          for (int f = 0; f < 3; ++f) st_mem(Q->mx[f] + mxs * pk, mxo, nm[f]);
         if (SY && iny)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) Q->my[f][OY(pk)] = nm[3 + f];
+          for (int f = 0; f < 3; ++f) st_mem(Q->my[f] + mys * pk, myo, nm[3 + f]);
         if (SZ && p.sz.in(pk))
 #pragma unroll
-          for (int f = 0; f < 3; ++f) Q->mz[f][OZ(pk)] = nm[6 + f];
+          for (int f = 0; f < 3; ++f) st_mem(Q->mz[f] + mzs * p.sz.s(pk), mzo, nm[6 + f]);
+      }
+      if (m == 1 && s < s1) {  // sigma and the coefficients of the next plane
+        load_s(s + 1);
+        if (SLAB) load_m(Int<0>{}, s + 1);
       }
 
       // ---------------- v^m at plane qk (3D:976-1121)
-      T vn[3] = {V[m - 1][0][0], V[m - 1][1][0], V[m - 1][2][0]};
+      T vn[3] = {V[m - 1][0][cm1], V[m - 1][1][cm1], V[m - 1][2][cm1]};
       T ov[9] = {};
       if (SLAB) {
 #pragma unroll
         for (int f = 0; f < 3; ++f) {
-          if (SX) ov[f] = m == 1 ? C.mx[3 + f] : MX[mb][3 + f][0];
-          if (SY) ov[3 + f] = m == 1 ? C.my[3 + f] : MY[mb][3 + f][0];
-          if (SZ) ov[6 + f] = m == 1 ? C.mz[3 + f] : MZ[mb][3 + f][0];
+          if (SX) ov[f] = m == 1 ? lx[3 + f] : MX[mb][3 + f][cm1];
+          if (SY) ov[3 + f] = m == 1 ? ly[3 + f] : MY[mb][3 + f][cm1];
+          if (SZ) ov[6 + f] = m == 1 ? lz[3 + f] : MZ[mb][3 + f][cm1];
         }
       }
       T nv[9];
 #pragma unroll
       for (int f = 0; f < 9; ++f) nv[f] = ov[f];
       {
-        const T(&sw)[6][3] = S[m - 1];  // planes qk - 1, qk, qk + 1
-        const T sxx_xm = lane_of(sw[0][1], up4);
-        const T sxy_xp = lane_of(sw[3][1], dn4);
-        const T sxz_xp = lane_of(sw[4][1], dn4);
-        const T sxy_ym = xl[br][ss + 0][wm][lane];
-        const T syz_ym = xl[br][ss + 1][wm][lane];
-        const T syy_yp = xl[br][ss + 2][wp][lane];
-        const bool inside = in_xy && qk >= 0 && qk < nz;
-        const bool inz = SZ && inside && p.sz.in(qk);
-        T Zq[6] = {T(0), T(0), T(1), T(0), T(0), T(1)};
-        if (inz) {
-          Zq[0] = p.pz.a[qk], Zq[1] = p.pz.b[qk], Zq[2] = p.pz.K[qk];
-          Zq[3] = p.pz.ah[qk], Zq[4] = p.pz.bh[qk], Zq[5] = p.pz.Kh[qk];
+        const T(&sw)[6][3] = S[m - 1];
+        const T xxc = sw[0][cm1], xyc = sw[3][cm1], xzc = sw[4][cm1], yzc = sw[5][cm1];
+        const T sxy_ym = rd[(ss + 0) * SLOT - 64];
+        const T syz_ym = rd[(ss + 1) * SLOT - 64];
+        const T syy_yp = rd[(ss + 2) * SLOT + 64];
+        const T dx_xx = xxc - lane_prev(xxc), dx_xy = lane_next(xyc) - xyc,
+                dx_xz = lane_next(xzc) - xzc;
+        const bool inz = SZ && p.sz.in(qk);
+        T Zq[4] = {T(0), T(0), T(0), T(0)};
+        if (SZ && inz)
+          Zq[0] = p.pz.a[qk], Zq[1] = p.pz.b[qk], Zq[2] = p.pz.ah[qk], Zq[3] = p.pz.bh[qk];
+        const T cb = Cb[cm1];
+        if (ylo && zlo(qk) && xlo) {
+          T dsxx_dx = dx_xx * p.odx;
+          T dsxy_dy = (xyc - sxy_ym) * p.ody;
+          T dsxz_dz = (xzc - sw[4][cm2]) * p.odz;
+          if (SX) dsxx_dx = pml(inx, kx1, dsxx_dx, ov[0], nv[0], X[0], X[1], p.px.K + i);
+          if (SY) dsxy_dy = pml(iny, ky1, dsxy_dy, ov[3], nv[3], Y[0], Y[1], p.py.K + j);
+          if (SZ) dsxz_dz = pml(inz, kz1, dsxz_dz, ov[6], nv[6], Zq[0], Zq[1], p.pz.K + qk);
+          vn[0] = cb * (dsxx_dx + dsxy_dy + dsxz_dz) + vn[0];
         }
-        if (inside) {
-          const T cb = Cw[2][cp - 1];
-          const bool r_vx = i >= 1 && j >= 1 && qk >= 1;
-          {
-            T dsxx_dx = (sw[0][1] - sxx_xm) * p.odx;
-            T dsxy_dy = (sw[3][1] - sxy_ym) * p.ody;
-            T dsxz_dz = (sw[4][1] - sw[4][0]) * p.odz;
-            dsxx_dx = pml(inx, r_vx, dsxx_dx, ov[0], nv[0], X[0], X[1], X[2]);
-            dsxy_dy = pml(iny, r_vx, dsxy_dy, ov[3], nv[3], Y[0], Y[1], Y[2]);
-            dsxz_dz = pml(inz, r_vx, dsxz_dz, ov[6], nv[6], Zq[0], Zq[1], Zq[2]);
-            if (r_vx) vn[0] = cb * (dsxx_dx + dsxy_dy + dsxz_dz) + vn[0];
-          }
-          const bool r_vy = i <= nx - 2 && j <= ny - 2 && qk >= 1;
-          {
-            T dsxy_dx = (sxy_xp - sw[3][1]) * p.odx;
-            T dsyy_dy = (syy_yp - sw[1][1]) * p.ody;
-            T dsyz_dz = (sw[5][1] - sw[5][0]) * p.odz;
-            dsxy_dx = pml(inx, r_vy, dsxy_dx, ov[1], nv[1], X[3], X[4], X[5]);
-            dsyy_dy = pml(iny, r_vy, dsyy_dy, ov[4], nv[4], Y[3], Y[4], Y[5]);
-            dsyz_dz = pml(inz, r_vy, dsyz_dz, ov[7], nv[7], Zq[0], Zq[1], Zq[2]);
-            if (r_vy) vn[1] = cb * (dsxy_dx + dsyy_dy + dsyz_dz) + vn[1];
-          }
-          const bool r_vz = i <= nx - 2 && j >= 1 && qk <= nz - 2;
-          {
-            T dsxz_dx = (sxz_xp - sw[4][1]) * p.odx;
-            T dsyz_dy = (sw[5][1] - syz_ym) * p.ody;
-            T dszz_dz = (sw[2][2] - sw[2][1]) * p.odz;
-            dsxz_dx = pml(inx, r_vz, dsxz_dx, ov[2], nv[2], X[3], X[4], X[5]);
-            dsyz_dy = pml(iny, r_vz, dsyz_dy, ov[5], nv[5], Y[0], Y[1], Y[2]);
-            dszz_dz = pml(inz, r_vz, dszz_dz, ov[8], nv[8], Zq[3], Zq[4], Zq[5]);
-            if (r_vz) vn[2] = cb * (dsxz_dx + dsyz_dy + dszz_dz) + vn[2];
-          }
-          // point force at step it0 + m - 1 (3D:1074-1082), rigid faces (3D:1087-1121)
-          if (i == p.isrc && j == p.jsrc && qk == p.ksrc) {
-            const int it = it0 + m - 1;
-            const T rsrc = Q->a.rho[i + (long)j * p.ld + (long)qk * p.ps];
-            vn[0] = vn[0] + Q->a.fx[it - 1] * p.dt / rsrc;
-            vn[1] = vn[1] + Q->a.fy[it - 1] * p.dt / rsrc;
-          }
-          if (i == 0 || i == nx - 1 || j == 0 || j == ny - 1 || qk == 0 || qk == nz - 1)
-            vn[0] = vn[1] = vn[2] = T(0);
+        if (yhi && zlo(qk) && xhi) {
+          T dsxy_dx = dx_xy * p.odx;
+          T dsyy_dy = (syy_yp - sw[1][cm1]) * p.ody;
+          T dsyz_dz = (yzc - sw[5][cm2]) * p.odz;
+          if (SX) dsxy_dx = pml(inx, kx1, dsxy_dx, ov[1], nv[1], X[2], X[3], p.px.Kh + i);
+          if (SY) dsyy_dy = pml(iny, ky1, dsyy_dy, ov[4], nv[4], Y[2], Y[3], p.py.Kh + j);
+          if (SZ) dsyz_dz = pml(inz, kz1, dsyz_dz, ov[7], nv[7], Zq[0], Zq[1], p.pz.K + qk);
+          vn[1] = cb * (dsxy_dx + dsyy_dy + dsyz_dz) + vn[1];
         }
+        if (ylo && zhi(qk) && xhi) {
+          T dsxz_dx = dx_xz * p.odx;
+          T dsyz_dy = (yzc - syz_ym) * p.ody;
+          T dszz_dz = (sw[2][c0] - sw[2][cm1]) * p.odz;
+          if (SX) dsxz_dx = pml(inx, kx1, dsxz_dx, ov[2], nv[2], X[2], X[3], p.px.Kh + i);
+          if (SY) dsyz_dy = pml(iny, ky1, dsyz_dy, ov[5], nv[5], Y[0], Y[1], p.py.K + j);
+          if (SZ) dszz_dz = pml(inz, kz1, dszz_dz, ov[8], nv[8], Zq[2], Zq[3], p.pz.Kh + qk);
+          vn[2] = cb * (dsxz_dx + dsyz_dy + dszz_dz) + vn[2];
+        }
+        // point force at step it0 + m - 1 (3D:1074-1082), rigid faces (3D:1087-1121)
+        if (qk == ksrc && i == p.isrc) {
+          const KArgs Q = args();
+          const int it = it0 + m - 1;
+          const T rsrc = Q->a.rho[i + (long)j * p.ld + (long)qk * p.ps];
+          vn[0] = vn[0] + Q->a.fx[it - 1] * p.dt / rsrc;
+          vn[1] = vn[1] + Q->a.fy[it - 1] * p.dt / rsrc;
+        }
+        if ((SX && (i == 0 || i == nx - 1)) || (SY && (j == 0 || j == ny - 1)) ||
+            (SZ && (qk == 0 || qk == nz - 1)))
+          vn[0] = vn[1] = vn[2] = T(0);
       }
-      if (m < NT) {
+      if constexpr (m < NT) {
 #pragma unroll
-        for (int f = 0; f < 3; ++f) push(V[m][f], vn[f]);
+        for (int f = 0; f < 3; ++f) V[m][f][cm1] = vn[f];
         if (SLAB) {
 #pragma unroll
           for (int f = 0; f < 3; ++f) {
-            if (SX) push(MX[m - 1][3 + f], nv[f]);
-            if (SY) push(MY[m - 1][3 + f], nv[3 + f]);
-            if (SZ) push(MZ[m - 1][3 + f], nv[6 + f]);
+            if (SX) MX[m - 1][3 + f][cm1] = nv[f];
+            if (SY) MY[m - 1][3 + f][cm1] = nv[3 + f];
+            if (SZ) MZ[m - 1][3 + f][cm1] = nv[6 + f];
           }
         }
-        xl[bw][ss + 3][w][lane] = vn[0];  // y neighbours of v^m at plane qk
-        xl[bw][ss + 4][w][lane] = vn[1];
-        xl[bw][ss + 5][w][lane] = vn[2];
+        wr[(ss + 3) * SLOT] = vn[0];  // y neighbours of v^m at plane qk
+        wr[(ss + 4) * SLOT] = vn[1];
+        wr[(ss + 5) * SLOT] = vn[2];
         // receivers of step it0 + m - 1 on plane qk (owned points only)
-        if (P.nrec > 0 && qk >= kb && qk < ke) {
-          int c = cur[m - 1];
-          while (c < rc1 && P.rec_k[c] < qk) ++c;
-          for (; c < rc1 && P.rec_k[c] == qk; ++c)
-            if (P.rec_i[c] == i && P.rec_j[c] == j && own) {
-              const long o = (long)(it0 + m - 2) * P.nrec + P.rec_slot[c];
-              P.sisx[o] = vn[0];
-              P.sisy[o] = vn[1];
-              if (P.sisz) P.sisz[o] = vn[2];
+        if (qk == rk[m - 1] && qk < ke) {
+          const KArgs Q = args();
+          int c = cur[m - 1], nk = qk;
+          while (nk == qk) {
+            if (Q->rec_i[c] == i && Q->rec_j[c] == j && own) {
+              const long o = (long)(it0 + m - 2) * Q->nrec + Q->rec_slot[c];
+              Q->sisx[o] = vn[0];
+              Q->sisy[o] = vn[1];
+              if (Q->sisz) Q->sisz[o] = vn[2];
             }
+            ++c;
+            nk = c < rc1 ? __builtin_amdgcn_readfirstlane(Q->rec_k[c]) : kNever;
+          }
           cur[m - 1] = c;
+          rk[m - 1] = nk;
         }
-      } else if (own && qk >= kb && qk < ke) {
-        STP(vn[0], Q->vx, qk);
-        STP(vn[1], Q->vy, qk);
-        STP(vn[2], Q->vz, qk);
+      } else if (qk >= kb && qk < ke && own) {
+        const unsigned o = pl(qk);
+        st_at(P.vx + corner, o, vn[0]);
+        st_at(P.vy + corner, o, vn[1]);
+        st_at(P.vz + corner, o, vn[2]);
+        const KArgs Q = args();
         if (SX && inx)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) Q->mx[3 + f][OX(qk)] = nv[f];
+          for (int f = 0; f < 3; ++f) st_mem(Q->mx[3 + f] + mxs * qk, mxo, nv[f]);
         if (SY && iny)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) Q->my[3 + f][OY(qk)] = nv[3 + f];
+          for (int f = 0; f < 3; ++f) st_mem(Q->my[3 + f] + mys * qk, myo, nv[3 + f]);
         if (SZ && p.sz.in(qk))
 #pragma unroll
-          for (int f = 0; f < 3; ++f) Q->mz[3 + f][OZ(qk)] = nv[6 + f];
+          for (int f = 0; f < 3; ++f) st_mem(Q->mz[3 + f] + mzs * p.sz.s(qk), mzo, nv[6 + f]);
       }
-    }
+      if (m == 1 && s < s1) {  // v of the plane after the next, buoyancy of this one
+        load_v(s + 2);
+        if (SLAB) load_m(Int<3>{}, s);
+      }
+    };
+    level(Int<1>{});
+    if constexpr (NT > 1) level(Int<2>{});
     __syncthreads();
-    C = N;
+  };
+  for (int s = s0, bw = 0;; s += 3, bw ^= 1) {
+    plane(Int<0>{}, s, bw);
+    if (s == s1) break;
+    plane(Int<1>{}, s + 1, bw ^ 1);
+    if (s + 1 == s1) break;
+    plane(Int<2>{}, s + 2, bw);
+    if (s + 2 == s1) break;
   }
 }
 
@@ -576,17 +611,18 @@ hipError_t tb3d_launch(const TB3D<T> &P0, hipStream_t s, hipStream_t side) {
   P.ty = NW - 2 * NT;
   if (P.ow < 1 || P.ow > 64 - 2 * NT) return hipErrorInvalidValue;
   // z regions: planes whose march (2NT - 1 planes of ring) avoids the z slabs
+  // and the first and last plane
   const int g = 2 * NT - 1, nz = p.nz, kc = p.kchunk;
-  int z0 = p.sz.wl > 0 ? p.sz.wl + g : 0;
-  int z1 = p.sz.wr > 0 ? nz - p.sz.wr - g : nz;
+  int z0 = std::max(p.sz.wl, 1) + g;
+  int z1 = nz - std::max(p.sz.wr, 1) - g;
   if (z1 <= z0) z0 = z1 = 0;
   P.z0 = z0;
   P.z1 = z1;
   P.zn[0] = (z0 + kc - 1) / kc;
   P.zn[1] = (z1 - z0 + kc - 1) / kc;
   P.zn[2] = (nz - z1 + kc - 1) / kc;
-  clean_tiles(p.nx, P.ow, NT, p.sx.wl, p.sx.wr, P.box[0], P.box[1]);
-  clean_tiles(p.ny, P.ty, NT, p.sy.wl, p.sy.wr, P.box[2], P.box[3]);
+  clean_tiles(p.nx, P.ow, NT, std::max(p.sx.wl, 1), std::max(p.sx.wr, 1), P.box[0], P.box[1]);
+  clean_tiles(p.ny, P.ty, NT, std::max(p.sy.wl, 1), std::max(p.sy.wr, 1), P.box[2], P.box[3]);
   if (P.box[1] < P.box[0]) P.box[0] = P.box[1] = 0;
   if (P.box[3] < P.box[2]) P.box[2] = P.box[3] = 0;
   const int n[3] = {(p.nx + P.ow - 1) / P.ow, (p.ny + P.ty - 1) / P.ty,

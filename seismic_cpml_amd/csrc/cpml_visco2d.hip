@@ -71,7 +71,7 @@ __global__ __launch_bounds__(BX *VTY) void k_stress2dve(Visco2D<T> v) {
   T *__restrict__ re11 = v.re11;
   T *__restrict__ re13 = v.re13;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const long mxo = p.sx.s(i) + (long)p.sx.w * j;
+  const long mxo = p.sx.at(i, j, p.ny);
   const long myo = i + p.mld * p.sy.s(j);
   // sigma_xx, sigma_yy: Fortran i = 1..NX-1, j = 2..NY (2D-visco2:742-800)
   if (i <= p.nx - 2 && j >= 1) {
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(BX *VTY) void k_velocity2dve(Visco2D<T> v) {
   const Step2D<T> &p = v.s;
   const long ld = p.ld, c = i + j * ld;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const long mxo = p.sx.s(i) + (long)p.sx.w * j;
+  const long mxo = p.sx.at(i, j, p.ny);
   const long myo = i + p.mld * p.sy.s(j);
   const T *__restrict__ sxx = p.sxx;
   const T *__restrict__ syy = p.syy;
