@@ -177,12 +177,13 @@ int cpml_gpu_set_fused(cpml_solver *h, int on);
  * ping-pongs between two buffers: one more set of field arrays and memory
  * variables).  steps 0 turns it off.  2D (orders 2, 4, 8): at most 4 / 3 / 2
  * steps in float, 2 in double; one 64-lane wavefront per strip of
- * strip_width columns marching through chunks of chunk_rows rows (0: 40).
+ * strip_width columns marching through chunks of chunk_rows rows (0: 16 to
+ * 64, by the grid's size).
  * 3D (order 2): at most 2 steps; a workgroup owns strip_width columns x
  * 12 (float; double: 4) rows for 2 steps (14 / 6 for 1) and marches through
- * z chunks of chunk_rows planes (0: 64).  strip_width 0 = every column the
- * ring of steps*(order-1) columns per side leaves (3D: rounded down to a
- * multiple of 8).  Used
+ * z chunks of chunk_rows planes (0: 8 to 64, by the grid's size).  strip_width 0 =
+ * the columns that the ring of steps*(order-1) columns per side leaves,
+ * rounded down to whole 64-byte sectors.  Used
  * on the elastic step without a learned boundary; with the energy curve on
  * (set_energy), in 2D at any cadence (the kernel sums the energy terms of
  * every level it computes; the curve equals the single-step one to
@@ -298,10 +299,10 @@ int cpml_batch_autotune(cpml_batch *b, int trial_steps, const char *cache_path, 
                         int *blocks_per_cu, double *best_ms);
 /* Time blocking of the whole batch: `steps` leapfrog steps of every shot per
  * launch (the kernel of cpml_gpu_set_time_block over a flat list of (shot,
- * strip, chunk) items; slab items beside the others on a second stream, each
- * covering half a chunk when chunks have 48 rows or more;
+ * strip, chunk) items; the items with C-PML code first, in chunks of half the
+ * rows (8 to 24);
  * state ping-ponging between two pools), 0 = single steps.  strip_width,
- * chunk_rows: as cpml_gpu_set_time_block (0 = defaults).  With energy on,
+ * chunk_rows: as cpml_gpu_set_time_block (rows 0: 40).  With energy on,
  * blocks are used when the cadence is a multiple of `steps`. */
 int cpml_batch_set_time_block(cpml_batch *b, int steps, int strip_width, int chunk_rows);
 /* The launch shape in use (after set_tiling / set_time_block / autotune). */

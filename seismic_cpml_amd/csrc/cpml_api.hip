@@ -146,12 +146,11 @@ struct cpml_solver {
   bool fused = false;   // 3D: one fused kernel per step (ping-pong state)
   // 2D time blocking: tb steps per launch (0: off), strips of tb_ow columns
   // (0: every lane the ring leaves; 3D: a multiple of 8), chunks of tb_jc rows
-  int tb = 0, tb_ow = 0, tb_jc = 40;
-  // side stream of the time-blocked launches (slab classes beside the rest)
-  hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  // (2D items with C-PML code: tb_js)
+  int tb = 0, tb_ow = 0, tb_jc = 40, tb_js = 16;
   int *tb_rec = nullptr;        // per-strip receiver lists (device)
-  double *tb_epart = nullptr;   // 2D time-blocked energy: per-item sums of every level
+  int tb_pending = 0;           // time-blocked launches since the step counter was advanced
+  double *tb_epart = nullptr;   // 2D time-blocked energy: per-item sums of every pending level
   size_t tb_epart_cap = 0;      // its size in doubles
   int tb_rec_ow = -1;           // strip width they were built for (-1: stale)
   std::vector<int> rec_ix, rec_iy, rec_iz;  // receiver grid indices (0-based), host copy
@@ -368,6 +367,8 @@ cpml::Step2D<T> step2d(cpml_solver *h) {
   // 2D2:564 divides by DELTAX; 2D4:565 by (24*DELTAX); ADE8:734 by DELTAX
   p.den_x = h->order == 4 ? T(24) * T(h->dx) : T(h->dx);
   p.den_y = h->order == 4 ? T(24) * T(h->dy) : T(h->dy);
+  p.div_x = cpml::const_div(p.den_x);
+  p.div_y = cpml::const_div(p.den_y);
   p.dt = T(h->dt);
   p.isrc = h->isrc;
   p.jsrc = h->jsrc;
@@ -672,16 +673,31 @@ int build_tb_receivers(cpml_solver *h) {
   return CPML_OK;
 }
 
-// Items of a 2D time-blocked launch (strips x chunks): the energy slots.
+// Items of a 2D time-blocked launch: the energy slots.
 int tb2d_slots(const cpml_solver *h) {
-  return ((h->nx + h->tb_ow - 1) / h->tb_ow) * ((h->ny + h->tb_jc - 1) / h->tb_jc);
+  cpml::TB2D<float> P{};  // the split does not depend on the precision
+  P.a.nx = h->nx;
+  P.a.ny = h->ny;
+  P.a.sx = h->sx;
+  P.a.sy = h->sy;
+  P.ow = h->tb_ow;
+  P.jc = h->tb_jc;
+  P.js = h->tb_js;
+  cpml::tb2d_split(h->order, h->tb, P);
+  const cpml::Tb2dItems n = cpml::tb2d_items(P);
+  return n.clean + n.edge + n.cap;
 }
 
-// The per-item energy sums of a 2D time-blocked launch (allocated before any
+// Time-blocked launches between two advances of the step counter (and, in 2D,
+// two sums of their energy): the launches record their own receivers and know
+// their distance from the counter, so nothing runs between them.
+constexpr int kTbPending = 8;
+
+// The per-item energy sums of 2D time-blocked launches (allocated before any
 // graph capture: enqueue_steps calls this first).
 int ensure_tb_energy(cpml_solver *h) {
   if (h->ndim != 2 || h->cadence <= 0) return CPML_OK;
-  const size_t need = (size_t)h->tb * tb2d_slots(h) * 2;
+  const size_t need = (size_t)kTbPending * h->tb * tb2d_slots(h) * 2;
   if (need <= h->tb_epart_cap) return CPML_OK;
   dev_free(h, *(void **)&h->tb_epart);
   h->tb_epart_cap = 0;
@@ -707,6 +723,7 @@ cpml::TB2D<T> tb_of(cpml_solver *h) {
   }
   P.ow = h->tb_ow;
   P.jc = h->tb_jc;
+  P.js = h->tb_js;
   const int nt = tb_tiles(h);
   P.rec_start = h->tb_rec;
   P.rec_i = h->tb_rec + nt + 1;
@@ -715,8 +732,9 @@ cpml::TB2D<T> tb_of(cpml_solver *h) {
   P.sisx = static_cast<T *>(h->seis[0]);
   P.sisy = static_cast<T *>(h->seis[1]);
   P.nrec = h->nrec;
+  P.ahead = h->tb_pending * h->tb;
   if (h->cadence > 0) {  // energy of every level, summed inside the kernel
-    P.epart = h->tb_epart;
+    P.epart = h->tb_epart + (size_t)h->tb_pending * h->tb * tb2d_slots(h) * 2;
     for (int q = 0; q < 4; ++q) P.ew[q] = h->ewin[q] - 1;
     P.eslots = tb2d_slots(h);
   }
@@ -748,40 +766,40 @@ cpml::TB3D<T> tb3_of(cpml_solver *h) {
   P.sisy = static_cast<T *>(h->seis[1]);
   P.sisz = static_cast<T *>(h->seis[2]);
   P.nrec = h->nrec;
+  P.ahead = h->tb_pending * h->tb;
   return P;
 }
 
 // One time-blocked launch (tb steps): the kernel writes the other state
-// buffer and records the receivers of its first tb - 1 steps; the record
-// kernel takes the last one and advances the step counter by tb.
+// buffer and records the receivers of its steps.
 template <typename T>
 hipError_t enqueue_tb(cpml_solver *h) {
-  hipError_t e = hipEventRecord(h->ev_fork, h->stream);  // fork: side waits for main
-  if (e == hipSuccess) e = hipStreamWaitEvent(h->side, h->ev_fork, 0);
-  if (e == hipSuccess)
-    e = h->ndim == 3 ? cpml::launch_tb3d<T>(h->tb, tb3_of<T>(h), h->stream, h->side)
-                     : cpml::launch_tb2d<T>(h->order, h->tb, tb_of<T>(h), h->stream, h->side);
-  if (e == hipSuccess) e = hipEventRecord(h->ev_join, h->side);  // join: main waits for side
-  if (e == hipSuccess) e = hipStreamWaitEvent(h->stream, h->ev_join, 0);
+  hipError_t e = h->ndim == 3 ? cpml::launch_tb3d<T>(h->tb, tb3_of<T>(h), h->stream)
+                              : cpml::launch_tb2d<T>(h->order, h->tb, tb_of<T>(h), h->stream);
   h->cur ^= 1;
+  if (e == hipSuccess && h->ndim == 3 && h->cadence > 0) {  // the block's last step, from memory
+    cpml::Energy<T> en = energy_of<T>(h);
+    en.offset = (h->tb_pending + 1) * h->tb - 1;
+    e = cpml::launch_energy<T>(en, h->eblocks, h->stream);
+  }
+  ++h->tb_pending;
   return e;
 }
+
+// Brings the step counter (and the 2D energy curve) up to the launches enqueued.
 template <typename T>
-hipError_t enqueue_tb_tail(cpml_solver *h) {
-  if (h->cadence > 0) {
-    hipError_t err;
-    if (h->ndim == 2) {  // every level, from the sums of the block's items
-      err = cpml::launch_tb2d_energy<T>(energy_of<T>(h), h->tb_epart, tb2d_slots(h), h->tb,
-                                        h->stream);
-    } else {  // the block's last step, from the state in memory
-      cpml::Energy<T> e = energy_of<T>(h);
-      e.offset = h->tb - 1;
-      err = cpml::launch_energy<T>(e, h->eblocks, h->stream);
-    }
-    if (err != hipSuccess) return err;
+hipError_t flush_tb(cpml_solver *h) {
+  if (h->tb_pending == 0) return hipSuccess;
+  const int steps = h->tb_pending * h->tb;
+  h->tb_pending = 0;
+  if (h->ndim == 2 && h->cadence > 0) {  // every level, from the sums of the launches' items
+    hipError_t e = cpml::launch_tb2d_energy<T>(energy_of<T>(h), h->tb_epart, tb2d_slots(h), steps,
+                                               h->stream);
+    if (e != hipSuccess) return e;
   }
   cpml::Record<T> r = record_of<T>(h);
-  r.skip = h->tb - 1;
+  r.nrec = 0;
+  r.skip = steps - 1;
   return cpml::launch_record<T>(r, h->stream);
 }
 
@@ -823,11 +841,14 @@ int graph_units(const cpml_solver *h) {
 hipError_t enqueue_step_any(cpml_solver *h) {
   return h->prec == 4 ? enqueue_step<float>(h) : enqueue_step<double>(h);
 }
+hipError_t flush_any(cpml_solver *h) {
+  return h->prec == 4 ? flush_tb<float>(h) : flush_tb<double>(h);
+}
 // one launch unit: unit_steps(h) steps
 hipError_t enqueue_unit_any(cpml_solver *h) {
   if (!tb_active(h)) return enqueue_step_any(h);
   hipError_t e = h->prec == 4 ? enqueue_tb<float>(h) : enqueue_tb<double>(h);
-  if (e == hipSuccess) e = h->prec == 4 ? enqueue_tb_tail<float>(h) : enqueue_tb_tail<double>(h);
+  if (e == hipSuccess && h->tb_pending == kTbPending) e = flush_any(h);
   return e;
 }
 
@@ -846,6 +867,8 @@ int build_graph(cpml_solver *h) {
   HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
   hipError_t e = hipSuccess;
   for (int s = 0; s < graph_units(h) && e == hipSuccess; ++s) e = enqueue_unit_any(h);
+  if (e == hipSuccess) e = flush_any(h);
+  h->tb_pending = 0;
   h->cur = slot;  // capture does not execute: the state is still where it was
   hipError_t e2 = hipStreamEndCapture(h->stream, &g);
   if (e != hipSuccess || e2 != hipSuccess) {
@@ -877,6 +900,7 @@ int enqueue_steps(cpml_solver *h, int n, int *ev_used) {
     if (!rc) rc = ensure_tb_energy(h);
     if (rc) return rc;
   }
+  h->tb_pending = 0;
   const int u = unit_steps(h);
   if (h->ktiming) {
     int rc = ensure_events(h, (size_t)(*ev_used + 3 * n));
@@ -887,7 +911,7 @@ int enqueue_steps(cpml_solver *h, int n, int *ev_used) {
       HIPCHK(h, h->prec == 4 ? enqueue_tb<float>(h) : enqueue_tb<double>(h));
       HIPCHK(h, hipEventRecord(e[1], h->stream));
       HIPCHK(h, hipEventRecord(e[2], h->stream));
-      HIPCHK(h, h->prec == 4 ? enqueue_tb_tail<float>(h) : enqueue_tb_tail<double>(h));
+      HIPCHK(h, flush_any(h));
       h->ev_tb.push_back(*ev_used);
       *ev_used += 3;
     }
@@ -928,6 +952,7 @@ int enqueue_steps(cpml_solver *h, int n, int *ev_used) {
     }
   }
   for (; n >= u && tb_active(h); n -= u) HIPCHK(h, enqueue_unit_any(h));
+  HIPCHK(h, flush_any(h));
   for (int s = 0; s < n; ++s) HIPCHK(h, enqueue_step_any(h));
   return CPML_OK;
 }
@@ -1240,13 +1265,9 @@ int cpml_gpu_finalize(cpml_solver *h) {
   for (auto g : h->gexec)
     if (g) (void)hipGraphExecDestroy(g);
   for (hipEvent_t e : h->evpool) (void)hipEventDestroy(e);
-  if (h->side) (void)hipStreamSynchronize(h->side);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
-  if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
-  if (h->ev_join) (void)hipEventDestroy(h->ev_join);
   for (void *p : h->allocs) (void)hipFree(p);
-  if (h->side) (void)hipStreamDestroy(h->side);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
   return CPML_OK;
@@ -2082,28 +2103,30 @@ int cpml_gpu_set_time_block(cpml_solver *h, int steps, int strip_width, int chun
     return fail(h, CPML_ERR_ARG, "strip width must be 0 (default) or 1.." +
                                      std::to_string(64 - 2 * g) + " for this order and step count");
   if (chunk_rows < 0) return fail(h, CPML_ERR_ARG, "chunk rows must be >= 0");
-  const int jc = chunk_rows > 0 ? chunk_rows : (h->ndim == 3 ? 64 : 40);
+  // default strip: whole 64-byte sectors of the lanes the ring leaves, so no tile
+  // stores part of one (order 4, 2 steps, float, 64-row chunks of 4096^2: 48
+  // columns 286 us, 52 columns 295; the batch of 32 shots 908 and 967)
+  const int widest = 64 - 2 * g, sector = 64 / (int)h->esize;
+  const int ow = strip_width > 0 ? strip_width
+                                 : (widest >= sector ? widest / sector * sector : widest);
+  int jc = chunk_rows;
+  if (jc == 0)
+    jc = h->ndim == 3 ? cpml::tb3d_default_planes(h->nx, h->ny, h->nz, ow,
+                                                  (h->esize == 4 ? 16 : 8) - 2 * steps)
+                      : cpml::tb2d_default_rows(h->nx, h->ny, ow);
+  if (h->ndim == 2) jc = std::min(jc, cpml::tb2d_max_rows(h->ld, h->esize));
+  if (chunk_rows == 0)
+    while (jc > 1 && !chunk_fits(h, jc)) --jc;
   if (!chunk_fits(h, jc))
     return fail(h, CPML_ERR_ARG, "chunk too deep for the kernels' 32-bit buffer offsets");
   int rc = set_device(h);
   if (rc) return rc;
   if (steps > 0 && (rc = ensure_second_state(h))) return rc;
   if (steps == 0 && (rc = restore_first_state(h))) return rc;
-  if (steps > 0 && !h->side) {
-    HIPCHK(h, hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking));
-    HIPCHK(h, hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming));
-    HIPCHK(h, hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming));
-  }
   h->tb = steps;
-  // default strip: every lane the ring leaves (2D, measured fastest: 52 columns
-  // at order 4 and 2 steps gave 79.4 Gcell/s against 75.7 for 48); 3D rounds
-  // it down to whole 64-byte sectors, so no tile stores part of one
-  const int widest = 64 - 2 * g;
-  const int sector = 64 / (int)h->esize;
-  h->tb_ow = strip_width > 0 ? strip_width
-                             : (h->ndim == 3 ? std::max(8, widest / sector * sector) : widest);
-  if (h->tb_ow > widest) h->tb_ow = widest;
+  h->tb_ow = ow;
   h->tb_jc = jc;
+  h->tb_js = cpml::tb2d_slab_rows(jc);
   h->tb_rec_ow = -1;
   h->graph_dirty = true;
   return CPML_OK;

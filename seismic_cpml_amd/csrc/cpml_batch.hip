@@ -8,10 +8,10 @@
 //    contiguous bands, one per XCD; a launch has one workgroup per tile or a
 //    fixed "persistent" grid whose workgroups stride through their band;
 //  * time-blocked: NT leapfrog steps per launch for all shots (the kernel of
-//    cpml_tb2d.hip over a flat list of (shot, strip, chunk) items, TB2D
+//    cpml_tb2d.h over a flat list of (shot, strip, chunk) items, TB2D
 //    descriptors per shot, persistent or one wavefront per item), the state
-//    ping-ponging between two pools; the items that touch a C-PML slab run
-//    beside the others on a second stream.
+//    ping-ponging between two pools; the items that touch a C-PML slab come
+//    first in the list.
 // Per point the arithmetic is the single-grid kernels', so a batched shot
 // equals the same shot run on its own, bit for bit.  Each shot has its own
 // step counter, energy curve (per-tile partial sums, then a per-shot sum in
@@ -88,11 +88,11 @@ __global__ __launch_bounds__(BX *TY) void k_batch2d(const Step2D<T> *__restrict_
 // before advanced skip + 1 steps), then that shot's step counter advances
 template <typename T>
 __global__ __launch_bounds__(kMaxRecBlock) void k_batch_record(const Record<T> *__restrict__ r,
-                                                               int skip) {
+                                                               int skip, int record) {
   const Record<T> &p = r[blockIdx.x];
   const int it = *p.step + skip;
   const long row = (long)(it - 1) * p.nrec;
-  for (int q = threadIdx.x; q < p.nrec; q += blockDim.x) {
+  for (int q = threadIdx.x; record && q < p.nrec; q += blockDim.x) {
     const long o = p.idx[q];
     p.sx[row + q] = p.vx[o];
     p.sy[row + q] = p.vy[o];
@@ -245,9 +245,9 @@ hipError_t batch_phase(int order, int rows, bool stress, bool streaming, const v
 }
 
 template <typename T>
-hipError_t batch_record(const void *rec, int nshots, int skip, hipStream_t s) {
+hipError_t batch_record(const void *rec, int nshots, int skip, bool record, hipStream_t s) {
   hipLaunchKernelGGL(k_batch_record<T>, dim3(nshots), dim3(kMaxRecBlock), 0, s,
-                     static_cast<const Record<T> *>(rec), skip);
+                     static_cast<const Record<T> *>(rec), skip, record ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -331,13 +331,12 @@ struct cpml_batch {
   void *d_desc2 = nullptr;   // Step2D<T>[nshots] over pool2
   void *d_rec2 = nullptr;    // Record<T>[nshots] over pool2
   void *d_tbd[2] = {};       // TB2D<T>[nshots]: state in pool (0) / pool2 (1)
-  int4 *d_items = nullptr;   // time-blocked items: the slab-free ones, then the others
+  int4 *d_items = nullptr;   // time-blocked items, classes in the order 3, 1, 2, 0
   // time-blocked items by class: slab-free, x slabs only, y slabs only, both
   int items_cap = 0, nitems[4] = {0, 0, 0, 0};
   int tb = 0, tb_ow = 0, tb_jc = 128;
-  int tb_jc_slab = 0;  // rows per slab item (0: tb_jc), set with tb_jc
-  hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  int tb_js = 16;  // rows per slab item, set with tb_jc
+  int tb_pending = 0;  // time-blocked launches since the step counters were advanced
   // energy (per shot, every `cadence` steps) and the stability check
   int cadence = 0;
   double *d_ekin = nullptr, *d_epot = nullptr;  // [nshots][nstep]
@@ -434,6 +433,8 @@ cpml::Step2D<T> shot_step(cpml_batch *b, int q, int parity) {
   p.mld = s.mld;
   p.den_x = b->order == 4 ? T(24) * T(s.dx) : T(s.dx);
   p.den_y = b->order == 4 ? T(24) * T(s.dy) : T(s.dy);
+  p.div_x = cpml::const_div(p.den_x);
+  p.div_y = cpml::const_div(p.den_y);
   p.dt = T(s.dt);
   p.isrc = s.isrc;
   p.jsrc = s.jsrc;
@@ -565,8 +566,8 @@ int upload_tables(cpml_batch *b) {
         }
         P.ow = b->tb_ow;
         P.jc = b->tb_jc;
-        P.nstrips = (s.nx + b->tb_ow - 1) / b->tb_ow;
-        P.nchunks = (s.ny + b->tb_jc - 1) / b->tb_jc;
+        P.js = b->tb_js;
+        cpml::tb2d_split(b->order, b->tb, P);
         const size_t m = (size_t)std::max(s.nrec, 1);
         P.rec_start = s.tbrec;
         P.rec_i = s.tbrec + P.nstrips + 1;
@@ -582,24 +583,31 @@ int upload_tables(cpml_batch *b) {
     }
   }
   if (b->tb > 0) {  // items (strip, rows) of every shot by class: slab-free, x, y, both
-    // A slab item runs the C-PML code and its class has few items, so its
-    // launch is bound by the latency of one wavefront's march: slab chunks
-    // are cut into sub-chunks of tb_jc_slab rows (more, shorter marches).
+    // A slab item runs the C-PML code and its launch has few items, so it is
+    // bound by the latency of one wavefront's march: shorter chunks (tb_js).
     std::vector<int4> it[4];
-    const int js = b->tb_jc_slab > 0 ? std::min(b->tb_jc_slab, b->tb_jc) : b->tb_jc;
     for (int q = 0; q < b->nshots; ++q) {
       const Shot &s = b->shots[q];
-      int box[4];
-      cpml::tb2d_clean_box(b->order, b->tb, s.nx, s.ny, b->tb_ow, b->tb_jc, s.sx, s.sy, box);
-      const int ns = (s.nx + b->tb_ow - 1) / b->tb_ow, nc = (s.ny + b->tb_jc - 1) / b->tb_jc;
-      for (int c = 0; c < nc; ++c)
-        for (int t = 0; t < ns; ++t) {
-          const int cls = (t >= box[0] && t < box[1] ? 0 : 1) | (c >= box[2] && c < box[3] ? 0 : 2);
-          const int jb = c * b->tb_jc, je = std::min(jb + b->tb_jc, s.ny);
-          const int step = cls ? js : b->tb_jc;
-          for (int r = jb; r < je; r += step)
-            it[cls].push_back(make_int4(q, t, r, std::min(r + step, je)));
-        }
+      cpml::TB2D<float> P{};  // the split does not depend on the precision
+      P.a.nx = s.nx;
+      P.a.ny = s.ny;
+      P.a.sx = s.sx;
+      P.a.sy = s.sy;
+      P.ow = b->tb_ow;
+      cpml::tb2d_split(b->order, b->tb, P);
+      auto rows = [&](int cls, int j0, int j1, int step, int t0, int t1) {
+        for (int r = j0; r < j1; r += step)
+          for (int t = t0; t < t1; ++t)
+            it[cls].push_back(make_int4(q, t, r, std::min(r + step, j1)));
+      };
+      rows(0, P.y0, P.y1, b->tb_jc, P.sx0, P.sx1);
+      for (int r = 0; r < s.ny; r += b->tb_js) {  // strips at the x slabs
+        const int e = std::min(r + b->tb_js, s.ny), cls = r >= P.y0 && e <= P.y1 ? 1 : 3;
+        rows(cls, r, e, b->tb_js, 0, P.sx0);
+        rows(cls, r, e, b->tb_js, P.sx1, P.nstrips);
+      }
+      rows(2, 0, P.y0, b->tb_js, P.sx0, P.sx1);
+      rows(2, P.y1, s.ny, b->tb_js, P.sx0, P.sx1);
     }
     int n = 0;
     for (int k = 0; k < 4; ++k) n += b->nitems[k] = (int)it[k].size();
@@ -609,8 +617,8 @@ int upload_tables(cpml_batch *b) {
       if (rc) return rc;
       b->items_cap = n;
     }
-    for (int k = 1; k < 4; ++k) it[0].insert(it[0].end(), it[k].begin(), it[k].end());
-    BCHK(b, hipMemcpy(b->d_items, it[0].data(), (size_t)n * sizeof(int4), hipMemcpyHostToDevice));
+    for (int k : {1, 2, 0}) it[3].insert(it[3].end(), it[k].begin(), it[k].end());
+    BCHK(b, hipMemcpy(b->d_items, it[3].data(), (size_t)n * sizeof(int4), hipMemcpyHostToDevice));
   }
   if (b->cadence > 0) {  // energy tiles of 64 x 16 points over every shot's window
     std::vector<int2> et;
@@ -645,13 +653,11 @@ int grid_of(const cpml_batch *b) {
   return std::max(8, std::min(b->ntiles, b->blocks_per_cu * b->ncu));
 }
 
-// workgroups of a time-blocked launch over n items: one wavefront per item, or
-// a persistent grid of blocks_per_cu per CU; never fewer than 8, since the
-// kernel hands every XCD (blockIdx.x % 8) its own eighth of the items
-int tb_blocks(const cpml_batch *b, int n) {
-  const int one = (n + 3) / 4;
-  if (b->blocks_per_cu <= 0) return std::max(one, 8);
-  return std::max(8, std::min(one, b->blocks_per_cu * b->ncu));
+// wavefronts of a time-blocked launch: one per item, or a persistent grid of
+// blocks_per_cu workgroups (4 wavefronts) per CU
+int tb_waves(const cpml_batch *b) {
+  const int n = b->nitems[0] + b->nitems[1] + b->nitems[2] + b->nitems[3];
+  return b->blocks_per_cu <= 0 ? n : std::min(n, 4 * b->blocks_per_cu * b->ncu);
 }
 
 void *cur_desc(const cpml_batch *b) { return b->cur ? b->d_desc2 : b->d_desc; }
@@ -669,36 +675,37 @@ hipError_t bstep_t(cpml_batch *b) {
   if (e == hipSuccess && b->cadence > 0)
     e = cpml::batch_energy<T>(b->d_en[b->cur], b->d_etab, b->netiles, b->d_estart, b->nshots, 0,
                               b->d_epart, b->stream);
-  if (e == hipSuccess) e = cpml::batch_record<T>(cur_rec(b), b->nshots, 0, b->stream);
+  if (e == hipSuccess) e = cpml::batch_record<T>(cur_rec(b), b->nshots, 0, true, b->stream);
   return e;
 }
 
-// NT = tb steps of every shot: the slab-free items on the main stream, the
-// slab classes (both axes first, then x, then y) beside them on the side
-// stream, then energy and receivers of the last step (the kernel recorded
-// the first tb - 1)
+// NT = tb steps of every shot in one launch (the items with C-PML code, few and
+// long, start first), then the energy of the last step
 template <typename T>
 hipError_t bunit_t(cpml_batch *b) {
   const auto *g = static_cast<const cpml::TB2D<T> *>(b->d_tbd[b->cur]);
-  int off[4] = {0, 0, 0, 0};  // start of each class in the item list
-  for (int k = 1; k < 4; ++k) off[k] = off[k - 1] + b->nitems[k - 1];
-  hipError_t e = hipEventRecord(b->ev_fork, b->stream);
-  if (e == hipSuccess) e = hipStreamWaitEvent(b->side, b->ev_fork, 0);
-  for (int k : {3, 1, 2})
-    if (e == hipSuccess && b->nitems[k])
-      e = cpml::launch_tb2d_multi<T>(b->order, b->tb, k, g, b->d_items + off[k], b->nitems[k],
-                                     tb_blocks(b, b->nitems[k]), b->side);
-  if (e == hipSuccess)
-    e = cpml::launch_tb2d_multi<T>(b->order, b->tb, 0, g, b->d_items, b->nitems[0],
-                                   tb_blocks(b, b->nitems[0]), b->stream);
-  if (e == hipSuccess) e = hipEventRecord(b->ev_join, b->side);
-  if (e == hipSuccess) e = hipStreamWaitEvent(b->stream, b->ev_join, 0);
+  hipError_t e = cpml::launch_tb2d_multi<T>(b->order, b->tb, g, b->d_items, b->nitems, tb_waves(b),
+                                            b->tb_pending * b->tb, b->stream);
   b->cur ^= 1;
   if (e == hipSuccess && b->cadence > 0)
     e = cpml::batch_energy<T>(b->d_en[b->cur], b->d_etab, b->netiles, b->d_estart, b->nshots,
-                              b->tb - 1, b->d_epart, b->stream);
-  if (e == hipSuccess) e = cpml::batch_record<T>(cur_rec(b), b->nshots, b->tb - 1, b->stream);
+                              (b->tb_pending + 1) * b->tb - 1, b->d_epart, b->stream);
+  ++b->tb_pending;
   return e;
+}
+
+// Advances every shot's step counter by the time-blocked steps enqueued since
+// the last time (the launches record their receivers themselves and know how
+// far they are from the counter).
+template <typename T>
+hipError_t bflush_t(cpml_batch *b) {
+  if (b->tb_pending == 0) return hipSuccess;
+  const int steps = b->tb_pending * b->tb;
+  b->tb_pending = 0;
+  return cpml::batch_record<T>(cur_rec(b), b->nshots, steps - 1, false, b->stream);
+}
+hipError_t enqueue_bflush(cpml_batch *b) {
+  return b->prec == 4 ? bflush_t<float>(b) : bflush_t<double>(b);
 }
 
 hipError_t enqueue_bstep(cpml_batch *b) {
@@ -737,7 +744,10 @@ int build_bgraph(cpml_batch *b) {
   hipGraph_t g = nullptr;
   BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   hipError_t e = hipSuccess;
+  b->tb_pending = 0;
   for (int u = 0; u < bgraph_units(b) && e == hipSuccess; ++u) e = enqueue_bany(b);
+  if (e == hipSuccess) e = enqueue_bflush(b);
+  b->tb_pending = 0;
   b->cur = slot;  // capture does not execute
   hipError_t e2 = hipStreamEndCapture(b->stream, &g);
   if (e != hipSuccess || e2 != hipSuccess) {
@@ -779,7 +789,9 @@ int enqueue_bsteps(cpml_batch *b, int it, int n) {
     }
     for (; n >= gl; n -= gl, it += gl) BCHK(b, hipGraphLaunch(b->gexec[b->cur], b->stream));
   }
+  b->tb_pending = 0;
   for (; n >= u && btb_active(b); n -= u, it += u) BCHK(b, enqueue_bunit(b));
+  BCHK(b, enqueue_bflush(b));
   for (; n > 0; --n, ++it) BCHK(b, enqueue_bstep(b));
   return CPML_OK;
 }
@@ -1017,14 +1029,10 @@ int cpml_batch_finalize(cpml_batch *b) {
   if (!b) return CPML_OK;
   (void)hipSetDevice(b->device);
   if (b->stream) (void)hipStreamSynchronize(b->stream);
-  if (b->side) (void)hipStreamSynchronize(b->side);
   drop_bgraphs(b);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
-  if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
-  if (b->ev_join) (void)hipEventDestroy(b->ev_join);
   for (void *p : b->allocs) (void)hipFree(p);
-  if (b->side) (void)hipStreamDestroy(b->side);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
   return CPML_OK;
@@ -1244,9 +1252,6 @@ int cpml_batch_set_time_block(cpml_batch *b, int steps, int strip_width, int chu
           rc = balloc(b, &s.mem2[k], std::max<size_t>(e, 1) * b->esize);
         }
     if (rc) return rc;
-    BCHK(b, hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
-    BCHK(b, hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming));
-    BCHK(b, hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming));
     BCHK(b, hipStreamSynchronize(b->stream));
   }
   if (steps == 0 && b->cur) {  // bring the state back to the first buffer
@@ -1265,12 +1270,14 @@ int cpml_batch_set_time_block(cpml_batch *b, int steps, int strip_width, int chu
     b->cur = 0;
   }
   b->tb = steps;
-  b->tb_ow = strip_width > 0 ? strip_width : 64 - 2 * g;  // every lane the ring leaves
-  if (steps > 0 && b->tb_ow > 64 - 2 * g) b->tb_ow = 64 - 2 * g;
+  // whole 64-byte sectors of the lanes the ring leaves, as cpml_gpu_set_time_block
+  const int widest = 64 - 2 * g, sector = 64 / b->esize;
+  b->tb_ow = strip_width > 0 ? strip_width
+                             : (widest >= sector ? widest / sector * sector : widest);
   b->tb_jc = chunk_rows > 0 ? chunk_rows : 40;
-  // slab items: half chunks from 48 rows up (128 shots of 512..2048, 64-row
-  // chunks: 32-row slab items 82.4 Gcell/s, 64: 80.5, 16: 78.0, 8: 70.9)
-  b->tb_jc_slab = b->tb_jc >= 48 ? (b->tb_jc + 1) / 2 : 0;
+  for (const Shot &s : b->shots)
+    b->tb_jc = std::min(b->tb_jc, cpml::tb2d_max_rows(s.ld, b->esize));
+  b->tb_js = cpml::tb2d_slab_rows(b->tb_jc);
   b->dirty = true;
   return CPML_OK;
 }

@@ -83,6 +83,16 @@ __device__ __forceinline__ T lane_prev(T x) {
   return dpp_shift<0x138>(x);  // wave_shr:1
 }
 
+// First index in [lo, hi) whose (ascending) value is not below v; hi if none.
+__device__ __forceinline__ int first_from(const int *a, int lo, int hi, int v) {
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (a[mid] < v) lo = mid + 1;
+    else hi = mid;
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
+}
+
 // Raw buffer resource over `bytes` bytes at p (gfx9 family word 3).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes,

@@ -22,6 +22,7 @@
 #include <string>
 
 #include "../../include/cpml_gpu.h"
+#include "cpml_constdiv.h"
 
 namespace cpml {
 
@@ -97,6 +98,7 @@ struct Step2D {
   long ld;   // row stride of fields
   long mld;  // row stride of y-slab memories
   T den_x, den_y, dt;
+  ConstDiv<T> div_x, div_y;  // division by den_x, den_y
   // source (0-based, isrc < 0: none) and step counter
   int isrc, jsrc;
   const T *fx, *fy;
@@ -160,9 +162,8 @@ struct Record {
   const int *idx;  // nrec offsets (i + j*ld + k*ps)
   T *sx, *sy, *sz;  // [nstep][nrec]
   int *step;
-  // the state is that of step it + skip (a launch that advanced skip + 1 steps
-  // and recorded the first skip itself): recorded as step it + skip, and the
-  // counter advances by skip + 1
+  // recorded as step it + skip, and the counter advances by skip + 1 (with
+  // nrec = 0 after launches that recorded skip + 1 steps themselves)
   int skip;
 };
 
@@ -179,32 +180,42 @@ struct TB3D {
   int ow, ty;          // owned columns and rows of a tile
   int box[4];
   int z0, z1, zn[3];
+  int ncls[8];  // tiles of each class (bit 0: x slabs or faces, bit 1: y, bit 2: z)
   // receivers of each x-y tile (t = ty * ntx + tx) sorted by plane: entries
   // [rec_start[t], rec_start[t+1]) of rec_i, rec_j, rec_k (0-based) and rec_slot
   const int *rec_start, *rec_i, *rec_j, *rec_k, *rec_slot;
   T *sisx, *sisy, *sisz;  // [nstep][nrec]
   int nrec;
+  int ahead;  // the launch's first step is *a.step + ahead
 };
 
+// Most rows of a 2D time-blocked chunk: an item addresses its rows and their
+// ring with unsigned 32-bit byte offsets.
+inline int tb2d_max_rows(long ld, size_t esize) {
+  const double rows = 4294967295.0 / ((double)ld * (double)esize) - 64.0;
+  return rows > 1e9 ? 1000000000 : rows < 1.0 ? 1 : (int)rows;
+}
+
 // Time-blocked 2D step: nt leapfrog steps per launch, state a -> the arrays
-// below.  Work items are (strip, chunk): 64-lane wavefronts owning `ow`
-// columns of a strip and the rows [jb, jb + jc) of a chunk.  Items whose
-// columns and rows (with their rings) avoid the absorbing slabs form the box
-// of strips [sx0, sx1) x chunks [cy0, cy1); the others run in the launch built
-// with the C-PML code.
+// below.  Work items are 64-lane wavefronts owning `ow` columns of a strip and
+// the rows [jb, je) of a chunk.  Strips [sx0, sx1) x rows [y0, y1) (with their
+// rings) lie strictly inside the grid and outside the absorbing slabs: cut into
+// chunks of jc rows; the rest into chunks of js rows, in the launch built with
+// the C-PML code.
 template <typename T>
 struct TB2D {
   Step2D<T> a;                   // state in (fields, memory variables, coefficients)
   T *vx, *vy, *sxx, *syy, *sxy;  // state out, interior origin
   T *mx[4], *my[4];              // memory variables out (layout of a.mx, a.my)
-  int ow, jc, nstrips, nchunks;
-  int sx0, sx1, cy0, cy1;
+  int ow, jc, js, nstrips;
+  int sx0, sx1, y0, y1;
   // receivers of each strip sorted by row: strip t owns entries
   // [rec_start[t], rec_start[t+1]) of rec_i, rec_j (0-based) and rec_slot
   // (the receiver's index in the seismogram rows)
   const int *rec_start, *rec_i, *rec_j, *rec_slot;
   T *sisx, *sisy;  // [nstep][nrec]
   int nrec;
+  int ahead;  // the launch's first step is *a.step + ahead
   // energy of every level (single grid, energy on): each item's sums over
   // its owned points inside the window ew (0-based i0, i1, j0, j1), written
   // to epart[(level * eslots + item) * 2 + {kinetic, potential}]
@@ -212,6 +223,69 @@ struct TB2D {
   int ew[4];
   int eslots;
 };
+
+// Default rows of a slab-free chunk: about 3000 items (the machine holds 4096
+// float or 2048 double wavefronts), between 16 rows (the ring rows of a march
+// cost as much from there on) and 64.  4096^2, order 4, float: 40, 64 and 100
+// rows 288, 286 and 300-320 us per 2 steps; 1701 x 1403, order 2, double: 12, 16,
+// 20 and 40 rows 92, 87, 87 and 111.
+inline int tb2d_default_rows(int nx, int ny, int ow) {
+  const double rows = (double)((nx + ow - 1) / ow) * ny / 3000.0;
+  return rows > 64.0 ? 64 : rows < 16.0 ? 16 : (int)rows;
+}
+// Rows of an item with C-PML code beside slab-free chunks of jc rows: these run
+// twice the instructions per row and start first, so they are shorter, but
+// every one marches its ring rows too.  4096^2 with 64-row chunks: 8, 16, 24 and
+// 32 rows 292, 287, 286 and 294 us.
+inline int tb2d_slab_rows(int jc) {
+  const int half = jc / 2;
+  return half > 24 ? 24 : half < 8 ? (jc < 8 ? jc : 8) : half;
+}
+// Default planes of a 3D time-blocked chunk: three workgroups per CU in all,
+// between 8 and 64 planes (two steps per launch, float: 96 x 80 x 72 with 8, 16
+// and 64 planes 83, 106 and 142 us per step, 200 x 180 x 160 with 8, 16, 32 and
+// 64 206, 175, 178 and 254, 320 x 300 x 310 with 16, 32 and 64 566, 523 and 532).
+inline int tb3d_default_planes(int nx, int ny, int nz, int ow, int rows) {
+  const double tiles = (double)((nx + ow - 1) / ow) * ((ny + rows - 1) / rows);
+  const double planes = tiles * nz / (3.0 * 256.0);
+  return planes > 64.0 ? 64 : planes < 8.0 ? 8 : (int)planes;
+}
+
+// Items of one grid by kind: slab-free; of the strips that touch an x slab or
+// face, all rows; of the other strips below y0 and from y1.
+struct Tb2dItems {
+  int clean, edge, cap;
+};
+template <typename T>
+__host__ __device__ inline Tb2dItems tb2d_items(const TB2D<T> &P) {
+  const int bx = P.sx1 - P.sx0, ny = P.a.ny;
+  Tb2dItems n;
+  n.clean = bx * ((P.y1 - P.y0 + P.jc - 1) / P.jc);
+  n.edge = (P.nstrips - bx) * ((ny + P.js - 1) / P.js);
+  n.cap = bx * ((P.y0 + P.js - 1) / P.js + (ny - P.y1 + P.js - 1) / P.js);
+  return n;
+}
+
+// Strips of ow columns whose points and ring of g columns avoid the slabs and
+// the faces: [t0, t1).
+inline void clean_strips(int n, int ow, int g, const Slab &s, int &t0, int &t1) {
+  const int nt = (n + ow - 1) / ow, wl = s.wl > 1 ? s.wl : 1, wr = s.wr > 1 ? s.wr : 1;
+  t0 = (wl + g + ow - 1) / ow;
+  t1 = t0;
+  while (t1 < nt && t1 * ow + ow - 1 + g < n - wr) ++t1;
+}
+
+// Fills nstrips, sx0, sx1, y0, y1 from a, ow (and the order and steps).
+template <typename T>
+inline void tb2d_split(int order, int nt, TB2D<T> &P) {
+  const Slab &sy = P.a.sy;
+  const int g = nt * order;  // rows the march reads below and above a chunk
+  P.nstrips = (P.a.nx + P.ow - 1) / P.ow;
+  clean_strips(P.a.nx, P.ow, nt * (order - 1), P.a.sx, P.sx0, P.sx1);
+  P.y0 = (sy.wl > 1 ? sy.wl : 1) + g;
+  P.y1 = P.a.ny - (sy.wr > 1 ? sy.wr : 1) - g;
+  if (P.y1 <= P.y0 || P.sx1 <= P.sx0) P.sx0 = P.sx1 = P.y0 = P.y1 = 0;
+}
 
 // Energy over a window, per step, accumulated in double.
 template <typename T>
@@ -308,30 +382,28 @@ template <typename T>
 hipError_t launch_record(const Record<T> &p, hipStream_t s);
 // nt steps per launch (3D, second order); tiles of ow columns x (nw - 2 nt)
 // rows marching through z chunks of at most kchunk planes
-// (the launches of tiles that touch a slab go to `side` when given, so they
-// run beside the slab-free tiles; the caller joins the two streams)
 template <typename T>
-hipError_t launch_tb3d(int nt, const TB3D<T> &p, hipStream_t s, hipStream_t side);
+hipError_t launch_tb3d(int nt, const TB3D<T> &p, hipStream_t s);
 int tb3d_max_nt(int prec);
-// nt steps per launch (2D, plain elastic); clean = items without C-PML code
+// nt steps per launch (2D, plain elastic)
 template <typename T>
-hipError_t launch_tb2d(int order, int nt, const TB2D<T> &p, hipStream_t s, hipStream_t side);
-// The energy of the NT levels of one time-blocked launch from its items' sums
-// (TB2D::epart), into e.out_kin / e.out_pot at steps *e.step .. + NT - 1.
+hipError_t launch_tb2d(int order, int nt, const TB2D<T> &p, hipStream_t s);
+// The energy of the levels of consecutive time-blocked launches from their
+// items' sums (TB2D::epart), into e.out_kin / e.out_pot at steps *e.step ...
 template <typename T>
-hipError_t launch_tb2d_energy(const Energy<T> &e, const double *epart, int eslots, int nt,
+hipError_t launch_tb2d_energy(const Energy<T> &e, const double *epart, int eslots, int nlevels,
                               hipStream_t s);
 // largest nt launch_tb2d has a kernel for, per order and precision
-int tb2d_max_nt(int order, int prec);
-// many grids: items (grid, strip, chunk) of one class (cls bit 0: the x
-// slabs' C-PML code, bit 1: the y slabs') from the descriptor table `grids`,
-// on `blocks` workgroups of 4 wavefronts
+inline int tb2d_max_nt(int order, int prec) {
+  if (prec == 8) return 2;
+  return order == 2 ? 4 : order == 4 ? 3 : 2;
+}
+// many grids: items (grid, strip, first row, end row) from the descriptor table
+// `grids`, on `waves` wavefronts; n[c] items of class c (bit 0: the x slabs'
+// C-PML code, bit 1: the y slabs'), in the order 3, 1, 2, 0
 template <typename T>
-hipError_t launch_tb2d_multi(int order, int nt, int cls, const TB2D<T> *grids,
-                             const int4 *items, int nitems, int blocks, hipStream_t s);
-// strips [box[0], box[1]) x chunks [box[2], box[3]) of one grid need no C-PML code
-void tb2d_clean_box(int order, int nt, int nx, int ny, int ow, int jc, const Slab &sx,
-                    const Slab &sy, int box[4]);
+hipError_t launch_tb2d_multi(int order, int nt, const TB2D<T> *grids, const int4 *items,
+                             const int (&n)[4], int waves, int ahead, hipStream_t s);
 template <typename T>
 hipError_t launch_energy(const Energy<T> &p, int nblocks, hipStream_t s);
 template <typename T>

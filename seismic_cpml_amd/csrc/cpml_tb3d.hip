@@ -14,7 +14,7 @@
 //     across lanes, y neighbours through LDS (written the iteration before:
 //     one barrier per plane, two buffers),
 //   * stores level NT (sigma at s - 2(NT-1), v at s - 2NT + 1) for the owned
-//     points and planes, and records the receivers of levels 1..NT-1.
+//     points and planes, and records the receivers of every level.
 // Every intermediate level stays in registers and LDS; HBM sees the state
 // read once (v 3, sigma 6, DELTAT*lambda, DELTAT*mu, DELTAT/rho: 12 words)
 // and written once (9 words) per NT steps, plus the slab memory variables
@@ -28,8 +28,10 @@
 // expressions, no FMA contraction), so results are bit-identical to them.
 //
 // Tiles are split by the axes along which their points and ring touch an
-// absorbing slab or a grid face; each class is one launch of the kernel built
-// with just the C-PML code and the predicates of those axes.
+// absorbing slab or a grid face; each class has code with just the C-PML terms
+// and the predicates of those axes.  All are one kernel, the classes with the
+// most of them first: a launch per class on streams of their own cost 20 us per
+// launch and 768^3 12.5 ms against 12.3.
 #include <algorithm>
 
 #include "cpml_device.h"
@@ -66,23 +68,15 @@ __device__ __forceinline__ int axis_count(int n, int c0, int c1) {
   return S ? n - (c1 - c0) : c1 - c0;
 }
 
-// Tile of this workgroup.  Along each axis the tiles (z: chunks) whose
-// points and ring avoid that axis' slabs form a range [cl[2a], cl[2a+1]);
-// the launch of class (SX, SY, SZ) covers the product of the clean (flag
-// false) or slab (flag true) tiles of each axis, x fastest, then y, then z,
-// in XCD-banded order (each XCD owns one contiguous band of the launch).
+// Tile t of class (SX, SY, SZ).  Along each axis the tiles (z: chunks) whose
+// points and ring avoid that axis' slabs form a range [cl[2a], cl[2a+1]); the
+// class covers the product of the clean (flag false) or slab (flag true) tiles
+// of each axis, x fastest, then y, then z.
 template <bool SX, bool SY, bool SZ, typename P>
-__device__ __forceinline__ Tile tb_tile(const P &Q, int nx, int ny, int nz, int kchunk) {
+__device__ __forceinline__ Tile tb_tile(const P &Q, int t, int nx, int ny, int nz, int kchunk) {
   const int ntx = (nx + Q.ow - 1) / Q.ow, nty = (ny + Q.ty - 1) / Q.ty;
-  const int ntz = Q.zn[0] + Q.zn[1] + Q.zn[2];
   const int cx = axis_count<SX>(ntx, Q.box[0], Q.box[1]);
   const int cy = axis_count<SY>(nty, Q.box[2], Q.box[3]);
-  const int cz = axis_count<SZ>(ntz, Q.zn[0], Q.zn[0] + Q.zn[1]);
-  const int nt = cx * cy * cz;
-  const int h = blockIdx.x;
-  const int xcd = h & 7, loc = h >> 3;
-  const int q = nt >> 3, rem = nt & 7;
-  const int t = xcd * q + min(xcd, rem) + loc;
   Tile f;
   f.tx = axis_tile<SX>(t % cx, Q.box[0], Q.box[1]);
   f.ty = axis_tile<SY>((t / cx) % cy, Q.box[2], Q.box[3]);
@@ -153,16 +147,13 @@ __device__ __forceinline__ void st_mem(T *base, unsigned byte_off, T x) {
 //    selections, and K is read only where it is not 1.
 // Loads two planes ahead (128 registers, 15 spilled): 16.8 against 15.1.
 template <typename T, int NT, int NW, bool SX, bool SY, bool SZ>
-__global__ __launch_bounds__(64 * NW) void k_tb3d(TB3D<T> P) {
+__device__ __forceinline__ void tb3d_tile(const TB3D<T> &P, int t, T *xl) {
   constexpr bool SLAB = SX || SY || SZ;
   constexpr int NL = NT > 1 ? NT - 1 : 1;      // memory-variable windows (levels 1..NT-1)
   constexpr int NS = 6 * NT;                   // LDS slots per buffer
-  // one row of padding at both ends: the row below row 0 of slot 0 and above
-  // the last row of the last slot are read (by ring rows only)
-  __shared__ T xl[2 * NS * NW * 64 + 128];
   const Step3D<T> &p = P.a;
   const int nx = p.nx, ny = p.ny, nz = p.nz;
-  const Tile ft = tb_tile<SX, SY, SZ>(P, nx, ny, nz, p.kchunk);
+  const Tile ft = tb_tile<SX, SY, SZ>(P, t, nx, ny, nz, p.kchunk);
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = ft.i0 - NT + lane, j = ft.j0 - NT + w;
@@ -302,22 +293,21 @@ __global__ __launch_bounds__(64 * NW) void k_tb3d(TB3D<T> P) {
   }
   __syncthreads();
 
-  // receivers of this tile: a cursor per recorded level (planes only
-  // increase), the plane of the next one held in a register
+  // receivers of this tile: a cursor per level (planes only increase), the
+  // plane of the next one held in a register
   const int tix = ft.ty * ((nx + P.ow - 1) / P.ow) + ft.tx;
   constexpr int kNever = 0x7fffffff;
-  int rc1 = 0, cur[NL], rk[NL];
+  int rc1 = 0, cur[NT], rk[NT];
 #pragma unroll
-  for (int m = 0; m < NL; ++m) cur[m] = 0, rk[m] = kNever;
-  if (NT > 1 && P.nrec > 0) {
+  for (int m = 0; m < NT; ++m) cur[m] = 0, rk[m] = kNever;
+  if (P.nrec > 0) {
     rc1 = __builtin_amdgcn_readfirstlane(P.rec_start[tix + 1]);
-    int c = __builtin_amdgcn_readfirstlane(P.rec_start[tix]);
-    while (c < rc1 && P.rec_k[c] < kb) ++c;
+    const int c = first_from(P.rec_k, P.rec_start[tix], rc1, kb);
     const int k0 = c < rc1 ? __builtin_amdgcn_readfirstlane(P.rec_k[c]) : kNever;
 #pragma unroll
-    for (int m = 0; m < NL; ++m) cur[m] = c, rk[m] = k0;
+    for (int m = 0; m < NT; ++m) cur[m] = c, rk[m] = k0;
   }
-  const int it0 = *p.step;
+  const int it0 = *p.step + P.ahead;  // this launch's first step
   // the source's column: its plane if this wavefront holds its row
   const int ksrc = (j >= 0 && j == p.jsrc) ? p.ksrc : -1000;
 
@@ -512,6 +502,23 @@ __global__ __launch_bounds__(64 * NW) void k_tb3d(TB3D<T> P) {
             (SZ && (qk == 0 || qk == nz - 1)))
           vn[0] = vn[1] = vn[2] = T(0);
       }
+      // receivers of step it0 + m - 1 on plane qk (owned points only)
+      if (qk == rk[m - 1] && qk < ke) {
+        const KArgs Q = args();
+        int c = cur[m - 1], nk = qk;
+        while (nk == qk) {
+          if (Q->rec_i[c] == i && Q->rec_j[c] == j && own) {
+            const long o = (long)(it0 + m - 2) * Q->nrec + Q->rec_slot[c];
+            Q->sisx[o] = vn[0];
+            Q->sisy[o] = vn[1];
+            if (Q->sisz) Q->sisz[o] = vn[2];
+          }
+          ++c;
+          nk = c < rc1 ? __builtin_amdgcn_readfirstlane(Q->rec_k[c]) : kNever;
+        }
+        cur[m - 1] = c;
+        rk[m - 1] = nk;
+      }
       if constexpr (m < NT) {
 #pragma unroll
         for (int f = 0; f < 3; ++f) V[m][f][cm1] = vn[f];
@@ -526,23 +533,6 @@ __global__ __launch_bounds__(64 * NW) void k_tb3d(TB3D<T> P) {
         wr[(ss + 3) * SLOT] = vn[0];  // y neighbours of v^m at plane qk
         wr[(ss + 4) * SLOT] = vn[1];
         wr[(ss + 5) * SLOT] = vn[2];
-        // receivers of step it0 + m - 1 on plane qk (owned points only)
-        if (qk == rk[m - 1] && qk < ke) {
-          const KArgs Q = args();
-          int c = cur[m - 1], nk = qk;
-          while (nk == qk) {
-            if (Q->rec_i[c] == i && Q->rec_j[c] == j && own) {
-              const long o = (long)(it0 + m - 2) * Q->nrec + Q->rec_slot[c];
-              Q->sisx[o] = vn[0];
-              Q->sisy[o] = vn[1];
-              if (Q->sisz) Q->sisz[o] = vn[2];
-            }
-            ++c;
-            nk = c < rc1 ? __builtin_amdgcn_readfirstlane(Q->rec_k[c]) : kNever;
-          }
-          cur[m - 1] = c;
-          rk[m - 1] = nk;
-        }
       } else if (qk >= kb && qk < ke && own) {
         const unsigned o = pl(qk);
         st_at(P.vx + corner, o, vn[0]);
@@ -578,6 +568,41 @@ __global__ __launch_bounds__(64 * NW) void k_tb3d(TB3D<T> P) {
   }
 }
 
+// Every tile of the grid in one launch, class by class: all axes' slabs first
+// (the most code), the slab-free tiles last; P.ncls[c] tiles of class c (bit 0
+// x, bit 1 y, bit 2 z).  Each XCD gets one contiguous band of every class.  One
+// launch, because a workgroup fills a CU whatever its class (LDS), and launches
+// of single classes leave the machine idle at their ends: seven small ones in
+// a row cost more than the step itself on small grids.
+template <typename T, int NT, int NW>
+__global__ __launch_bounds__(64 * NW) void k_tb3d(TB3D<T> P) {
+  // one row of padding at both ends: the row below row 0 of slot 0 and above
+  // the last row of the last slot are read (by ring rows only)
+  __shared__ T xl[2 * 6 * NT * NW * 64 + 128];
+  const int xcd = blockIdx.x & 7;
+  int u = blockIdx.x >> 3;
+#pragma unroll 1
+  for (int c = 7; c >= 0; --c) {
+    const int q = P.ncls[c] >> 3, r = P.ncls[c] & 7, n = q + (xcd < r ? 1 : 0);
+    if (u >= n) {
+      u -= n;
+      continue;
+    }
+    const int t = xcd * q + min(xcd, r) + u;
+    switch (c) {
+      case 7: tb3d_tile<T, NT, NW, true, true, true>(P, t, xl); break;
+      case 6: tb3d_tile<T, NT, NW, false, true, true>(P, t, xl); break;
+      case 5: tb3d_tile<T, NT, NW, true, false, true>(P, t, xl); break;
+      case 4: tb3d_tile<T, NT, NW, false, false, true>(P, t, xl); break;
+      case 3: tb3d_tile<T, NT, NW, true, true, false>(P, t, xl); break;
+      case 2: tb3d_tile<T, NT, NW, false, true, false>(P, t, xl); break;
+      case 1: tb3d_tile<T, NT, NW, true, false, false>(P, t, xl); break;
+      default: tb3d_tile<T, NT, NW, false, false, false>(P, t, xl);
+    }
+    return;
+  }
+}
+
 // Tiles along one axis (size B, extent n, slab widths wl, wr) whose points and
 // ring of g avoid both slabs: [t0, t1), empty when t1 <= t0.
 void clean_tiles(int n, int B, int g, int wl, int wr, int &t0, int &t1) {
@@ -593,19 +618,8 @@ void clean_tiles(int n, int B, int g, int wl, int wr, int &t0, int &t1) {
   }
 }
 
-template <typename T, int NT, int NW, bool SX, bool SY, bool SZ>
-void tb3d_class(const TB3D<T> &P, const int (&n)[3], hipStream_t s) {
-  const int cx = SX ? n[0] - (P.box[1] - P.box[0]) : P.box[1] - P.box[0];
-  const int cy = SY ? n[1] - (P.box[3] - P.box[2]) : P.box[3] - P.box[2];
-  const int cz = SZ ? n[2] - P.zn[1] : P.zn[1];
-  const long nt = (long)cx * cy * cz;
-  if (nt > 0)
-    hipLaunchKernelGGL((k_tb3d<T, NT, NW, SX, SY, SZ>), dim3((unsigned)nt), dim3(64 * NW), 0, s,
-                       P);
-}
-
 template <typename T, int NT, int NW>
-hipError_t tb3d_launch(const TB3D<T> &P0, hipStream_t s, hipStream_t side) {
+hipError_t tb3d_launch(const TB3D<T> &P0, hipStream_t s) {
   TB3D<T> P = P0;
   const Step3D<T> &p = P.a;
   P.ty = NW - 2 * NT;
@@ -627,17 +641,15 @@ hipError_t tb3d_launch(const TB3D<T> &P0, hipStream_t s, hipStream_t side) {
   if (P.box[3] < P.box[2]) P.box[2] = P.box[3] = 0;
   const int n[3] = {(p.nx + P.ow - 1) / P.ow, (p.ny + P.ty - 1) / P.ty,
                     P.zn[0] + P.zn[1] + P.zn[2]};
-  // slab classes first on the side stream (the corners, with the most code,
-  // start earliest), the slab-free class on the main stream
-  hipStream_t t = side ? side : s;
-  tb3d_class<T, NT, NW, true, true, true>(P, n, t);
-  tb3d_class<T, NT, NW, true, true, false>(P, n, t);
-  tb3d_class<T, NT, NW, true, false, true>(P, n, t);
-  tb3d_class<T, NT, NW, false, true, true>(P, n, t);
-  tb3d_class<T, NT, NW, true, false, false>(P, n, t);
-  tb3d_class<T, NT, NW, false, true, false>(P, n, t);
-  tb3d_class<T, NT, NW, false, false, true>(P, n, t);
-  tb3d_class<T, NT, NW, false, false, false>(P, n, s);
+  long most = 0;  // tiles of the XCD that gets most
+  for (int c = 0; c < 8; ++c) {
+    const int cx = c & 1 ? n[0] - (P.box[1] - P.box[0]) : P.box[1] - P.box[0];
+    const int cy = c & 2 ? n[1] - (P.box[3] - P.box[2]) : P.box[3] - P.box[2];
+    const int cz = c & 4 ? n[2] - P.zn[1] : P.zn[1];
+    P.ncls[c] = cx * cy * cz;
+    most += (P.ncls[c] + 7) / 8;
+  }
+  hipLaunchKernelGGL((k_tb3d<T, NT, NW>), dim3((unsigned)(8 * most)), dim3(64 * NW), 0, s, P);
   return hipGetLastError();
 }
 
@@ -648,14 +660,14 @@ int tb3d_max_nt(int) { return 2; }
 // rows per workgroup: 16 wavefronts in float, 8 in double (LDS: 6 NT values
 // per point and buffer)
 template <typename T>
-hipError_t launch_tb3d(int nt, const TB3D<T> &p, hipStream_t s, hipStream_t side) {
+hipError_t launch_tb3d(int nt, const TB3D<T> &p, hipStream_t s) {
   constexpr int NW = sizeof(T) == 4 ? 16 : 8;
-  if (nt == 1) return tb3d_launch<T, 1, NW>(p, s, side);
-  if (nt == 2) return tb3d_launch<T, 2, NW>(p, s, side);
+  if (nt == 1) return tb3d_launch<T, 1, NW>(p, s);
+  if (nt == 2) return tb3d_launch<T, 2, NW>(p, s);
   return hipErrorInvalidValue;
 }
 
-template hipError_t launch_tb3d<float>(int, const TB3D<float> &, hipStream_t, hipStream_t);
-template hipError_t launch_tb3d<double>(int, const TB3D<double> &, hipStream_t, hipStream_t);
+template hipError_t launch_tb3d<float>(int, const TB3D<float> &, hipStream_t);
+template hipError_t launch_tb3d<double>(int, const TB3D<double> &, hipStream_t);
 
 }  // namespace cpml
