@@ -126,6 +126,8 @@ long round_up(long v, long m) { return (v + m - 1) / m * m; }
 
 }  // namespace
 
+constexpr size_t kStageBytes = 4 << 20;
+
 struct cpml_solver {
   int ndim = 2, order = 2, prec = 8, nx = 0, ny = 0, nz = 1, npml = 0, nstep = 0;
   double dx = 0, dy = 0, dz = 0, dt = 0;
@@ -188,6 +190,8 @@ struct cpml_solver {
   double last_ms = 0;
   double last_vnorm = 0;
   int host_step = 0;
+  void *stage[2] = {};          // pinned buffers of copy_padded, allocated at its first use
+  hipEvent_t stage_ev[2] = {};  // recorded after the kernel that last used each
   cpml_abc_net *abc = nullptr;  // learned boundary corrector (not owned)
   void *abc_corr = nullptr;     // its per-step correction buffer
   // 2D viscoelastic attenuation (cpml_gpu_set_attenuation)
@@ -296,32 +300,93 @@ size_t host_at(const cpml_solver *h, long i, long j, long k) {
   return (size_t)(i + h->hlo) + host_x(h) * ((size_t)(j + h->hlo) + host_y(h) * kk);
 }
 
+// Rows [row0, row0 + nrows) of the grid (row r: j = r % ny, k = r / ny) between a
+// padded array and a dense buffer in host memory: one wavefront per row.
+template <typename T, bool PACK>
+__global__ __launch_bounds__(256) void k_stage_rows(T *grid, T *dense, int nx, int ny, long ld,
+                                                    long ps, int row0, int nrows) {
+  const int r = blockIdx.x * 4 + threadIdx.x / 64;
+  if (r >= nrows) return;
+  const int k = (row0 + r) / ny, j = (row0 + r) - k * ny;
+  T *g = grid + j * ld + k * ps;
+  T *d = dense + (long)r * nx;
+  for (int i = threadIdx.x % 64; i < nx; i += 64) {
+    if (PACK) d[i] = g[i];
+    else g[i] = d[i];
+  }
+}
+
+int stage_rows(cpml_solver *h, bool pack, void *grid_alloc, void *dense, int row0, int nrows) {
+  char *g = static_cast<char *>(grid_alloc) + h->base * h->esize;
+  const dim3 grid((nrows + 3) / 4), block(256);
+  auto go = [&](auto kernel, auto *p) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, h->stream, p, (decltype(p))dense, h->nx, h->ny,
+                       h->ld, h->ps, row0, nrows);
+  };
+  if (h->esize == 4) pack ? go(k_stage_rows<float, true>, (float *)g)
+                          : go(k_stage_rows<float, false>, (float *)g);
+  else pack ? go(k_stage_rows<double, true>, (double *)g)
+            : go(k_stage_rows<double, false>, (double *)g);
+  HIPCHK(h, hipGetLastError());
+  return CPML_OK;
+}
+
 // Copy the interior of a host grid array into / out of a padded device array
-// (ghost cells of the host array are neither read nor written).
-int upload_padded(cpml_solver *h, void *dst_alloc, const void *src) {
-  const size_t es = h->esize;
-  char *dst = static_cast<char *>(dst_alloc) + h->base * es;
-  const char *s = static_cast<const char *>(src);
-  const int nzz = h->ndim == 3 ? h->nz : 1;
-  for (int k = 0; k < nzz; ++k)
-    HIPCHK(h, hipMemcpy2DAsync(dst + k * h->ps * es, h->ld * es, s + host_at(h, 0, 0, k) * es,
-                               host_x(h) * es, h->nx * es, h->ny, hipMemcpyHostToDevice,
-                               h->stream));
+// (ghost cells of the host array are neither read nor written).  The device
+// packs stretches of rows straight into (or unpacks them from) one of two
+// pinned buffers of 4 MiB while the host copies the other: a pitched copy to
+// ordinary memory costs the runtime 6 us per row and 500 us per plane (50 float steps
+// at 96 x 80 x 72 and three fields read: 123 -> 3.8 ms; 100 at 1013 x 1187 and
+// two fields: 20.3 -> 3.3 ms).
+int copy_padded(cpml_solver *h, bool download, void *grid_alloc, char *host) {
+  const size_t row = h->nx * h->esize;
+  const int rows = h->ny * (h->ndim == 3 ? h->nz : 1);
+  const int per = (int)std::clamp<size_t>(kStageBytes / row, 1, rows);
+  for (int q = 0; q < 2; ++q) {
+    if (!h->stage_ev[q])
+      HIPCHK(h, hipEventCreateWithFlags(&h->stage_ev[q], hipEventDisableTiming));
+    if (!h->stage[q])
+      HIPCHK(h, hipHostMalloc(&h->stage[q], per * row, hipHostMallocDefault));
+  }
+  auto host_rows = [&](int row0, int n, char *dense) {
+    for (int r = 0; r < n; ++r) {
+      const int k = (row0 + r) / h->ny, j = row0 + r - k * h->ny;
+      char *p = host + host_at(h, 0, j, k) * h->esize;
+      // rows without ghost cells between them in one copy
+      const int run = host_x(h) == (size_t)h->nx ? std::min(n - r, h->ny - j) : 1;
+      if (download) std::memcpy(p, dense + r * row, run * row);
+      else std::memcpy(dense + r * row, p, run * row);
+      r += run - 1;
+    }
+  };
+  int rc = 0;
+  const int parts = (rows + per - 1) / per;
+  for (int c = 0; c < parts + (download ? 1 : 0); ++c) {
+    const int b = c & 1, row0 = c * per, n = std::min(per, rows - row0);
+    if (!download) {
+      if (c >= 2) HIPCHK(h, hipEventSynchronize(h->stage_ev[b]));
+      host_rows(row0, n, static_cast<char *>(h->stage[b]));
+    }
+    if (c < parts) {
+      if ((rc = stage_rows(h, download, grid_alloc, h->stage[b], row0, n))) return rc;
+      HIPCHK(h, hipEventRecord(h->stage_ev[b], h->stream));
+    }
+    if (download && c > 0) {
+      HIPCHK(h, hipEventSynchronize(h->stage_ev[b ^ 1]));
+      host_rows(row0 - per, std::min(per, rows - row0 + per),
+                static_cast<char *>(h->stage[b ^ 1]));
+    }
+  }
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return CPML_OK;
 }
 
+int upload_padded(cpml_solver *h, void *dst_alloc, const void *src) {
+  return copy_padded(h, false, dst_alloc, static_cast<char *>(const_cast<void *>(src)));
+}
+
 int download_padded(cpml_solver *h, const void *src_alloc, void *dst) {
-  const size_t es = h->esize;
-  const char *src = static_cast<const char *>(src_alloc) + h->base * es;
-  char *d = static_cast<char *>(dst);
-  const int nzz = h->ndim == 3 ? h->nz : 1;
-  for (int k = 0; k < nzz; ++k)
-    HIPCHK(h, hipMemcpy2DAsync(d + host_at(h, 0, 0, k) * es, host_x(h) * es,
-                               src + k * h->ps * es, h->ld * es, h->nx * es, h->ny,
-                               hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  return CPML_OK;
+  return copy_padded(h, true, const_cast<void *>(src_alloc), static_cast<char *>(dst));
 }
 
 bool field_valid(const cpml_solver *h, int which) {
@@ -1265,6 +1330,10 @@ int cpml_gpu_finalize(cpml_solver *h) {
   for (auto g : h->gexec)
     if (g) (void)hipGraphExecDestroy(g);
   for (hipEvent_t e : h->evpool) (void)hipEventDestroy(e);
+  for (int q = 0; q < 2; ++q) {
+    if (h->stage_ev[q]) (void)hipEventDestroy(h->stage_ev[q]);
+    if (h->stage[q]) (void)hipHostFree(h->stage[q]);
+  }
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   for (void *p : h->allocs) (void)hipFree(p);
