@@ -161,7 +161,8 @@ int cpml_velocity_norm_noalloc(int prec, int ndim, int NX, int NY, int NZ, const
 
 /* Steps captured per HIP graph replay (default 16; 0 = launch eagerly). */
 int cpml_gpu_set_graph_steps(cpml_solver *h, int steps);
-/* Tiling: planes per block along z (3D, default 8) and rows of 64 points per
+/* Tiling: planes per block along z (3D; default 2 to 32 by
+ * the grid and the order) and rows of 64 points per
  * tile (4, 8 or 16; default 4; 2D also 32 or 64, walked by 16-row blocks; the
  * fused 3D step owns 62-point rows, 6 of them per block for 4 or 8 and 14 for
  * 16).  Results do not depend on either. */

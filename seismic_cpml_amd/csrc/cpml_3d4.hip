@@ -17,62 +17,98 @@
 // and the stress increment is (sum of coefficient * derivative) * DELTAT.
 //
 // Mapping: a 64 x TY block (TY = 4, 8 or 16 rows, the handle's tile) covers
-// 64 points along x (one wavefront per row, coalesced); each (i, j) column
-// marches through a chunk of z
+// 64 columns (tile3 says which); each (i, j) column marches through a chunk of z
 // planes.  The column's own z neighbours are carried in registers from plane
 // to plane (one new plane per field and step); the x and y neighbours are
 // read from global memory and come from the same or adjacent rows of the
-// block, so they hit in L1/L2.  Profile values of the column are loaded once.  Tiles are
-// dealt to the 8 XCDs in contiguous bands (neighbouring tiles share an L2).
+// block, so they hit in L1/L2.  Profile values of the column are loaded once.
+//
+// Bound by HBM: 30 words per point and step at 3.3 TB/s (210 x 800 x 220, float),
+// a rate that the loads in flight set.  So the loads of the next plane, memory
+// variables included, go into a second register set before this plane's
+// arithmetic and stores, through buffers whose offsets the scalar unit adds:
+// 1536 -> 1382 us per step, double 3203 -> 2746, 256^3 float 627 -> 583.
 #include <hip/hip_runtime.h>
 
+#include "cpml_constdiv.h"
 #include "cpml_device.h"
 #include "cpml_internal.h"
 
 namespace cpml {
 namespace {
 
-struct Col4 {
-  int i, j, kb, ke;
-  bool ok;
-};
+// Doubles number the columns through the plane (tile3).
+template <typename T>
+constexpr bool kFlat4 = sizeof(T) == 8;
 
-template <int TY4>
-__device__ __forceinline__ Col4 col4(int nx, int ny, int nz, int kchunk) {
-  const int ntx = (nx + BX - 1) / BX, nty = (ny + TY4 - 1) / TY4;
-  const int ntz = (nz + kchunk - 1) / kchunk;
-  const int nt = ntx * nty * ntz;
-  const int h = blockIdx.x;
-  const int xcd = h & 7, loc = h >> 3;
-  const int q = nt >> 3, r = nt & 7;
-  const int t = xcd * q + min(xcd, r) + loc;  // band of XCD `xcd`, position loc
-  const int tx = t % ntx, rest = t / ntx;
-  const int ty = rest % nty, tz = zchunk_of(rest / nty, ntz);
-  Col4 c;
-  c.i = tx * BX + threadIdx.x;
-  c.j = ty * TY4 + threadIdx.y;
-  c.kb = tz * kchunk;
-  c.ke = min(c.kb + kchunk, nz);
-  c.ok = c.i < nx && c.j < ny;
-  return c;
-}
-
-// (27 fp - 27 f0 - fpp + fm) * od / 24, in the reference's order
+// (27 fp - 27 f0 - fpp + fm) * od, in the reference's order; its callers divide
+// by 24
 template <typename T>
 __device__ __forceinline__ T d4(T fp, T f0, T fpp, T fm, T od) {
-  return (((T(27) * fp - T(27) * f0) - fpp) + fm) * od / T(24);
+  return (((T(27) * fp - T(27) * f0) - fpp) + fm) * od;
 }
 
-// Every read of a point is issued before its arithmetic and stores (all
-// offsets stay inside the two halo cells of each side, so the loads are
-// unconditional), through restrict-qualified pointers: the loads of one
-// point are in flight together instead of waiting behind its stores.
+// The chunk's planes kb - 2 .. ke + 1 as buffers: per-lane 32-bit byte offset
+// of the column, scalar offset of the plane and row, x shift in the
+// instruction (the host keeps a chunk's planes and 8 more below 4 GiB).
+template <typename T>
+struct Chunk4 {
+  unsigned v0, ldb, psb, bytes;
+  long origin;
+  __device__ Chunk4(const Step3D<T> &p, const Tile3 &c) {
+    ldb = (unsigned)(p.ld * sizeof(T));
+    psb = (unsigned)(p.ps * sizeof(T));
+    bytes = (unsigned)((c.ke - c.kb + 4) * p.ps * sizeof(T));
+    origin = (long)(c.kb - 2 + p.R) * p.ps;
+    v0 = (unsigned)(((c.j - 2 + p.R) * p.ld + p.xpad + c.i - 2) * sizeof(T));
+  }
+  __device__ __amdgpu_buffer_rsrc_t rsrc(const T *interior_origin, long base) const {
+    return make_rsrc(interior_origin - base + origin, bytes);
+  }
+  // f(i + dx, j + dy, k + dz) of buffer plane kk = k - kb + 2
+  __device__ T ld(__amdgpu_buffer_rsrc_t r, int dx, int dy, int dz, int kk) const {
+    return BufOp<T>::ld(r, v0 + (2 + dx) * (unsigned)sizeof(T),
+                        (unsigned)(kk + dz) * psb + (unsigned)(2 + dy) * ldb);
+  }
+  __device__ void st(T x, __amdgpu_buffer_rsrc_t r, int kk) const {
+    BufOp<T>::st(x, r, v0 + 2 * (unsigned)sizeof(T), (unsigned)kk * psb + 2 * ldb);
+  }
+};
+
+// C-PML of one axis on three derivatives of a point inside its slab, with the
+// memory variables m read a plane ahead: psi <- b*psi + a*d ; d <- d/K + psi
+// where `in` (the update's loop range).
+template <typename T>
+__device__ __forceinline__ void pml4(bool in, T &d, T m, T *psi, T a, T b, T K) {
+  if (!in) return;
+  m = b * m + a * d;
+  *psi = m;
+  d = over_k(d, K) + m;
+}
+
+// Values the stress kernel reads at plane k.
+template <typename T>
+struct SPlane4 {
+  T vx_zpp, vx_xp, vx_xpp, vx_xm, vx_yp, vx_ypp, vx_ym;
+  T vy_zpp, vy_xm, vy_xp, vy_xmm, vy_ym, vy_yp, vy_ymm;
+  T vz_zp, vz_xm, vz_xp, vz_xmm, vz_yp, vz_ypp, vz_ym;
+  T mu, lam, xx, yy, zz, xy, xz, yz;
+  T px[3], py[3], pz[3];  // memory variables, where the point lies in the axis' slab
+};
+
+// Float: at least 4 waves per SIMD (128 VGPRs against 132 unbounded, which
+// leave 3); more would spill.
 template <typename T, int TY4>
-__global__ __launch_bounds__(BX *TY4) void k_stress3d4(Step3D<T> p) {
-  const Col4 c = col4<TY4>(p.nx, p.ny, p.nz, p.kchunk);
+__global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_stress3d4(Step3D<T> p) {
+  const Tile3 c = tile3<TY4, kFlat4<T>>(p);
   if (!c.ok) return;
   const int i = c.i, j = c.j, nx = p.nx, ny = p.ny, nz = p.nz;
-  const long ld = p.ld, ps = p.ps;
+  const Chunk4<T> g(p, c);
+  const auto rvx = g.rsrc(p.vx, p.base), rvy = g.rsrc(p.vy, p.base), rvz = g.rsrc(p.vz, p.base);
+  const auto rla = g.rsrc(p.lam, p.base), rmu = g.rsrc(p.mu, p.base);
+  const auto rxx = g.rsrc(p.sxx, p.base), ryy = g.rsrc(p.syy, p.base);
+  const auto rzz = g.rsrc(p.szz, p.base), rxy = g.rsrc(p.sxy, p.base);
+  const auto rxz = g.rsrc(p.sxz, p.base), ryz = g.rsrc(p.syz, p.base);
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
   const long mxo = p.sx.at(i, j, ny), mxs = (long)p.sx.w * ny;
   const long myo = i + p.mld * p.sy.s(j), mys = p.mld * p.sy.w;
@@ -93,90 +129,131 @@ __global__ __launch_bounds__(BX *TY4) void k_stress3d4(Step3D<T> p) {
     ya = p.py.a[j]; yb = p.py.b[j]; yK = p.py.K[j];
     yah = p.py.ah[j]; ybh = p.py.bh[j]; yKh = p.py.Kh[j];
   }
+  auto load = [&](SPlane4<T> &L, int k) {
+    const auto Q = kernarg<Step3D<T>>();
+    const int kk = k - c.kb + 2;
+    L.vx_zpp = g.ld(rvx, 0, 0, 2, kk);
+    L.vy_zpp = g.ld(rvy, 0, 0, 2, kk);
+    L.vz_zp = g.ld(rvz, 0, 0, 1, kk);
+    L.vx_xp = g.ld(rvx, 1, 0, 0, kk), L.vx_xpp = g.ld(rvx, 2, 0, 0, kk);
+    L.vx_xm = g.ld(rvx, -1, 0, 0, kk);
+    L.vx_yp = g.ld(rvx, 0, 1, 0, kk), L.vx_ypp = g.ld(rvx, 0, 2, 0, kk);
+    L.vx_ym = g.ld(rvx, 0, -1, 0, kk);
+    L.vy_xm = g.ld(rvy, -1, 0, 0, kk), L.vy_xp = g.ld(rvy, 1, 0, 0, kk);
+    L.vy_xmm = g.ld(rvy, -2, 0, 0, kk);
+    L.vy_ym = g.ld(rvy, 0, -1, 0, kk), L.vy_yp = g.ld(rvy, 0, 1, 0, kk);
+    L.vy_ymm = g.ld(rvy, 0, -2, 0, kk);
+    L.vz_xm = g.ld(rvz, -1, 0, 0, kk), L.vz_xp = g.ld(rvz, 1, 0, 0, kk);
+    L.vz_xmm = g.ld(rvz, -2, 0, 0, kk);
+    L.vz_yp = g.ld(rvz, 0, 1, 0, kk), L.vz_ypp = g.ld(rvz, 0, 2, 0, kk);
+    L.vz_ym = g.ld(rvz, 0, -1, 0, kk);
+    L.mu = g.ld(rmu, 0, 0, 0, kk), L.lam = g.ld(rla, 0, 0, 0, kk);
+    L.xx = g.ld(rxx, 0, 0, 0, kk), L.yy = g.ld(ryy, 0, 0, 0, kk);
+    L.zz = g.ld(rzz, 0, 0, 0, kk), L.xy = g.ld(rxy, 0, 0, 0, kk);
+    L.xz = g.ld(rxz, 0, 0, 0, kk), L.yz = g.ld(ryz, 0, 0, 0, kk);
+    if (inx) {
+      const long m = mxo + k * mxs;
+      L.px[0] = Q->mx[0][m], L.px[1] = Q->mx[1][m], L.px[2] = Q->mx[2][m];
+    }
+    if (iny) {
+      const long m = myo + k * mys;
+      L.py[0] = Q->my[0][m], L.py[1] = Q->my[1][m], L.py[2] = Q->my[2][m];
+    }
+    if (p.sz.in(k)) {
+      const long m = mzo + p.sz.s(k) * mzs;
+      L.pz[0] = Q->mz[0][m], L.pz[1] = Q->mz[1][m], L.pz[2] = Q->mz[2][m];
+    }
+  };
   // the column's own z neighbours, carried from plane to plane
-  const long q0 = i + j * ld + c.kb * ps;
-  T vx_zm = p.vx[q0 - ps], vx0 = p.vx[q0], vx_zp = p.vx[q0 + ps];
-  T vy_zm = p.vy[q0 - ps], vy0 = p.vy[q0], vy_zp = p.vy[q0 + ps];
-  T vz_zmm = p.vz[q0 - 2 * ps], vz_zm = p.vz[q0 - ps], vz0 = p.vz[q0];
-  for (int k = c.kb; k < c.ke; ++k) {
-    const long q = i + j * ld + k * ps;
-    const T *__restrict__ vx = p.vx + q;
-    const T *__restrict__ vy = p.vy + q;
-    const T *__restrict__ vz = p.vz + q;
-    T *__restrict__ sxx = p.sxx + q;
-    T *__restrict__ syy = p.syy + q;
-    T *__restrict__ szz = p.szz + q;
-    T *__restrict__ sxy = p.sxy + q;
-    T *__restrict__ sxz = p.sxz + q;
-    T *__restrict__ syz = p.syz + q;
-    const T vx_xp = vx[1], vx_xpp = vx[2], vx_xm = vx[-1];
-    const T vx_yp = vx[ld], vx_ypp = vx[2 * ld], vx_ym = vx[-ld];
-    const T vx_zpp = vx[2 * ps];
-    const T vy_xm = vy[-1], vy_xp = vy[1], vy_xmm = vy[-2];
-    const T vy_ym = vy[-ld], vy_yp = vy[ld], vy_ymm = vy[-2 * ld];
-    const T vy_zpp = vy[2 * ps];
-    const T vz_xm = vz[-1], vz_xp = vz[1], vz_xmm = vz[-2];
-    const T vz_yp = vz[ld], vz_ypp = vz[2 * ld], vz_ym = vz[-ld];
-    const T vz_zp = vz[ps];
-    const T mu = p.mu[q], lam = p.lam[q];
-    const T oxx = sxx[0], oyy = syy[0], ozz = szz[0], oxy = sxy[0], oxz = sxz[0], oyz = syz[0];
+  constexpr int k0 = 2;  // buffer plane of kb
+  T vx_zm = g.ld(rvx, 0, 0, -1, k0), vx0 = g.ld(rvx, 0, 0, 0, k0), vx_zp = g.ld(rvx, 0, 0, 1, k0);
+  T vy_zm = g.ld(rvy, 0, 0, -1, k0), vy0 = g.ld(rvy, 0, 0, 0, k0), vy_zp = g.ld(rvy, 0, 0, 1, k0);
+  T vz_zmm = g.ld(rvz, 0, 0, -2, k0), vz_zm = g.ld(rvz, 0, 0, -1, k0);
+  T vz0 = g.ld(rvz, 0, 0, 0, k0);
+  // one plane: L holds its values, N receives the next one's.  The caller
+  // alternates two sets, so no copy waits for the loads in flight, and they are
+  // issued before this plane's stores, so waiting for them does not wait for
+  // those.
+  auto plane = [&](int k, const SPlane4<T> &L, SPlane4<T> &N) {
+    const auto Q = kernarg<Step3D<T>>();
+    const int kk = k - c.kb + 2;
+    load(N, min(k + 1, c.ke - 1));
+    const T mu = L.mu, lam = L.lam;
     const bool inz = p.sz.in(k);
-    const long mzk = mzo + (inz ? p.sz.s(k) : 0) * mzs;
-    T za = 0, zb = 0, zK = 1, zah = 0, zbh = 0, zKh = 1;
+    const bool r_k1 = k >= 1, r_kn = k <= nz - 2;
+    T dvx_dx = d4(L.vx_xp, vx0, L.vx_xpp, L.vx_xm, p.odx);
+    T dvy_dy = d4(vy0, L.vy_ym, L.vy_yp, L.vy_ymm, p.ody);
+    T dvz_dz = d4(vz0, vz_zm, L.vz_zp, vz_zmm, p.odz);
+    T dvy_dx = d4(vy0, L.vy_xm, L.vy_xp, L.vy_xmm, p.odx);
+    T dvx_dy = d4(L.vx_yp, vx0, L.vx_ypp, L.vx_ym, p.ody);
+    T dvz_dx = d4(vz0, L.vz_xm, L.vz_xp, L.vz_xmm, p.odx);
+    T dvx_dz = d4(vx_zp, vx0, L.vx_zpp, vx_zm, p.odz);
+    T dvz_dy = d4(L.vz_yp, vz0, L.vz_ypp, L.vz_ym, p.ody);
+    T dvy_dz = d4(vy_zp, vy0, L.vy_zpp, vy_zm, p.odz);
+    const_divide(p.div24, dvx_dx, dvy_dy, dvz_dz);
+    const_divide(p.div24, dvy_dx, dvx_dy, dvz_dx);
+    const_divide(p.div24, dvx_dz, dvz_dy, dvy_dz);
+    if (inx) {
+      const long m = mxo + k * mxs;
+      pml4(r_n && r_k1, dvx_dx, L.px[0], Q->mx[0] + m, xah, xbh, xKh);
+      pml4(r_xy, dvy_dx, L.px[1], Q->mx[1] + m, xa, xb, xK);
+      pml4(r_xz && r_kn, dvz_dx, L.px[2], Q->mx[2] + m, xa, xb, xK);
+    }
+    if (iny) {
+      const long m = myo + k * mys;
+      pml4(r_n && r_k1, dvy_dy, L.py[0], Q->my[0] + m, ya, yb, yK);
+      pml4(r_xy, dvx_dy, L.py[1], Q->my[1] + m, yah, ybh, yKh);
+      pml4(r_yz && r_kn, dvz_dy, L.py[2], Q->my[2] + m, yah, ybh, yKh);
+    }
     if (inz) {
-      za = p.pz.a[k]; zb = p.pz.b[k]; zK = p.pz.K[k];
-      zah = p.pz.ah[k]; zbh = p.pz.bh[k]; zKh = p.pz.Kh[k];
+      const long m = mzo + p.sz.s(k) * mzs;
+      const T zah = Q->pz.ah[k], zbh = Q->pz.bh[k], zKh = Q->pz.Kh[k];
+      pml4(r_n && r_k1, dvz_dz, L.pz[0], Q->mz[0] + m, Q->pz.a[k], Q->pz.b[k], Q->pz.K[k]);
+      pml4(r_xz && r_kn, dvx_dz, L.pz[1], Q->mz[1] + m, zah, zbh, zKh);
+      pml4(r_yz && r_kn, dvy_dz, L.pz[2], Q->mz[2] + m, zah, zbh, zKh);
     }
-    if (r_n && k >= 1) {
-      const T lu = (lam + c23 * mu) - c23 * mu;
-      const T l2u = lu + T(2) * mu;
-      T dvx_dx = d4(vx_xp, vx0, vx_xpp, vx_xm, p.odx);
-      T dvy_dy = d4(vy0, vy_ym, vy_yp, vy_ymm, p.ody);
-      T dvz_dz = d4(vz0, vz_zm, vz_zp, vz_zmm, p.odz);
-      if (inx) dvx_dx = cpml(dvx_dx, p.mx[0] + mxo + k * mxs, xah, xbh, xKh);
-      if (iny) dvy_dy = cpml(dvy_dy, p.my[0] + myo + k * mys, ya, yb, yK);
-      if (inz) dvz_dz = cpml(dvz_dz, p.mz[0] + mzk, za, zb, zK);
-      sxx[0] = oxx + (l2u * dvx_dx + lu * dvy_dy + lu * dvz_dz) * p.dt;
-      syy[0] = oyy + (lu * dvx_dx + l2u * dvy_dy + lu * dvz_dz) * p.dt;
-      szz[0] = ozz + (lu * dvx_dx + lu * dvy_dy + l2u * dvz_dz) * p.dt;
+    const T lu = (lam + c23 * mu) - c23 * mu;
+    const T l2u = lu + T(2) * mu;
+    if (r_n && r_k1) {
+      g.st(L.xx + (l2u * dvx_dx + lu * dvy_dy + lu * dvz_dz) * p.dt, rxx, kk);
+      g.st(L.yy + (lu * dvx_dx + l2u * dvy_dy + lu * dvz_dz) * p.dt, ryy, kk);
+      g.st(L.zz + (lu * dvx_dx + lu * dvy_dy + l2u * dvz_dz) * p.dt, rzz, kk);
     }
-    if (r_xy) {
-      T dvy_dx = d4(vy0, vy_xm, vy_xp, vy_xmm, p.odx);
-      T dvx_dy = d4(vx_yp, vx0, vx_ypp, vx_ym, p.ody);
-      if (inx) dvy_dx = cpml(dvy_dx, p.mx[1] + mxo + k * mxs, xa, xb, xK);
-      if (iny) dvx_dy = cpml(dvx_dy, p.my[1] + myo + k * mys, yah, ybh, yKh);
-      sxy[0] = oxy + mu * (dvx_dy + dvy_dx) * p.dt;
-    }
-    if (r_xz && k <= nz - 2) {
-      T dvz_dx = d4(vz0, vz_xm, vz_xp, vz_xmm, p.odx);
-      T dvx_dz = d4(vx_zp, vx0, vx_zpp, vx_zm, p.odz);
-      if (inx) dvz_dx = cpml(dvz_dx, p.mx[2] + mxo + k * mxs, xa, xb, xK);
-      if (inz) dvx_dz = cpml(dvx_dz, p.mz[1] + mzk, zah, zbh, zKh);
-      sxz[0] = oxz + mu * (dvx_dz + dvz_dx) * p.dt;
-    }
-    if (r_yz && k <= nz - 2) {
-      T dvz_dy = d4(vz_yp, vz0, vz_ypp, vz_ym, p.ody);
-      T dvy_dz = d4(vy_zp, vy0, vy_zpp, vy_zm, p.odz);
-      if (iny) dvz_dy = cpml(dvz_dy, p.my[2] + myo + k * mys, yah, ybh, yKh);
-      if (inz) dvy_dz = cpml(dvy_dz, p.mz[2] + mzk, zah, zbh, zKh);
-      syz[0] = oyz + mu * (dvy_dz + dvz_dy) * p.dt;
-    }
-    vx_zm = vx0, vx0 = vx_zp, vx_zp = vx_zpp;
-    vy_zm = vy0, vy0 = vy_zp, vy_zp = vy_zpp;
-    vz_zmm = vz_zm, vz_zm = vz0, vz0 = vz_zp;
+    if (r_xy) g.st(L.xy + mu * (dvx_dy + dvy_dx) * p.dt, rxy, kk);
+    if (r_xz && r_kn) g.st(L.xz + mu * (dvx_dz + dvz_dx) * p.dt, rxz, kk);
+    if (r_yz && r_kn) g.st(L.yz + mu * (dvy_dz + dvz_dy) * p.dt, ryz, kk);
+    vx_zm = vx0, vx0 = vx_zp, vx_zp = L.vx_zpp;
+    vy_zm = vy0, vy0 = vy_zp, vy_zp = L.vy_zpp;
+    vz_zmm = vz_zm, vz_zm = vz0, vz0 = L.vz_zp;
+  };
+  SPlane4<T> A, B;
+  load(A, c.kb);
+  for (int k = c.kb; k < c.ke; k += 2) {
+    plane(k, A, B);
+    if (k + 1 < c.ke) plane(k + 1, B, A);
   }
 }
 
-// Float: at least 6 waves per SIMD.  The register limit that sets (80 VGPRs,
-// against 82 unbounded, which leaves 5) costs no spill here, and the step ran
-// 1.2% faster at 768^3; the stress kernel spills under the same bound and
-// keeps its 90 registers, and so does the double velocity kernel.
+// Values the velocity kernel reads at plane k.
+template <typename T>
+struct VPlane4 {
+  T xx0, xx_xm, xx_xp, xx_xmm, xy0, xy_ym, xy_yp, xy_ymm, xy_xp, xy_xpp, xy_xm;
+  T xz_zp, xz_xp, xz_xpp, xz_xm, yy0, yy_yp, yy_ypp, yy_ym, yz_zp, yz_ym, yz_yp, yz_ymm;
+  T zz_zpp, cb, vx, vy, vz;
+  T px[3], py[3], pz[3];
+};
+
 template <typename T, int TY4>
-__global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 6 : 1) void k_velocity3d4(Step3D<T> p) {
-  const Col4 c = col4<TY4>(p.nx, p.ny, p.nz, p.kchunk);
+__global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_velocity3d4(Step3D<T> p) {
+  const Tile3 c = tile3<TY4, kFlat4<T>>(p);
   if (!c.ok) return;
   const int i = c.i, j = c.j, nx = p.nx, ny = p.ny, nz = p.nz;
-  const long ld = p.ld, ps = p.ps;
+  const Chunk4<T> g(p, c);
+  const auto rvx = g.rsrc(p.vx, p.base), rvy = g.rsrc(p.vy, p.base), rvz = g.rsrc(p.vz, p.base);
+  const auto rcb = g.rsrc(p.cbuoy, p.base);  // DELTAT_over_rho
+  const auto rxx = g.rsrc(p.sxx, p.base), ryy = g.rsrc(p.syy, p.base);
+  const auto rzz = g.rsrc(p.szz, p.base), rxy = g.rsrc(p.sxy, p.base);
+  const auto rxz = g.rsrc(p.sxz, p.base), ryz = g.rsrc(p.syz, p.base);
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
   const long mxo = p.sx.at(i, j, ny), mxs = (long)p.sx.w * ny;
   const long myo = i + p.mld * p.sy.s(j), mys = p.mld * p.sy.w;
@@ -197,72 +274,97 @@ __global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 6 : 1) void k_velocity3d4
     ya = p.py.a[j]; yb = p.py.b[j]; yK = p.py.K[j];
     yah = p.py.ah[j]; ybh = p.py.bh[j]; yKh = p.py.Kh[j];
   }
-  const long q0 = i + j * ld + c.kb * ps;
-  T sxz_zmm = p.sxz[q0 - 2 * ps], sxz_zm = p.sxz[q0 - ps], sxz0 = p.sxz[q0];
-  T syz_zmm = p.syz[q0 - 2 * ps], syz_zm = p.syz[q0 - ps], syz0 = p.syz[q0];
-  T szz_zm = p.szz[q0 - ps], szz0 = p.szz[q0], szz_zp = p.szz[q0 + ps];
-  for (int k = c.kb; k < c.ke; ++k) {
-    const long q = i + j * ld + k * ps;
-    const T *__restrict__ sxx = p.sxx + q;
-    const T *__restrict__ syy = p.syy + q;
-    const T *__restrict__ szz = p.szz + q;
-    const T *__restrict__ sxy = p.sxy + q;
-    const T *__restrict__ sxz = p.sxz + q;
-    const T *__restrict__ syz = p.syz + q;
-    T *__restrict__ vx = p.vx + q;
-    T *__restrict__ vy = p.vy + q;
-    T *__restrict__ vz = p.vz + q;
-    const T sxx0 = sxx[0], sxx_xm = sxx[-1], sxx_xp = sxx[1], sxx_xmm = sxx[-2];
-    const T sxy0 = sxy[0], sxy_ym = sxy[-ld], sxy_yp = sxy[ld], sxy_ymm = sxy[-2 * ld];
-    const T sxy_xp = sxy[1], sxy_xpp = sxy[2], sxy_xm = sxy[-1];
-    const T sxz_zp = sxz[ps];
-    const T sxz_xp = sxz[1], sxz_xpp = sxz[2], sxz_xm = sxz[-1];
-    const T syy0 = syy[0], syy_yp = syy[ld], syy_ypp = syy[2 * ld], syy_ym = syy[-ld];
-    const T syz_zp = syz[ps];
-    const T syz_ym = syz[-ld], syz_yp = syz[ld], syz_ymm = syz[-2 * ld];
-    const T szz_zpp = szz[2 * ps];
-    const T cb = p.cbuoy[q];  // DELTAT_over_rho
-    T vxn = vx[0], vyn = vy[0], vzn = vz[0];
+  auto load = [&](VPlane4<T> &L, int k) {
+    const auto Q = kernarg<Step3D<T>>();
+    const int kk = k - c.kb + 2;
+    L.zz_zpp = g.ld(rzz, 0, 0, 2, kk);
+    L.xz_zp = g.ld(rxz, 0, 0, 1, kk), L.yz_zp = g.ld(ryz, 0, 0, 1, kk);
+    L.xx0 = g.ld(rxx, 0, 0, 0, kk), L.xx_xm = g.ld(rxx, -1, 0, 0, kk);
+    L.xx_xp = g.ld(rxx, 1, 0, 0, kk), L.xx_xmm = g.ld(rxx, -2, 0, 0, kk);
+    L.xy0 = g.ld(rxy, 0, 0, 0, kk), L.xy_ym = g.ld(rxy, 0, -1, 0, kk);
+    L.xy_yp = g.ld(rxy, 0, 1, 0, kk), L.xy_ymm = g.ld(rxy, 0, -2, 0, kk);
+    L.xy_xp = g.ld(rxy, 1, 0, 0, kk), L.xy_xpp = g.ld(rxy, 2, 0, 0, kk);
+    L.xy_xm = g.ld(rxy, -1, 0, 0, kk);
+    L.xz_xp = g.ld(rxz, 1, 0, 0, kk), L.xz_xpp = g.ld(rxz, 2, 0, 0, kk);
+    L.xz_xm = g.ld(rxz, -1, 0, 0, kk);
+    L.yy0 = g.ld(ryy, 0, 0, 0, kk), L.yy_yp = g.ld(ryy, 0, 1, 0, kk);
+    L.yy_ypp = g.ld(ryy, 0, 2, 0, kk), L.yy_ym = g.ld(ryy, 0, -1, 0, kk);
+    L.yz_ym = g.ld(ryz, 0, -1, 0, kk), L.yz_yp = g.ld(ryz, 0, 1, 0, kk);
+    L.yz_ymm = g.ld(ryz, 0, -2, 0, kk);
+    L.cb = g.ld(rcb, 0, 0, 0, kk);
+    L.vx = g.ld(rvx, 0, 0, 0, kk), L.vy = g.ld(rvy, 0, 0, 0, kk), L.vz = g.ld(rvz, 0, 0, 0, kk);
+    if (inx) {
+      const long m = mxo + k * mxs;
+      L.px[0] = Q->mx[3][m], L.px[1] = Q->mx[4][m], L.px[2] = Q->mx[5][m];
+    }
+    if (iny) {
+      const long m = myo + k * mys;
+      L.py[0] = Q->my[3][m], L.py[1] = Q->my[4][m], L.py[2] = Q->my[5][m];
+    }
+    if (p.sz.in(k)) {
+      const long m = mzo + p.sz.s(k) * mzs;
+      L.pz[0] = Q->mz[3][m], L.pz[1] = Q->mz[4][m], L.pz[2] = Q->mz[5][m];
+    }
+  };
+  constexpr int k0 = 2;  // buffer plane of kb
+  T sxz_zmm = g.ld(rxz, 0, 0, -2, k0), sxz_zm = g.ld(rxz, 0, 0, -1, k0);
+  T sxz0 = g.ld(rxz, 0, 0, 0, k0);
+  T syz_zmm = g.ld(ryz, 0, 0, -2, k0), syz_zm = g.ld(ryz, 0, 0, -1, k0);
+  T syz0 = g.ld(ryz, 0, 0, 0, k0);
+  T szz_zm = g.ld(rzz, 0, 0, -1, k0), szz0 = g.ld(rzz, 0, 0, 0, k0);
+  T szz_zp = g.ld(rzz, 0, 0, 1, k0);
+  // one plane: L holds its values, N receives the next one's.  The caller
+  // alternates two sets, so no copy waits for the loads in flight, and they are
+  // issued before this plane's stores, so waiting for them does not wait for
+  // those.
+  auto plane = [&](int k, const VPlane4<T> &L, VPlane4<T> &N) {
+    const auto Q = kernarg<Step3D<T>>();
+    const int kk = k - c.kb + 2;
+    load(N, min(k + 1, c.ke - 1));
+    const T cb = L.cb;
+    T vxn = L.vx, vyn = L.vy, vzn = L.vz;
     const bool inz = p.sz.in(k);
-    const long mzk = mzo + (inz ? p.sz.s(k) : 0) * mzs;
-    T za = 0, zb = 0, zK = 1, zah = 0, zbh = 0, zKh = 1;
+    const bool r_k1 = k >= 1, r_kn = k <= nz - 2;
+    T dsxx_dx = d4(L.xx0, L.xx_xm, L.xx_xp, L.xx_xmm, p.odx);
+    T dsxy_dy = d4(L.xy0, L.xy_ym, L.xy_yp, L.xy_ymm, p.ody);
+    T dsxz_dz = d4(sxz0, sxz_zm, L.xz_zp, sxz_zmm, p.odz);
+    T dsxy_dx = d4(L.xy_xp, L.xy0, L.xy_xpp, L.xy_xm, p.odx);
+    T dsyy_dy = d4(L.yy_yp, L.yy0, L.yy_ypp, L.yy_ym, p.ody);
+    T dsyz_dz = d4(syz0, syz_zm, L.yz_zp, syz_zmm, p.odz);
+    T dsxz_dx = d4(L.xz_xp, sxz0, L.xz_xpp, L.xz_xm, p.odx);
+    T dsyz_dy = d4(syz0, L.yz_ym, L.yz_yp, L.yz_ymm, p.ody);
+    T dszz_dz = d4(szz_zp, szz0, L.zz_zpp, szz_zm, p.odz);
+    const_divide(p.div24, dsxx_dx, dsxy_dy, dsxz_dz);
+    const_divide(p.div24, dsxy_dx, dsyy_dy, dsyz_dz);
+    const_divide(p.div24, dsxz_dx, dsyz_dy, dszz_dz);
+    if (inx) {
+      const long m = mxo + k * mxs;
+      pml4(r_vx && r_k1, dsxx_dx, L.px[0], Q->mx[3] + m, xa, xb, xK);
+      pml4(r_vy && r_k1, dsxy_dx, L.px[1], Q->mx[4] + m, xah, xbh, xKh);
+      pml4(r_vz && r_kn, dsxz_dx, L.px[2], Q->mx[5] + m, xah, xbh, xKh);
+    }
+    if (iny) {
+      const long m = myo + k * mys;
+      pml4(r_vx && r_k1, dsxy_dy, L.py[0], Q->my[3] + m, ya, yb, yK);
+      pml4(r_vy && r_k1, dsyy_dy, L.py[1], Q->my[4] + m, yah, ybh, yKh);
+      pml4(r_vz && r_kn, dsyz_dy, L.py[2], Q->my[5] + m, ya, yb, yK);
+    }
     if (inz) {
-      za = p.pz.a[k]; zb = p.pz.b[k]; zK = p.pz.K[k];
-      zah = p.pz.ah[k]; zbh = p.pz.bh[k]; zKh = p.pz.Kh[k];
+      const long m = mzo + p.sz.s(k) * mzs;
+      const T za = Q->pz.a[k], zb = Q->pz.b[k], zK = Q->pz.K[k];
+      pml4(r_vx && r_k1, dsxz_dz, L.pz[0], Q->mz[3] + m, za, zb, zK);
+      pml4(r_vy && r_k1, dsyz_dz, L.pz[1], Q->mz[4] + m, za, zb, zK);
+      pml4(r_vz && r_kn, dszz_dz, L.pz[2], Q->mz[5] + m, Q->pz.ah[k], Q->pz.bh[k], Q->pz.Kh[k]);
     }
-    if (r_vx && k >= 1) {
-      T dsxx_dx = d4(sxx0, sxx_xm, sxx_xp, sxx_xmm, p.odx);
-      T dsxy_dy = d4(sxy0, sxy_ym, sxy_yp, sxy_ymm, p.ody);
-      T dsxz_dz = d4(sxz0, sxz_zm, sxz_zp, sxz_zmm, p.odz);
-      if (inx) dsxx_dx = cpml(dsxx_dx, p.mx[3] + mxo + k * mxs, xa, xb, xK);
-      if (iny) dsxy_dy = cpml(dsxy_dy, p.my[3] + myo + k * mys, ya, yb, yK);
-      if (inz) dsxz_dz = cpml(dsxz_dz, p.mz[3] + mzk, za, zb, zK);
-      vxn = cb * (dsxx_dx + dsxy_dy + dsxz_dz) + vxn;
-    }
-    if (r_vy && k >= 1) {
-      T dsxy_dx = d4(sxy_xp, sxy0, sxy_xpp, sxy_xm, p.odx);
-      T dsyy_dy = d4(syy_yp, syy0, syy_ypp, syy_ym, p.ody);
-      T dsyz_dz = d4(syz0, syz_zm, syz_zp, syz_zmm, p.odz);
-      if (inx) dsxy_dx = cpml(dsxy_dx, p.mx[4] + mxo + k * mxs, xah, xbh, xKh);
-      if (iny) dsyy_dy = cpml(dsyy_dy, p.my[4] + myo + k * mys, yah, ybh, yKh);
-      if (inz) dsyz_dz = cpml(dsyz_dz, p.mz[4] + mzk, za, zb, zK);
-      vyn = cb * (dsxy_dx + dsyy_dy + dsyz_dz) + vyn;
-    }
-    if (r_vz && k <= nz - 2) {
-      T dsxz_dx = d4(sxz_xp, sxz0, sxz_xpp, sxz_xm, p.odx);
-      T dsyz_dy = d4(syz0, syz_ym, syz_yp, syz_ymm, p.ody);
-      T dszz_dz = d4(szz_zp, szz0, szz_zpp, szz_zm, p.odz);
-      if (inx) dsxz_dx = cpml(dsxz_dx, p.mx[5] + mxo + k * mxs, xah, xbh, xKh);
-      if (iny) dsyz_dy = cpml(dsyz_dy, p.my[5] + myo + k * mys, ya, yb, yK);
-      if (inz) dszz_dz = cpml(dszz_dz, p.mz[5] + mzk, zah, zbh, zKh);
-      vzn = cb * (dsxz_dx + dsyz_dy + dszz_dz) + vzn;
-    }
+    if (r_vx && r_k1) vxn = cb * (dsxx_dx + dsxy_dy + dsxz_dz) + vxn;
+    if (r_vy && r_k1) vyn = cb * (dsxy_dx + dsyy_dy + dsyz_dz) + vyn;
+    if (r_vz && r_kn) vzn = cb * (dsxz_dx + dsyz_dy + dszz_dz) + vzn;
     // point force on the cut plane (3D-visco:1350-1352)
     if (src_col && k == p.ksrc) {
-      const int it = *p.step;
-      const T rs = p.rho[q];
-      vxn = vxn + p.fx[it - 1] * p.dt / rs;
-      vyn = vyn + p.fy[it - 1] * p.dt / rs;
+      const int it = *Q->step;
+      const T rs = Q->rho[i + (long)j * p.ld + (long)k * p.ps];
+      vxn = vxn + Q->fx[it - 1] * p.dt / rs;
+      vyn = vyn + Q->fy[it - 1] * p.dt / rs;
     }
     // rigid faces: planes 1 and N of every axis (3D-visco:1355-1398)
     if (edge_xy || k == 0 || k == nz - 1) {
@@ -270,42 +372,51 @@ __global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 6 : 1) void k_velocity3d4
       vyn = T(0);
       vzn = T(0);
     }
-    vx[0] = vxn;
-    vy[0] = vyn;
-    vz[0] = vzn;
-    sxz_zmm = sxz_zm, sxz_zm = sxz0, sxz0 = sxz_zp;
-    syz_zmm = syz_zm, syz_zm = syz0, syz0 = syz_zp;
-    szz_zm = szz0, szz0 = szz_zp, szz_zp = szz_zpp;
+    g.st(vxn, rvx, kk);
+    g.st(vyn, rvy, kk);
+    g.st(vzn, rvz, kk);
+    sxz_zmm = sxz_zm, sxz_zm = sxz0, sxz0 = L.xz_zp;
+    syz_zmm = syz_zm, syz_zm = syz0, syz0 = L.yz_zp;
+    szz_zm = szz0, szz0 = szz_zp, szz_zp = L.zz_zpp;
+  };
+  VPlane4<T> A, B;
+  load(A, c.kb);
+  for (int k = c.kb; k < c.ke; k += 2) {
+    plane(k, A, B);
+    if (k + 1 < c.ke) plane(k + 1, B, A);
   }
 }
 
 template <typename T>
 unsigned ntiles4(const Step3D<T> &p, int ty) {
-  return (unsigned)((p.nx + BX - 1) / BX) * ((p.ny + ty - 1) / ty) *
+  return (unsigned)plane_tiles3<kFlat4<T>>(p.nx, p.ny, ty) *
          ((p.nz + p.kchunk - 1) / p.kchunk);
 }
 
 }  // namespace
 
-// p.tile_y selects the rows per block (4, 8 or 16)
+// p.tile_y selects the rows per block (4, 8 or 16; double: at most 8, whose two
+// planes of values fit in registers)
 template <typename T>
 hipError_t launch_stress3d4(const Step3D<T> &p, hipStream_t s) {
-  if (p.tile_y == 16)
-    hipLaunchKernelGGL((k_stress3d4<T, 16>), dim3(ntiles4(p, 16)), dim3(BX, 16), 0, s, p);
-  else if (p.tile_y == 8)
-    hipLaunchKernelGGL((k_stress3d4<T, 8>), dim3(ntiles4(p, 8)), dim3(BX, 8), 0, s, p);
-  else
+  if (p.tile_y >= 8) {
+    if (p.tile_y == 16 && sizeof(T) == 4)
+      hipLaunchKernelGGL((k_stress3d4<T, 16>), dim3(ntiles4(p, 16)), dim3(BX, 16), 0, s, p);
+    else
+      hipLaunchKernelGGL((k_stress3d4<T, 8>), dim3(ntiles4(p, 8)), dim3(BX, 8), 0, s, p);
+  } else
     hipLaunchKernelGGL((k_stress3d4<T, 4>), dim3(ntiles4(p, 4)), dim3(BX, 4), 0, s, p);
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_velocity3d4(const Step3D<T> &p, hipStream_t s) {
-  if (p.tile_y == 16)
-    hipLaunchKernelGGL((k_velocity3d4<T, 16>), dim3(ntiles4(p, 16)), dim3(BX, 16), 0, s, p);
-  else if (p.tile_y == 8)
-    hipLaunchKernelGGL((k_velocity3d4<T, 8>), dim3(ntiles4(p, 8)), dim3(BX, 8), 0, s, p);
-  else
+  if (p.tile_y >= 8) {
+    if (p.tile_y == 16 && sizeof(T) == 4)
+      hipLaunchKernelGGL((k_velocity3d4<T, 16>), dim3(ntiles4(p, 16)), dim3(BX, 16), 0, s, p);
+    else
+      hipLaunchKernelGGL((k_velocity3d4<T, 8>), dim3(ntiles4(p, 8)), dim3(BX, 8), 0, s, p);
+  } else
     hipLaunchKernelGGL((k_velocity3d4<T, 4>), dim3(ntiles4(p, 4)), dim3(BX, 4), 0, s, p);
   return hipGetLastError();
 }

@@ -179,7 +179,7 @@ struct cpml_solver {
   int graph_steps = 16;
   hipGraphExec_t gexec[2] = {nullptr, nullptr};  // per starting state buffer
   bool graph_dirty = true;
-  int kchunk = 8;
+  int kchunk = 0;  // planes per block of the 3D kernels (0: kchunk_of)
   int tile_y = 4;
   bool ktiming = false;
   std::vector<hipEvent_t> evpool;
@@ -232,6 +232,26 @@ bool chunk_fits(const cpml_solver *h, int kchunk) {
     if (e_ != hipSuccess)                                                                \
       return fail((h), CPML_ERR_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
+
+// Planes per block of the 3D two-phase and fused kernels.  Each block reads its
+// halo planes again, so deep chunks read less, but the machine wants about four
+// blocks per CU: 8 planes (order 4, whose halo is deeper, 32 where that leaves
+// four rounds of blocks: 210 x 800 x 220 float 1442 and 1382 us per step, 256^3
+// 583 with 8 and 605 with 16), halved for small grids (96 x 80 x 72 float 45 us
+// with 8 planes, 41 with 2; the fused kernel, which recomputes its halo
+// planes, keeps 8), and less where a chunk's buffer would pass 4 GiB.
+int kchunk_of(const cpml_solver *h) {
+  if (h->kchunk > 0) return h->kchunk;
+  const long tiles = (long)((h->nx + 63) / 64) * ((h->ny + h->tile_y - 1) / h->tile_y);
+  auto blocks = [&](int k) { return tiles * ((h->nz + k - 1) / k); };
+  int k = 8;
+  if (!h->fused) {
+    if (h->order == 4 && blocks(32) >= 4096) k = 32;
+    while (k > 2 && blocks(k) < 1024) k /= 2;
+  }
+  while (k > 1 && !chunk_fits(h, k)) --k;
+  return k;
+}
 
 int dev_alloc(cpml_solver *h, void **p, size_t bytes) {
   if (bytes == 0) bytes = 256;
@@ -517,6 +537,7 @@ cpml::Step3D<T> step3d(cpml_solver *h) {
   p.R = h->R;
   // 3D:134-137 ONE_OVER_DELTA = 1/DELTA, applied by multiplication (3D:841)
   p.odx = T(1) / T(h->dx);
+  p.div24 = cpml::const_div(T(24));
   p.ody = T(1) / T(h->dy);
   p.odz = T(1) / T(h->dz);
   p.dt = T(h->dt);
@@ -526,7 +547,7 @@ cpml::Step3D<T> step3d(cpml_solver *h) {
   p.fx = static_cast<const T *>(h->fx);
   p.fy = static_cast<const T *>(h->fy);
   p.step = h->step;
-  p.kchunk = h->kchunk;
+  p.kchunk = kchunk_of(h);
   p.tile_y = h->tile_y;
   p.streaming = h->bytes > cpml::kStreamingBytes;
   return p;
@@ -1253,8 +1274,6 @@ int cpml_gpu_init(cpml_solver **hp, int ndim, int order, int prec, int NX, int N
   h->base = h->xpad + h->R * h->ld + (ndim == 3 ? h->R * h->ps : 0);
   h->total = h->ps * (ndim == 3 ? NZ + 2 * h->R : 1);
   h->mld = round_up(NX, align);
-  // default chunk depth, reduced where a chunk's buffer would pass 4 GiB
-  while (h->kchunk > 1 && !chunk_fits(h, h->kchunk)) --h->kchunk;
   if (!chunk_fits(h, 1)) {
     delete h;
     return fail(nullptr, CPML_ERR_OOM, "3D grid planes too large for 32-bit buffer offsets");

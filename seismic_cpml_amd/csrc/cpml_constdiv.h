@@ -97,6 +97,25 @@ __device__ __forceinline__ void const_divide(T &a, const ConstDiv<T> &A, T &b,
     a = qa, b = qb, c = qc, d = qd;
   }
 }
+// The same of up to three numbers and one divisor.
+template <typename T>
+__device__ __forceinline__ void const_divide(const ConstDiv<T> &D, T &a, T &b, T &c) {
+  const T m = fmax(fmax(fabs(a), fabs(b)), fabs(c));
+  const uint32_t k = min(min(magnitude_key(a), magnitude_key(b)), magnitude_key(c));
+  const T qa = D.quot(a), qb = D.quot(b), qc = D.quot(c);
+  if (__builtin_expect(m >= D.hi || k < D.lo, 0)) {
+    a = a / D.d;
+    b = b / D.d;
+    c = c / D.d;
+  } else {
+    a = qa, b = qb, c = qc;
+  }
+}
+template <typename T>
+__device__ __forceinline__ void const_divide(const ConstDiv<T> &D, T &a, T &b) {
+  T c = b;
+  const_divide(D, a, c, b);
+}
 #endif
 
 }  // namespace cpml

@@ -17,6 +17,56 @@ __device__ __forceinline__ int zchunk_of(int band_pos, int ntz) {
   return band_pos / m + 8 * (band_pos % m);
 }
 
+// Tile of the two-phase 3D kernels: 64 columns by TY rows (one wavefront per
+// row) marching the z planes [kb, ke).
+struct Tile3 {
+  int i, j, kb, ke;
+  bool ok;
+};
+
+// FLAT numbers the columns through the TY-row groups of a plane, one group after
+// the other, and cuts them into wavefronts of 64, so that only a plane's last
+// tile has idle lanes; otherwise each group of rows is cut by itself, so that
+// every wavefront but a row's last stores whole cache lines.  Double, order 4,
+// 210 columns: FLAT 2746 us per step, by rows 3020; elsewhere the whole lines
+// count for more (float, order 4: 1505 and 1382; double, order 2, 101 columns:
+// 3068 and 2827).
+template <bool FLAT>
+inline __host__ __device__ int plane_tiles3(int nx, int ny, int ty) {
+  const int groups = (ny + ty - 1) / ty;
+  return FLAT ? (int)(((long)nx * groups + BX - 1) / BX) : (nx + BX - 1) / BX * groups;
+}
+// Workgroups are dispatched round-robin over the 8 XCDs; each XCD gets one
+// contiguous band of tiles (x fastest, then y, then z chunk) so the tiles that
+// read each other's halo rows share its L2; the z chunks are interleaved over
+// the bands (zchunk_of).
+template <int TY, bool FLAT, typename P>
+__device__ __forceinline__ Tile3 tile3(const P &p) {
+  const int nxy = plane_tiles3<FLAT>(p.nx, p.ny, TY);
+  const int ntz = (p.nz + p.kchunk - 1) / p.kchunk;
+  const int nt = nxy * ntz;
+  const int h = blockIdx.x;
+  const int xcd = h & 7, loc = h >> 3;
+  const int q = nt >> 3, r = nt & 7;
+  const int t = xcd * q + min(xcd, r) + loc, txy = t % nxy;
+  Tile3 o;
+  int group;
+  if (FLAT) {
+    const int col = txy * BX + threadIdx.x;
+    group = col / p.nx;
+    o.i = col - group * p.nx;
+  } else {
+    const int ntx = (p.nx + BX - 1) / BX;
+    group = txy / ntx;
+    o.i = (txy - group * ntx) * BX + threadIdx.x;
+  }
+  o.j = group * TY + threadIdx.y;
+  o.kb = zchunk_of(t / nxy, ntz) * p.kchunk;
+  o.ke = min(o.kb + p.kchunk, p.nz);
+  o.ok = o.i < p.nx && o.j < p.ny;
+  return o;
+}
+
 // d / K.  The reference profiles use K_MAX_PML = 1 (2D2:215), so K is 1 at
 // every point and x / 1 == x exactly in IEEE arithmetic: the correctly
 // rounded division (a dozen instructions) is only executed where K != 1.

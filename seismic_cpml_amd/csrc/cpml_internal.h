@@ -128,6 +128,7 @@ struct Step3D {
   int R;          // halo rows / planes on each side
   long mld, mps;  // memory strides: x-slab (w, w*ny), y-slab (mld, mld*wy), z (mld, mld*ny)
   T odx, ody, odz;
+  ConstDiv<T> div24;  // order 4: division by 24
   T dt;
   int isrc, jsrc, ksrc;
   const T *fx, *fy;

@@ -73,37 +73,11 @@ __global__ __launch_bounds__(BX *TY) void k_velocity2d(Step2D<T> p) {
 // registers.  Field offsets are unsigned 32-bit byte offsets into a buffer
 // rebased at the tile's first halo plane (the host keeps a chunk's planes plus
 // 8 halo and pipeline planes below 4 GiB: chunk_fits() in cpml_api.hip),
-// added to uniform base pointers, and the loads of plane k+1 are issued
-// before the arithmetic and stores of plane k (register double buffering).
-
-struct Tile3 {
-  int i, j, kb, ke;
-  bool ok;
-};
-
-// Workgroups are dispatched round-robin over the 8 XCDs; give each XCD one
-// contiguous band of tiles (x fastest, then y, then z chunk) so the tiles that
-// read each other's halo rows run on the same XCD and share its L2; the z
-// chunks are interleaved over the bands (zchunk_of).
-template <int TY3>
-__device__ __forceinline__ Tile3 tile3(int nx, int ny, int nz, int kchunk) {
-  const int ntx = (nx + BX - 1) / BX, nty = (ny + TY3 - 1) / TY3;
-  const int ntz = (nz + kchunk - 1) / kchunk;
-  const int nt = ntx * nty * ntz;
-  const int h = blockIdx.x;
-  const int xcd = h & 7, loc = h >> 3;
-  const int q = nt >> 3, r = nt & 7;
-  const int t = xcd * q + min(xcd, r) + loc;
-  const int tx = t % ntx, rest = t / ntx;
-  const int ty = rest % nty, tz = zchunk_of(rest / nty, ntz);
-  Tile3 o;
-  o.i = tx * BX + threadIdx.x;
-  o.j = ty * TY3 + threadIdx.y;
-  o.kb = tz * kchunk;
-  o.ke = min(o.kb + kchunk, nz);
-  o.ok = o.i < nx && o.j < ny;
-  return o;
-}
+// added to uniform base pointers, and the loads of plane k+1, memory
+// variables included, are issued before the arithmetic and stores of plane k
+// into the other of two register sets.  Bound by HBM latency and rate: with one
+// set copied at each plane's end the copies waited for those loads and stores
+// (200^3 float 317 us per step, now 273; 96 x 80 x 72 66, now 45).
 
 // Geometry of the rebased chunk buffers of one tile.
 template <typename T>
@@ -138,17 +112,27 @@ struct Chunk3 {
 #define CPML_ST(x, r) \
   BufOp<T>::template stp<NT ? kNonTemporal : 0>(x, r, g.v0 + (unsigned)sizeof(T), g.so(kk, 0, 0))
 
+// C-PML correction of a derivative with the memory variable m read a plane
+// ahead: psi <- b*psi + a*d ; d <- d/K + psi.
+template <typename T>
+__device__ __forceinline__ T pml3(T d, T m, T *psi, T a, T b, T K) {
+  m = b * m + a * d;
+  *psi = m;
+  return over_k(d, K) + m;
+}
+
 // Values the stress kernel reads at one plane.
 template <typename T>
 struct SPlane {
   T vx_p, vy_p, vz_k;                              // vx, vy at k+1; vz at k
   T vx_xp, vx_yp, vy_ym, vy_xm, vz_xm, vz_yp;      // x/y neighbours at k
   T cl, cm, sxx, syy, szz, sxy, sxz, syz;
+  T px[3], py[3], pz[3];  // memory variables, where the point lies in the axis' slab
 };
 
 template <typename T, int TY3, bool NT>
 __global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p) {
-  const Tile3 t = tile3<TY3>(p.nx, p.ny, p.nz, p.kchunk);
+  const Tile3 t = tile3<TY3, false>(p);
   if (!t.ok) return;
   const int i = t.i, j = t.j;
   const int nx = p.nx, ny = p.ny, nz = p.nz;
@@ -166,7 +150,9 @@ __global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p) {
   const bool r_xy = i >= 1 && j <= ny - 2;
   const bool r_xz = i >= 1;
   const bool r_yz = j <= ny - 2;
-  auto load = [&](SPlane<T> &L, int kk) {
+  auto load = [&](SPlane<T> &L, int k) {
+    const auto Q = kernarg<Step3D<T>>();
+    const int kk = k - t.kb + 1;
     L.vx_p = CPML_LD(rvx, 0, 0, 1);
     L.vy_p = CPML_LD(rvy, 0, 0, 1);
     L.vz_k = CPML_LD(rvz, 0, 0, 0);
@@ -184,6 +170,18 @@ __global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p) {
     L.sxy = CPML_LDN(rxy);
     L.sxz = CPML_LDN(rxz);
     L.syz = CPML_LDN(ryz);
+    if (inx) {
+      const unsigned m = mxo + k * mxs;
+      L.px[0] = Q->mx[0][m], L.px[1] = Q->mx[1][m], L.px[2] = Q->mx[2][m];
+    }
+    if (iny) {
+      const unsigned m = myo + k * mys;
+      L.py[0] = Q->my[0][m], L.py[1] = Q->my[1][m], L.py[2] = Q->my[2][m];
+    }
+    if (p.sz.in(k)) {
+      const unsigned m = mzo + (unsigned)p.sz.s(k) * mzs;
+      L.pz[0] = Q->mz[0][m], L.pz[1] = Q->mz[1][m], L.pz[2] = Q->mz[2][m];
+    }
   };
   // x / y profile values of this column (loop invariant; only read in the
   // absorbing slabs)
@@ -197,15 +195,17 @@ __global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p) {
     ya = p.py.a[j]; yb = p.py.b[j]; yK = p.py.K[j];
     yah = p.py.ah[j]; ybh = p.py.bh[j]; yKh = p.py.Kh[j];
   }
-  int kk = 1;  // buffer plane of k = kb
+  constexpr int kk = 1;  // buffer plane of kb
   T vz_m = CPML_LD(rvz, 0, 0, -1);
   T vx_k = CPML_LD(rvx, 0, 0, 0), vy_k = CPML_LD(rvy, 0, 0, 0);
-  SPlane<T> L;
-  load(L, kk);
-  for (int k = t.kb; k < t.ke; ++k, ++kk) {
+  // one plane: L holds its values, N receives the next one's.  The caller
+  // alternates two sets, so no copy waits for the loads in flight, and they are
+  // issued before this plane's stores, so waiting for them does not wait for
+  // those.
+  auto plane = [&](int k, const SPlane<T> &L, SPlane<T> &N) {
     const auto Q = kernarg<Step3D<T>>();
-    SPlane<T> N = L;
-    if (k + 1 < t.ke) load(N, kk + 1);
+    const int kk = k - t.kb + 1;  // buffer plane of k
+    load(N, min(k + 1, t.ke - 1));
     const bool inz = p.sz.in(k);
     const unsigned mzk = mzo + (unsigned)p.sz.s(k) * mzs;
     const T cl = L.cl, cm = L.cm;
@@ -214,9 +214,9 @@ __global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p) {
       T dvx_dx = (L.vx_xp - vx_k) * p.odx;
       T dvy_dy = (vy_k - L.vy_ym) * p.ody;
       T dvz_dz = (L.vz_k - vz_m) * p.odz;
-      if (inx) dvx_dx = cpml(dvx_dx, Q->mx[0] + mxo + k * mxs, xah, xbh, xKh);
-      if (iny) dvy_dy = cpml(dvy_dy, Q->my[0] + myo + k * mys, ya, yb, yK);
-      if (inz) dvz_dz = cpml(dvz_dz, Q->mz[0] + mzk, Q->pz.a[k], Q->pz.b[k], Q->pz.K[k]);
+      if (inx) dvx_dx = pml3(dvx_dx, L.px[0], Q->mx[0] + mxo + k * mxs, xah, xbh, xKh);
+      if (iny) dvy_dy = pml3(dvy_dy, L.py[0], Q->my[0] + myo + k * mys, ya, yb, yK);
+      if (inz) dvz_dz = pml3(dvz_dz, L.pz[0], Q->mz[0] + mzk, Q->pz.a[k], Q->pz.b[k], Q->pz.K[k]);
       const T lp2m = cl + T(2) * cm;
       CPML_ST(lp2m * dvx_dx + cl * (dvy_dy + dvz_dz) + L.sxx, rxx);
       CPML_ST(cl * (dvx_dx + dvz_dz) + lp2m * dvy_dy + L.syy, ryy);
@@ -226,30 +226,35 @@ __global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p) {
     if (r_xy) {
       T dvy_dx = (vy_k - L.vy_xm) * p.odx;
       T dvx_dy = (L.vx_yp - vx_k) * p.ody;
-      if (inx) dvy_dx = cpml(dvy_dx, Q->mx[1] + mxo + k * mxs, xa, xb, xK);
-      if (iny) dvx_dy = cpml(dvx_dy, Q->my[1] + myo + k * mys, yah, ybh, yKh);
+      if (inx) dvy_dx = pml3(dvy_dx, L.px[1], Q->mx[1] + mxo + k * mxs, xa, xb, xK);
+      if (iny) dvx_dy = pml3(dvx_dy, L.py[1], Q->my[1] + myo + k * mys, yah, ybh, yKh);
       CPML_ST(cm * (dvy_dx + dvx_dy) + L.sxy, rxy);
     }
     // sigma_xz: 3D:908-925 (global k <= NZ-1)
     if (r_xz && k <= nz - 2) {
       T dvz_dx = (L.vz_k - L.vz_xm) * p.odx;
       T dvx_dz = (L.vx_p - vx_k) * p.odz;
-      if (inx) dvz_dx = cpml(dvz_dx, Q->mx[2] + mxo + k * mxs, xa, xb, xK);
-      if (inz) dvx_dz = cpml(dvx_dz, Q->mz[1] + mzk, Q->pz.ah[k], Q->pz.bh[k], Q->pz.Kh[k]);
+      if (inx) dvz_dx = pml3(dvz_dx, L.px[2], Q->mx[2] + mxo + k * mxs, xa, xb, xK);
+      if (inz) dvx_dz = pml3(dvx_dz, L.pz[1], Q->mz[1] + mzk, Q->pz.ah[k], Q->pz.bh[k], Q->pz.Kh[k]);
       CPML_ST(cm * (dvz_dx + dvx_dz) + L.sxz, rxz);
     }
     // sigma_yz: 3D:927-943
     if (r_yz && k <= nz - 2) {
       T dvz_dy = (L.vz_yp - L.vz_k) * p.ody;
       T dvy_dz = (L.vy_p - vy_k) * p.odz;
-      if (iny) dvz_dy = cpml(dvz_dy, Q->my[2] + myo + k * mys, yah, ybh, yKh);
-      if (inz) dvy_dz = cpml(dvy_dz, Q->mz[2] + mzk, Q->pz.ah[k], Q->pz.bh[k], Q->pz.Kh[k]);
+      if (iny) dvz_dy = pml3(dvz_dy, L.py[2], Q->my[2] + myo + k * mys, yah, ybh, yKh);
+      if (inz) dvy_dz = pml3(dvy_dz, L.pz[2], Q->mz[2] + mzk, Q->pz.ah[k], Q->pz.bh[k], Q->pz.Kh[k]);
       CPML_ST(cm * (dvz_dy + dvy_dz) + L.syz, ryz);
     }
     vz_m = L.vz_k;
     vx_k = L.vx_p;
     vy_k = L.vy_p;
-    L = N;
+  };
+  SPlane<T> A, B;
+  load(A, t.kb);
+  for (int k = t.kb; k < t.ke; k += 2) {
+    plane(k, A, B);
+    if (k + 1 < t.ke) plane(k + 1, B, A);
   }
 }
 
@@ -259,11 +264,12 @@ struct VPlane {
   T szz_p, sxz_k, syz_k;                           // szz at k+1; sxz, syz at k
   T sxx_k, sxx_xm, sxy_k, sxy_ym, sxy_xp, syy_k, syy_yp, sxz_xp, syz_ym;
   T cb, vx, vy, vz;
+  T px[3], py[3], pz[3];
 };
 
 template <typename T, int TY3, bool NT>
 __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
-  const Tile3 t = tile3<TY3>(p.nx, p.ny, p.nz, p.kchunk);
+  const Tile3 t = tile3<TY3, false>(p);
   if (!t.ok) return;
   const int i = t.i, j = t.j;
   const int nx = p.nx, ny = p.ny, nz = p.nz;
@@ -282,7 +288,9 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
   const bool r_vz = i <= nx - 2 && j >= 1;
   const bool edge_xy = i == 0 || i == nx - 1 || j == 0 || j == ny - 1;
   const bool src_col = i == p.isrc && j == p.jsrc;
-  auto load = [&](VPlane<T> &L, int kk) {
+  auto load = [&](VPlane<T> &L, int k) {
+    const auto Q = kernarg<Step3D<T>>();
+    const int kk = k - t.kb + 1;
     L.szz_p = CPML_LD(rzz, 0, 0, 1);
     L.sxz_k = CPML_LD(rxz, 0, 0, 0);
     L.syz_k = CPML_LD(ryz, 0, 0, 0);
@@ -299,6 +307,18 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
     L.vx = CPML_LDN(rvx);
     L.vy = CPML_LDN(rvy);
     L.vz = CPML_LDN(rvz);
+    if (inx) {
+      const unsigned m = mxo + k * mxs;
+      L.px[0] = Q->mx[3][m], L.px[1] = Q->mx[4][m], L.px[2] = Q->mx[5][m];
+    }
+    if (iny) {
+      const unsigned m = myo + k * mys;
+      L.py[0] = Q->my[3][m], L.py[1] = Q->my[4][m], L.py[2] = Q->my[5][m];
+    }
+    if (p.sz.in(k)) {
+      const unsigned m = mzo + (unsigned)p.sz.s(k) * mzs;
+      L.pz[0] = Q->mz[3][m], L.pz[1] = Q->mz[4][m], L.pz[2] = Q->mz[5][m];
+    }
   };
   // x / y profile values of this column (loop invariant; only read in the
   // absorbing slabs)
@@ -312,15 +332,17 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
     ya = p.py.a[j]; yb = p.py.b[j]; yK = p.py.K[j];
     yah = p.py.ah[j]; ybh = p.py.bh[j]; yKh = p.py.Kh[j];
   }
-  int kk = 1;
+  constexpr int kk = 1;
   T sxz_m = CPML_LD(rxz, 0, 0, -1), syz_m = CPML_LD(ryz, 0, 0, -1);
   T szz_k = CPML_LD(rzz, 0, 0, 0);
-  VPlane<T> L;
-  load(L, kk);
-  for (int k = t.kb; k < t.ke; ++k, ++kk) {
+  // one plane: L holds its values, N receives the next one's.  The caller
+  // alternates two sets, so no copy waits for the loads in flight, and they are
+  // issued before this plane's stores, so waiting for them does not wait for
+  // those.
+  auto plane = [&](int k, const VPlane<T> &L, VPlane<T> &N) {
     const auto Q = kernarg<Step3D<T>>();
-    VPlane<T> N = L;
-    if (k + 1 < t.ke) load(N, kk + 1);
+    const int kk = k - t.kb + 1;  // buffer plane of k
+    load(N, min(k + 1, t.ke - 1));
     const bool inz = p.sz.in(k);
     const unsigned mzk = mzo + (unsigned)p.sz.s(k) * mzs;
     const T cb = L.cb;
@@ -330,9 +352,9 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
       T dsxx_dx = (L.sxx_k - L.sxx_xm) * p.odx;
       T dsxy_dy = (L.sxy_k - L.sxy_ym) * p.ody;
       T dsxz_dz = (L.sxz_k - sxz_m) * p.odz;
-      if (inx) dsxx_dx = cpml(dsxx_dx, Q->mx[3] + mxo + k * mxs, xa, xb, xK);
-      if (iny) dsxy_dy = cpml(dsxy_dy, Q->my[3] + myo + k * mys, ya, yb, yK);
-      if (inz) dsxz_dz = cpml(dsxz_dz, Q->mz[3] + mzk, Q->pz.a[k], Q->pz.b[k], Q->pz.K[k]);
+      if (inx) dsxx_dx = pml3(dsxx_dx, L.px[0], Q->mx[3] + mxo + k * mxs, xa, xb, xK);
+      if (iny) dsxy_dy = pml3(dsxy_dy, L.py[0], Q->my[3] + myo + k * mys, ya, yb, yK);
+      if (inz) dsxz_dz = pml3(dsxz_dz, L.pz[0], Q->mz[3] + mzk, Q->pz.a[k], Q->pz.b[k], Q->pz.K[k]);
       vxn = cb * (dsxx_dx + dsxy_dy + dsxz_dz) + vxn;
     }
     // vy: 3D:995-1017
@@ -340,9 +362,9 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
       T dsxy_dx = (L.sxy_xp - L.sxy_k) * p.odx;
       T dsyy_dy = (L.syy_yp - L.syy_k) * p.ody;
       T dsyz_dz = (L.syz_k - syz_m) * p.odz;
-      if (inx) dsxy_dx = cpml(dsxy_dx, Q->mx[4] + mxo + k * mxs, xah, xbh, xKh);
-      if (iny) dsyy_dy = cpml(dsyy_dy, Q->my[4] + myo + k * mys, yah, ybh, yKh);
-      if (inz) dsyz_dz = cpml(dsyz_dz, Q->mz[4] + mzk, Q->pz.a[k], Q->pz.b[k], Q->pz.K[k]);
+      if (inx) dsxy_dx = pml3(dsxy_dx, L.px[1], Q->mx[4] + mxo + k * mxs, xah, xbh, xKh);
+      if (iny) dsyy_dy = pml3(dsyy_dy, L.py[1], Q->my[4] + myo + k * mys, yah, ybh, yKh);
+      if (inz) dsyz_dz = pml3(dsyz_dz, L.pz[1], Q->mz[4] + mzk, Q->pz.a[k], Q->pz.b[k], Q->pz.K[k]);
       vyn = cb * (dsxy_dx + dsyy_dy + dsyz_dz) + vyn;
     }
     // vz: 3D:1031-1052 (global k <= NZ-1)
@@ -350,9 +372,9 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
       T dsxz_dx = (L.sxz_xp - L.sxz_k) * p.odx;
       T dsyz_dy = (L.syz_k - L.syz_ym) * p.ody;
       T dszz_dz = (L.szz_p - szz_k) * p.odz;
-      if (inx) dsxz_dx = cpml(dsxz_dx, Q->mx[5] + mxo + k * mxs, xah, xbh, xKh);
-      if (iny) dsyz_dy = cpml(dsyz_dy, Q->my[5] + myo + k * mys, ya, yb, yK);
-      if (inz) dszz_dz = cpml(dszz_dz, Q->mz[5] + mzk, Q->pz.ah[k], Q->pz.bh[k], Q->pz.Kh[k]);
+      if (inx) dsxz_dx = pml3(dsxz_dx, L.px[2], Q->mx[5] + mxo + k * mxs, xah, xbh, xKh);
+      if (iny) dsyz_dy = pml3(dsyz_dy, L.py[2], Q->my[5] + myo + k * mys, ya, yb, yK);
+      if (inz) dszz_dz = pml3(dszz_dz, L.pz[2], Q->mz[5] + mzk, Q->pz.ah[k], Q->pz.bh[k], Q->pz.Kh[k]);
       vzn = cb * (dsxz_dx + dsyz_dy + dszz_dz) + vzn;
     }
     // point force on the cut plane, no density average (3D:1074-1082)
@@ -374,7 +396,12 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
     sxz_m = L.sxz_k;
     syz_m = L.syz_k;
     szz_k = L.szz_p;
-    L = N;
+  };
+  VPlane<T> A, B;
+  load(A, t.kb);
+  for (int k = t.kb; k < t.ke; k += 2) {
+    plane(k, A, B);
+    if (k + 1 < t.ke) plane(k + 1, B, A);
   }
 }
 
@@ -552,18 +579,19 @@ hipError_t launch_velocity2d(int order, const Step2D<T> &p, hipStream_t s) {
 
 template <typename T>
 unsigned ntiles3(const Step3D<T> &p, int ty) {
-  return (unsigned)((p.nx + BX - 1) / BX) * ((p.ny + ty - 1) / ty) *
-         ((p.nz + p.kchunk - 1) / p.kchunk);
+  return (unsigned)plane_tiles3<false>(p.nx, p.ny, ty) * ((p.nz + p.kchunk - 1) / p.kchunk);
 }
 
-// p.tile_y selects the tile height (4, 8 or 16 rows of 64 points)
+// p.tile_y selects the tile height (4, 8 or 16 rows of 64 points; double: at
+// most 8, whose two planes of values fit in registers)
 template <typename T, bool NT>
 static hipError_t stress3d_nt(const Step3D<T> &p, hipStream_t s) {
-  if (p.tile_y == 16)
-    hipLaunchKernelGGL((k_stress3d<T, 16, NT>), dim3(ntiles3(p, 16)), dim3(BX, 16), 0, s, p);
-  else if (p.tile_y == 8)
-    hipLaunchKernelGGL((k_stress3d<T, 8, NT>), dim3(ntiles3(p, 8)), dim3(BX, 8), 0, s, p);
-  else
+  if (p.tile_y >= 8) {
+    if (p.tile_y == 16 && sizeof(T) == 4)
+      hipLaunchKernelGGL((k_stress3d<T, 16, NT>), dim3(ntiles3(p, 16)), dim3(BX, 16), 0, s, p);
+    else
+      hipLaunchKernelGGL((k_stress3d<T, 8, NT>), dim3(ntiles3(p, 8)), dim3(BX, 8), 0, s, p);
+  } else
     hipLaunchKernelGGL((k_stress3d<T, 4, NT>), dim3(ntiles3(p, 4)), dim3(BX, 4), 0, s, p);
   return hipGetLastError();
 }
@@ -575,11 +603,12 @@ hipError_t launch_stress3d(const Step3D<T> &p, hipStream_t s) {
 
 template <typename T, bool NT>
 static hipError_t velocity3d_nt(const Step3D<T> &p, hipStream_t s) {
-  if (p.tile_y == 16)
-    hipLaunchKernelGGL((k_velocity3d<T, 16, NT>), dim3(ntiles3(p, 16)), dim3(BX, 16), 0, s, p);
-  else if (p.tile_y == 8)
-    hipLaunchKernelGGL((k_velocity3d<T, 8, NT>), dim3(ntiles3(p, 8)), dim3(BX, 8), 0, s, p);
-  else
+  if (p.tile_y >= 8) {
+    if (p.tile_y == 16 && sizeof(T) == 4)
+      hipLaunchKernelGGL((k_velocity3d<T, 16, NT>), dim3(ntiles3(p, 16)), dim3(BX, 16), 0, s, p);
+    else
+      hipLaunchKernelGGL((k_velocity3d<T, 8, NT>), dim3(ntiles3(p, 8)), dim3(BX, 8), 0, s, p);
+  } else
     hipLaunchKernelGGL((k_velocity3d<T, 4, NT>), dim3(ntiles3(p, 4)), dim3(BX, 4), 0, s, p);
   return hipGetLastError();
 }
