@@ -33,6 +33,7 @@
 #include "cpml_constdiv.h"
 #include "cpml_device.h"
 #include "cpml_internal.h"
+#include "cpml_record.h"
 
 namespace cpml {
 namespace {
@@ -99,8 +100,11 @@ struct SPlane4 {
 // Float: at least 4 waves per SIMD (128 VGPRs against 132 unbounded, which
 // leave 3); more would spill.
 template <typename T, int TY4>
-__global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_stress3d4(Step3D<T> p) {
-  const Tile3 c = tile3<TY4, kFlat4<T>>(p);
+__global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_stress3d4(Step3D<T> p,
+    Record<T> prev, int lead) {
+  int h;
+  if (lead_block(prev, lead, h)) return;
+  const Tile3 c = tile3<TY4, kFlat4<T>>(p, h);
   if (!c.ok) return;
   const int i = c.i, j = c.j, nx = p.nx, ny = p.ny, nz = p.nz;
   const Chunk4<T> g(p, c);
@@ -245,7 +249,7 @@ struct VPlane4 {
 
 template <typename T, int TY4>
 __global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_velocity3d4(Step3D<T> p) {
-  const Tile3 c = tile3<TY4, kFlat4<T>>(p);
+  const Tile3 c = tile3<TY4, kFlat4<T>>(p, blockIdx.x);
   if (!c.ok) return;
   const int i = c.i, j = c.j, nx = p.nx, ny = p.ny, nz = p.nz;
   const Chunk4<T> g(p, c);
@@ -398,14 +402,19 @@ unsigned ntiles4(const Step3D<T> &p, int ty) {
 // p.tile_y selects the rows per block (4, 8 or 16; double: at most 8, whose two
 // planes of values fit in registers)
 template <typename T>
-hipError_t launch_stress3d4(const Step3D<T> &p, hipStream_t s) {
+hipError_t launch_stress3d4(const Step3D<T> &p, const Record<T> *prev, hipStream_t s) {
+  const int lead = prev ? kLead : 0;
+  const Record<T> rec = prev ? *prev : Record<T>{};
   if (p.tile_y >= 8) {
     if (p.tile_y == 16 && sizeof(T) == 4)
-      hipLaunchKernelGGL((k_stress3d4<T, 16>), dim3(ntiles4(p, 16)), dim3(BX, 16), 0, s, p);
+      hipLaunchKernelGGL((k_stress3d4<T, 16>), dim3(lead + ntiles4(p, 16)), dim3(BX, 16), 0, s, p, rec,
+                       lead);
     else
-      hipLaunchKernelGGL((k_stress3d4<T, 8>), dim3(ntiles4(p, 8)), dim3(BX, 8), 0, s, p);
+      hipLaunchKernelGGL((k_stress3d4<T, 8>), dim3(lead + ntiles4(p, 8)), dim3(BX, 8), 0, s, p, rec,
+                       lead);
   } else
-    hipLaunchKernelGGL((k_stress3d4<T, 4>), dim3(ntiles4(p, 4)), dim3(BX, 4), 0, s, p);
+    hipLaunchKernelGGL((k_stress3d4<T, 4>), dim3(lead + ntiles4(p, 4)), dim3(BX, 4), 0, s, p, rec,
+                       lead);
   return hipGetLastError();
 }
 
@@ -421,8 +430,10 @@ hipError_t launch_velocity3d4(const Step3D<T> &p, hipStream_t s) {
   return hipGetLastError();
 }
 
-template hipError_t launch_stress3d4<float>(const Step3D<float> &, hipStream_t);
-template hipError_t launch_stress3d4<double>(const Step3D<double> &, hipStream_t);
+template hipError_t launch_stress3d4<float>(const Step3D<float> &, const Record<float> *,
+                                             hipStream_t);
+template hipError_t launch_stress3d4<double>(const Step3D<double> &, const Record<double> *,
+                                              hipStream_t);
 template hipError_t launch_velocity3d4<float>(const Step3D<float> &, hipStream_t);
 template hipError_t launch_velocity3d4<double>(const Step3D<double> &, hipStream_t);
 

@@ -151,6 +151,7 @@ struct cpml_solver {
   // (2D items with C-PML code: tb_js)
   int tb = 0, tb_ow = 0, tb_jc = 40, tb_js = 16;
   int *tb_rec = nullptr;        // per-strip receiver lists (device)
+  bool rec_pending = false;     // a single step whose receivers are not recorded yet
   int tb_pending = 0;           // time-blocked launches since the step counter was advanced
   double *tb_epart = nullptr;   // 2D time-blocked energy: per-item sums of every pending level
   size_t tb_epart_cap = 0;      // its size in doubles
@@ -168,7 +169,8 @@ struct cpml_solver {
   void *seis[3] = {};
   int nrec = 0;
   double *ekin = nullptr, *epot = nullptr, *epart = nullptr;
-  int eblocks = 0;
+  int eblocks = 0;              // blocks of the energy pass
+  size_t epart_cap = 0;         // doubles that epart holds
   unsigned long long *scratch_max = nullptr;
   int *scratch_flag = nullptr;
   bool have_medium = false, have_pml = false;
@@ -240,12 +242,12 @@ bool chunk_fits(const cpml_solver *h, int kchunk) {
 // 583 with 8 and 605 with 16), halved for small grids (96 x 80 x 72 float 45 us
 // with 8 planes, 41 with 2; the fused kernel, which recomputes its halo
 // planes, keeps 8), and less where a chunk's buffer would pass 4 GiB.
-int kchunk_of(const cpml_solver *h) {
+int kchunk_of(const cpml_solver *h, bool fused) {
   if (h->kchunk > 0) return h->kchunk;
   const long tiles = (long)((h->nx + 63) / 64) * ((h->ny + h->tile_y - 1) / h->tile_y);
   auto blocks = [&](int k) { return tiles * ((h->nz + k - 1) / k); };
   int k = 8;
-  if (!h->fused) {
+  if (!fused) {
     if (h->order == 4 && blocks(32) >= 4096) k = 32;
     while (k > 2 && blocks(k) < 1024) k /= 2;
   }
@@ -547,7 +549,7 @@ cpml::Step3D<T> step3d(cpml_solver *h) {
   p.fx = static_cast<const T *>(h->fx);
   p.fy = static_cast<const T *>(h->fy);
   p.step = h->step;
-  p.kchunk = kchunk_of(h);
+  p.kchunk = kchunk_of(h, h->fused);
   p.tile_y = h->tile_y;
   p.streaming = h->bytes > cpml::kStreamingBytes;
   return p;
@@ -642,30 +644,112 @@ hipError_t enqueue_fused(cpml_solver *h) {
   return e;
 }
 
+// Single steps whose stress launch finishes the step before (receivers, energy
+// sum, step counter): the elastic two-phase kernels.
+bool lead_record(const cpml_solver *h) { return !h->ade && !h->fused && h->nsls == 0; }
+// ... and whose velocity launch sums the step's energy: orders 2 (and 2D 4, 8),
+// unless the learned boundary changes the velocities after it.
+bool fold_energy(const cpml_solver *h) {
+  return lead_record(h) && h->cadence > 0 && !h->abc && (h->ndim == 2 || h->order == 2);
+}
+// 3D order 2 sums the energy by the velocity launch's tiles, whoever does it.
+bool tiled_energy(const cpml_solver *h) {
+  return h->cadence > 0 && (fold_energy(h) || (h->ndim == 3 && h->order == 2));
+}
+template <typename T>
+cpml::Step3D<T> energy_step3d(cpml_solver *h) {
+  cpml::Step3D<T> p = step3d<T>(h);
+  p.kchunk = kchunk_of(h, false);
+  return p;
+}
+template <typename T>
+int energy_parts(cpml_solver *h) {
+  if (!tiled_energy(h)) return h->eblocks;
+  return h->ndim == 2 ? cpml::energy_tiles<T>(step2d<T>(h))
+                      : cpml::energy_tiles<T>(energy_step3d<T>(h));
+}
+template <typename T>
+cpml::EnergyFold<T> fold_of(cpml_solver *h) {
+  const cpml::Energy<T> e = energy_of<T>(h);
+  cpml::EnergyFold<T> f{};
+  f.lam = e.lam, f.mu = e.mu, f.rho = e.rho;
+  f.i0 = e.i0, f.i1 = e.i1, f.j0 = e.j0, f.j1 = e.j1, f.k0 = e.k0, f.k1 = e.k1;
+  f.cadence = e.cadence;
+  f.corrected3d = e.corrected3d;
+  f.partial = e.partial;
+  return f;
+}
+// Room for the partial sums of the tiles (allocated before any capture).
+int ensure_parts(cpml_solver *h) {
+  if (h->cadence == 0) return CPML_OK;
+  const size_t n = 2 * (size_t)(h->prec == 4 ? energy_parts<float>(h) : energy_parts<double>(h));
+  if (n <= h->epart_cap) return CPML_OK;
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  dev_free(h, *(void **)&h->epart);
+  h->epart_cap = 0;
+  int rc = dev_alloc(h, (void **)&h->epart, n * sizeof(double));
+  if (rc) return rc;
+  h->epart_cap = n;
+  h->graph_dirty = true;
+  return CPML_OK;
+}
+// The pass over the state that sums its energy, the state being that of step
+// *step + offset.
+template <typename T>
+hipError_t enqueue_energy(cpml_solver *h, int offset) {
+  if (tiled_energy(h))
+    return cpml::launch_energy_tiles<T>(energy_step3d<T>(h), fold_of<T>(h), offset, h->stream);
+  cpml::Energy<T> e = energy_of<T>(h);
+  e.offset = offset;
+  return cpml::launch_energy_partial<T>(e, h->eblocks, h->stream);
+}
+// Receivers, energy sum and counter of a single step.
+template <typename T>
+cpml::Record<T> finish_of(cpml_solver *h) {
+  cpml::Record<T> r = record_of<T>(h);
+  r.cadence = h->cadence;
+  r.partial = h->epart;
+  r.nparts = h->cadence > 0 ? energy_parts<T>(h) : 0;
+  r.out_kin = h->ekin;
+  r.out_pot = h->epot;
+  return r;
+}
+
+// A step whose receivers are still to be recorded (rec_pending) is finished by
+// the stress launch of the next one.
 template <typename T>
 hipError_t enqueue_stress(cpml_solver *h) {
+  const cpml::Record<T> rec = finish_of<T>(h);
+  const cpml::Record<T> *prev = h->rec_pending ? &rec : nullptr;
+  h->rec_pending = false;
   if (h->ndim == 2 && h->nsls > 0)
     return cpml::launch_stress2dve<T>(h->order, visco2d<T>(h), h->stream);
-  if (h->ndim == 2) return cpml::launch_stress2d<T>(h->order, step2d<T>(h), h->stream);
-  return h->order == 4 ? cpml::launch_stress3d4<T>(step3d<T>(h), h->stream)
-                       : cpml::launch_stress3d<T>(step3d<T>(h), h->stream);
+  if (h->ndim == 2) return cpml::launch_stress2d<T>(h->order, step2d<T>(h), prev, h->stream);
+  return h->order == 4 ? cpml::launch_stress3d4<T>(step3d<T>(h), prev, h->stream)
+                       : cpml::launch_stress3d<T>(step3d<T>(h), prev, h->stream);
 }
 template <typename T>
 hipError_t enqueue_velocity(cpml_solver *h) {
+  const cpml::EnergyFold<T> ef = fold_energy(h) ? fold_of<T>(h) : cpml::EnergyFold<T>{};
   if (h->ndim == 2 && h->nsls > 0)
     return cpml::launch_velocity2dve<T>(h->order, visco2d<T>(h), h->stream);
-  if (h->ndim == 2) return cpml::launch_velocity2d<T>(h->order, step2d<T>(h), h->stream);
+  if (h->ndim == 2) return cpml::launch_velocity2d<T>(h->order, step2d<T>(h), ef, h->stream);
   return h->order == 4 ? cpml::launch_velocity3d4<T>(step3d<T>(h), h->stream)
-                       : cpml::launch_velocity3d<T>(step3d<T>(h), h->stream);
+                       : cpml::launch_velocity3d<T>(step3d<T>(h), ef, h->stream);
+}
+template <typename T>
+hipError_t enqueue_finish(cpml_solver *h) {
+  h->rec_pending = false;
+  return cpml::launch_record<T>(finish_of<T>(h), h->stream);
 }
 template <typename T>
 hipError_t enqueue_tail(cpml_solver *h) {
-  hipError_t e = hipSuccess;
-  if (h->cadence > 0) {
-    e = cpml::launch_energy<T>(energy_of<T>(h), h->eblocks, h->stream);
+  if (h->cadence > 0 && !fold_energy(h)) {
+    hipError_t e = enqueue_energy<T>(h, 0);
     if (e != hipSuccess) return e;
   }
-  return cpml::launch_record<T>(record_of<T>(h), h->stream);
+  h->rec_pending = lead_record(h);
+  return h->rec_pending ? hipSuccess : enqueue_finish<T>(h);
 }
 
 cpml::SolverView view_of(cpml_solver *h) {
@@ -864,17 +948,22 @@ hipError_t enqueue_tb(cpml_solver *h) {
                               : cpml::launch_tb2d<T>(h->order, h->tb, tb_of<T>(h), h->stream);
   h->cur ^= 1;
   if (e == hipSuccess && h->ndim == 3 && h->cadence > 0) {  // the block's last step, from memory
+    const int offset = (h->tb_pending + 1) * h->tb - 1;
+    e = enqueue_energy<T>(h, offset);
     cpml::Energy<T> en = energy_of<T>(h);
-    en.offset = (h->tb_pending + 1) * h->tb - 1;
-    e = cpml::launch_energy<T>(en, h->eblocks, h->stream);
+    en.offset = offset;
+    if (e == hipSuccess)
+      e = cpml::launch_energy_final<T>(en, energy_parts<T>(h), h->stream);
   }
   ++h->tb_pending;
   return e;
 }
 
-// Brings the step counter (and the 2D energy curve) up to the launches enqueued.
+// Brings the step counter, the receivers of a single step and the 2D energy
+// curve up to the launches enqueued.
 template <typename T>
 hipError_t flush_tb(cpml_solver *h) {
+  if (h->rec_pending) return enqueue_finish<T>(h);
   if (h->tb_pending == 0) return hipSuccess;
   const int steps = h->tb_pending * h->tb;
   h->tb_pending = 0;
@@ -955,6 +1044,7 @@ int build_graph(cpml_solver *h) {
   for (int s = 0; s < graph_units(h) && e == hipSuccess; ++s) e = enqueue_unit_any(h);
   if (e == hipSuccess) e = flush_any(h);
   h->tb_pending = 0;
+  h->rec_pending = false;
   h->cur = slot;  // capture does not execute: the state is still where it was
   hipError_t e2 = hipStreamEndCapture(h->stream, &g);
   if (e != hipSuccess || e2 != hipSuccess) {
@@ -987,6 +1077,8 @@ int enqueue_steps(cpml_solver *h, int n, int *ev_used) {
     if (rc) return rc;
   }
   h->tb_pending = 0;
+  h->rec_pending = false;
+  if (int rc = ensure_parts(h)) return rc;
   const int u = unit_steps(h);
   if (h->ktiming) {
     int rc = ensure_events(h, (size_t)(*ev_used + 3 * n));
@@ -1020,6 +1112,7 @@ int enqueue_steps(cpml_solver *h, int n, int *ev_used) {
       HIPCHK(h, h->prec == 4 ? enqueue_tail<float>(h) : enqueue_tail<double>(h));
       *ev_used += 3;
     }
+    HIPCHK(h, flush_any(h));
     return CPML_OK;
   }
   const int gl = graph_units(h) * u;  // steps per graph replay
@@ -1040,6 +1133,7 @@ int enqueue_steps(cpml_solver *h, int n, int *ev_used) {
   for (; n >= u && tb_active(h); n -= u) HIPCHK(h, enqueue_unit_any(h));
   HIPCHK(h, flush_any(h));
   for (int s = 0; s < n; ++s) HIPCHK(h, enqueue_step_any(h));
+  HIPCHK(h, flush_any(h));
   return CPML_OK;
 }
 
@@ -1574,13 +1668,14 @@ int cpml_gpu_set_energy(cpml_solver *h, int cadence, const int *window, int flag
   dev_free(h, *(void **)&h->ekin);
   dev_free(h, *(void **)&h->epot);
   dev_free(h, *(void **)&h->epart);
+  h->epart_cap = 0;
   if (cadence > 0) {
     h->eblocks = h->prec == 4 ? cpml::energy_blocks<float>(energy_of<float>(h))
                               : cpml::energy_blocks<double>(energy_of<double>(h));
     if ((rc = dev_alloc(h, (void **)&h->ekin, (size_t)h->nstep * sizeof(double)))) return rc;
     if ((rc = dev_alloc(h, (void **)&h->epot, (size_t)h->nstep * sizeof(double)))) return rc;
-    if ((rc = dev_alloc(h, (void **)&h->epart, (size_t)h->eblocks * 2 * sizeof(double))))
-      return rc;
+    h->epart_cap = (size_t)h->eblocks * 2;
+    if ((rc = dev_alloc(h, (void **)&h->epart, h->epart_cap * sizeof(double)))) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
   }
   h->graph_dirty = true;

@@ -166,6 +166,11 @@ struct Record {
   // recorded as step it + skip, and the counter advances by skip + 1 (with
   // nrec = 0 after launches that recorded skip + 1 steps themselves)
   int skip;
+  // energy of the step from nparts pairs of partial sums, where the cadence
+  // (0: off) asks for it
+  const double *partial;
+  int nparts, cadence;
+  double *out_kin, *out_pot;  // [nstep]
 };
 
 // Time-blocked 3D step: nt leapfrog steps per launch, state a -> the arrays
@@ -302,6 +307,16 @@ struct Energy {
   int offset;  // the state is that of step *step + offset (time blocks: NT - 1)
 };
 
+// Energy of the step that a velocity launch computes: a pair of partial sums per
+// tile, for the steps of the cadence (partial null: off).
+template <typename T>
+struct EnergyFold {
+  const T *lam, *mu, *rho;     // raw media (field layout)
+  int i0, i1, j0, j1, k0, k1;  // 0-based inclusive
+  int cadence, corrected3d;
+  double *partial;  // [tiles][2]
+};
+
 // What the learned-boundary code needs of a solver handle: sizes, strides and
 // the current state (interior origin of each field), its stream and device.
 struct SolverView {
@@ -325,13 +340,13 @@ hipError_t abc_enqueue(cpml_abc_net *n, float *corr, const SolverView &v);
 
 // Kernel launchers (defined in the .hip files).
 template <typename T>
-hipError_t launch_stress2d(int order, const Step2D<T> &p, hipStream_t s);
+hipError_t launch_stress2d(int order, const Step2D<T> &p, const Record<T> *prev, hipStream_t s);
 template <typename T>
-hipError_t launch_velocity2d(int order, const Step2D<T> &p, hipStream_t s);
+hipError_t launch_velocity2d(int order, const Step2D<T> &p, const EnergyFold<T> &ef, hipStream_t s);
 template <typename T>
-hipError_t launch_stress3d(const Step3D<T> &p, hipStream_t s);
+hipError_t launch_stress3d(const Step3D<T> &p, const Record<T> *prev, hipStream_t s);
 template <typename T>
-hipError_t launch_velocity3d(const Step3D<T> &p, hipStream_t s);
+hipError_t launch_velocity3d(const Step3D<T> &p, const EnergyFold<T> &ef, hipStream_t s);
 // ADE-PML RK4 step of the 8th-order program: the 2D fields (s), three stage
 // copies of vx vy sxx syy sxy (d[level][field], padded like the fields), the
 // eight memory arrays (padded), the stage tables a, b ([4][n]: x, x_half, y,
@@ -374,7 +389,7 @@ template <typename T>
 hipError_t launch_velocity2dve(int order, const Visco2D<T> &v, hipStream_t s);
 // 4th-order 3D step (elastic part of the 3D viscoelastic program)
 template <typename T>
-hipError_t launch_stress3d4(const Step3D<T> &p, hipStream_t s);
+hipError_t launch_stress3d4(const Step3D<T> &p, const Record<T> *prev, hipStream_t s);
 template <typename T>
 hipError_t launch_velocity3d4(const Step3D<T> &p, hipStream_t s);
 template <typename T>
@@ -406,7 +421,17 @@ template <typename T>
 hipError_t launch_tb2d_multi(int order, int nt, const TB2D<T> *grids, const int4 *items,
                              const int (&n)[4], int waves, int ahead, hipStream_t s);
 template <typename T>
-hipError_t launch_energy(const Energy<T> &p, int nblocks, hipStream_t s);
+hipError_t launch_energy_final(const Energy<T> &p, int nparts, hipStream_t s);
+template <typename T>
+hipError_t launch_energy_tiles(const Step3D<T> &p, const EnergyFold<T> &ef, int offset,
+                               hipStream_t s);
+template <typename T>
+hipError_t launch_energy_partial(const Energy<T> &p, int nblocks, hipStream_t s);
+// tiles of the velocity launch that takes an EnergyFold
+template <typename T>
+int energy_tiles(const Step2D<T> &p);
+template <typename T>
+int energy_tiles(const Step3D<T> &p);
 template <typename T>
 int energy_blocks(const Energy<T> &p);
 // PNM snapshot parameters (Fortran indices): source, PML thickness, the

@@ -24,6 +24,7 @@
 #include "cpml_internal.h"
 #include "cpml_energy.h"
 #include "cpml_points2d.h"
+#include "cpml_record.h"
 
 namespace cpml {
 
@@ -35,35 +36,70 @@ namespace {
 // XCD-aware tile order: the hardware hands workgroup h to XCD h % 8; each XCD
 // gets one contiguous band of tiles (x fastest), so the rows and columns that
 // neighbouring tiles share are read through the same L2.  Sets this thread's
-// grid point (i, j).
+// grid point (i, j) of tile number h.
 template <int TY, int RG>
-__device__ __forceinline__ void tile2d(int nx, int ny, int &i, int &j) {
+__device__ __forceinline__ void tile2d(int h, int nx, int ny, int &i, int &j) {
   const int ntx = (nx + BX - 1) / BX, nt = ntx * ((ny + TY * RG - 1) / (TY * RG));
-  const int h = blockIdx.x, xcd = h & 7, loc = h >> 3;
+  const int xcd = h & 7, loc = h >> 3;
   const int q = nt >> 3, r = nt & 7;
   const int t = xcd * q + min(xcd, r) + loc;
   i = (t % ntx) * BX + threadIdx.x;
   j = (t / ntx) * (TY * RG) + threadIdx.y;
 }
 
+// Sums of a tile's TY wavefronts, to its pair of partial sums.
+template <int TY, typename T>
+__device__ __forceinline__ void tile_energy(const EnergyFold<T> &ef, int tile, double kin,
+                                            double pot) {
+  __shared__ double sk[TY], sp[TY];
+  for (int d = 32; d > 0; d >>= 1) {
+    kin += __shfl_xor(kin, d);
+    pot += __shfl_xor(pot, d);
+  }
+  if (threadIdx.x == 0) {
+    sk[threadIdx.y] = kin;
+    sp[threadIdx.y] = pot;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && threadIdx.y == 0) {
+    for (int w = 1; w < TY; ++w) {
+      kin += sk[w];
+      pot += sp[w];
+    }
+    ef.partial[2 * tile] = kin;
+    ef.partial[2 * tile + 1] = pot;
+  }
+}
+
 // A tile is 64 points by TY*RG rows; the block (64 x TY threads) walks its RG
 // row groups, so each wavefront lives for several rows.
 template <typename T, int ORDER, int TY, int RG, bool NT>
-__global__ __launch_bounds__(BX *TY) void k_stress2d(Step2D<T> p) {
-  int i, j;
-  tile2d<TY, RG>(p.nx, p.ny, i, j);
+__global__ __launch_bounds__(BX *TY) void k_stress2d(Step2D<T> p, Record<T> prev, int lead) {
+  int h, i, j;
+  if (lead_block(prev, lead, h)) return;
+  tile2d<TY, RG>(h, p.nx, p.ny, i, j);
 #pragma unroll
   for (int r = 0; r < RG; ++r)
     if (i < p.nx && j + r * TY < p.ny) stress2d_point<T, ORDER, NT>(p, i, j + r * TY);
 }
 
 template <typename T, int ORDER, int TY, int RG, bool NT>
-__global__ __launch_bounds__(BX *TY) void k_velocity2d(Step2D<T> p) {
+__global__ __launch_bounds__(BX *TY) void k_velocity2d(Step2D<T> p, EnergyFold<T> ef) {
   int i, j;
-  tile2d<TY, RG>(p.nx, p.ny, i, j);
+  tile2d<TY, RG>(blockIdx.x, p.nx, p.ny, i, j);
+  const bool en = ef.partial && *p.step % ef.cadence == 0;
+  double kin = 0.0, pot = 0.0;
 #pragma unroll
   for (int r = 0; r < RG; ++r)
-    if (i < p.nx && j + r * TY < p.ny) velocity2d_point<T, ORDER, NT>(p, i, j + r * TY);
+    if (i < p.nx && j + r * TY < p.ny) {
+      const int jr = j + r * TY;
+      velocity2d_point<T, ORDER, NT>(p, i, jr, [&](T vx, T vy, long c) {
+        if (en && i >= ef.i0 && i <= ef.i1 && jr >= ef.j0 && jr <= ef.j1)
+          point_energy2d(vx, vy, p.sxx[c], p.syy[c], p.sxy[c], p.lam[c], p.mu[c], p.rho[c], kin,
+                         pot);
+      });
+    }
+  if (en) tile_energy<TY>(ef, blockIdx.x, kin, pot);
 }
 
 // ---------------------------------------------------------------- 3D ----
@@ -131,8 +167,10 @@ struct SPlane {
 };
 
 template <typename T, int TY3, bool NT>
-__global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p) {
-  const Tile3 t = tile3<TY3, false>(p);
+__global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p, Record<T> prev, int lead) {
+  int h;
+  if (lead_block(prev, lead, h)) return;
+  const Tile3 t = tile3<TY3, false>(p, h);
   if (!t.ok) return;
   const int i = t.i, j = t.j;
   const int nx = p.nx, ny = p.ny, nz = p.nz;
@@ -263,14 +301,17 @@ template <typename T>
 struct VPlane {
   T szz_p, sxz_k, syz_k;                           // szz at k+1; sxz, syz at k
   T sxx_k, sxx_xm, sxy_k, sxy_ym, sxy_xp, syy_k, syy_yp, sxz_xp, syz_ym;
-  T cb, vx, vy, vz;
+  T cb, vx, vy, vz, la, mu, rho;
   T px[3], py[3], pz[3];
 };
 
-template <typename T, int TY3, bool NT>
-__global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
-  const Tile3 t = tile3<TY3, false>(p);
-  if (!t.ok) return;
+// EN: the energy of the points it computes, summed over the tile (a pass of its
+// own reads the state again: 101 x 641 x 640 double 3451 us per step so, 3005 in
+// here).
+template <typename T, int TY3, bool NT, bool EN>
+__device__ __forceinline__ void velocity3d_tile(const Step3D<T> &p, const Tile3 &t,
+                                                const EnergyFold<T> &ef, bool en, double &kin,
+                                                double &pot) {
   const int i = t.i, j = t.j;
   const int nx = p.nx, ny = p.ny, nz = p.nz;
   const Chunk3<T> g(p, t);
@@ -307,6 +348,10 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
     L.vx = CPML_LDN(rvx);
     L.vy = CPML_LDN(rvy);
     L.vz = CPML_LDN(rvz);
+    if (EN && en) {
+      const long q = i + (long)j * p.ld + (long)k * p.ps;
+      L.la = ef.lam[q], L.mu = ef.mu[q], L.rho = ef.rho[q];
+    }
     if (inx) {
       const unsigned m = mxo + k * mxs;
       L.px[0] = Q->mx[3][m], L.px[1] = Q->mx[4][m], L.px[2] = Q->mx[5][m];
@@ -393,6 +438,10 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
     CPML_ST(vxn, rvx);
     CPML_ST(vyn, rvy);
     CPML_ST(vzn, rvz);
+    if (EN && en && k >= ef.k0 && k <= ef.k1 && i >= ef.i0 && i <= ef.i1 && j >= ef.j0 &&
+        j <= ef.j1)
+      point_energy3d(vxn, vyn, vzn, L.sxx_k, L.syy_k, szz_k, L.sxy_k, L.sxz_k, L.syz_k, L.la, L.mu,
+                     L.rho, ef.corrected3d, kin, pot);
     sxz_m = L.sxz_k;
     syz_m = L.syz_k;
     szz_k = L.szz_p;
@@ -405,6 +454,15 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
   }
 }
 
+template <typename T, int TY3, bool NT, bool EN>
+__global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p, EnergyFold<T> ef) {
+  const Tile3 t = tile3<TY3, false>(p, blockIdx.x);
+  const bool en = EN && *p.step % ef.cadence == 0;
+  double kin = 0.0, pot = 0.0;
+  if (t.ok) velocity3d_tile<T, TY3, NT, EN>(p, t, ef, en, kin, pot);
+  if (EN && en) tile_energy<TY3>(ef, blockIdx.x, kin, pot);
+}
+
 #undef CPML_LD
 #undef CPML_LDN
 #undef CPML_ST
@@ -413,38 +471,12 @@ __global__ __launch_bounds__(BX *TY3) void k_velocity3d(Step3D<T> p) {
 
 template <typename T>
 __global__ __launch_bounds__(kMaxRecBlock) void k_record(Record<T> p) {
-  const int it = *p.step + p.skip;
-  const long row = (long)(it - 1) * p.nrec;
-  for (int r = threadIdx.x; r < p.nrec; r += blockDim.x) {
-    const long q = p.idx[r];
-    p.sx[row + r] = p.avg4 ? (p.vx[q] + p.vx[q + 1] + p.vx[q + p.ld] + p.vx[q + 1 + p.ld]) / T(4)
-                           : p.vx[q];
-    p.sy[row + r] = p.vy[q];
-    if (p.sz) p.sz[row + r] = p.vz[q];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) *p.step = it + 1;
+  record_step(p);
 }
 
 // -------------------------------------------------------------- energy --
 
 constexpr int EB = 256;
-
-__device__ void block_sum2(double &a, double &b) {
-  __shared__ double sa[EB], sb[EB];
-  sa[threadIdx.x] = a;
-  sb[threadIdx.x] = b;
-  __syncthreads();
-  for (int s = EB / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      sa[threadIdx.x] += sa[threadIdx.x + s];
-      sb[threadIdx.x] += sb[threadIdx.x + s];
-    }
-    __syncthreads();
-  }
-  a = sa[0];
-  b = sb[0];
-}
 
 template <typename T>
 __global__ __launch_bounds__(EB) void k_energy_partial(Energy<T> p) {
@@ -460,27 +492,36 @@ __global__ __launch_bounds__(EB) void k_energy_partial(Energy<T> p) {
     const int k = p.k0 + (int)(r / wy);
     cell_energy(p, i + j * p.ld + k * p.ps, kin, pot);
   }
-  block_sum2(kin, pot);
+  block_sum2(threadIdx.x, kin, pot);
   if (threadIdx.x == 0) {
     p.partial[2 * blockIdx.x] = kin;
     p.partial[2 * blockIdx.x + 1] = pot;
   }
 }
 
+// The sums of k_velocity3d's tiles, in its order (so the curve does not depend on
+// who computes it), where that kernel does not compute them itself: time-blocked
+// and fused steps, and steps whose velocities change after it.
+template <typename T, int TY3>
+__global__ __launch_bounds__(BX *TY3) void k_energy_tile3d(Step3D<T> p, EnergyFold<T> ef,
+                                                           int offset) {
+  if ((*p.step + offset) % ef.cadence != 0) return;
+  const Tile3 t = tile3<TY3, false>(p, blockIdx.x);
+  double kin = 0.0, pot = 0.0;
+  if (t.ok && t.i >= ef.i0 && t.i <= ef.i1 && t.j >= ef.j0 && t.j <= ef.j1)
+    for (int k = max(t.kb, ef.k0); k < min(t.ke, ef.k1 + 1); ++k) {
+      const long q = t.i + (long)t.j * p.ld + (long)k * p.ps;
+      point_energy3d(p.vx[q], p.vy[q], p.vz[q], p.sxx[q], p.syy[q], p.szz[q], p.sxy[q], p.sxz[q],
+                     p.syz[q], ef.lam[q], ef.mu[q], ef.rho[q], ef.corrected3d, kin, pot);
+    }
+  tile_energy<TY3>(ef, blockIdx.x, kin, pot);
+}
+
 template <typename T>
 __global__ __launch_bounds__(EB) void k_energy_final(Energy<T> p, int nblocks) {
   const int it = *p.step + p.offset;
   if (it % p.cadence != 0) return;
-  double kin = 0.0, pot = 0.0;
-  for (int b = threadIdx.x; b < nblocks; b += EB) {
-    kin += p.partial[2 * b];
-    pot += p.partial[2 * b + 1];
-  }
-  block_sum2(kin, pot);
-  if (threadIdx.x == 0) {
-    p.out_kin[it - 1] = p.ndim == 2 ? 0.5 * kin : kin;
-    p.out_pot[it - 1] = pot;
-  }
+  energy_final(p, threadIdx.x, it, nblocks, p.ndim == 2);
 }
 
 // ------------------------------------------------- max |v| (stability) --
@@ -525,55 +566,61 @@ __global__ __launch_bounds__(EB) void k_vmax(const T *vx, const T *vy, const T *
 // ------------------------------------------------------------ launchers --
 
 template <typename T, int TY, int RG, bool NT>
-static hipError_t stress2d_nt(int order, const Step2D<T> &p, hipStream_t s) {
-  dim3 grid(((p.nx + BX - 1) / BX) * ((p.ny + TY * RG - 1) / (TY * RG))), block(BX, TY);
-  if (order == 2) hipLaunchKernelGGL((k_stress2d<T, 2, TY, RG, NT>), grid, block, 0, s, p);
-  else if (order == 4) hipLaunchKernelGGL((k_stress2d<T, 4, TY, RG, NT>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((k_stress2d<T, 8, TY, RG, NT>), grid, block, 0, s, p);
+static hipError_t stress2d_nt(int order, const Step2D<T> &p, const Record<T> *prev,
+                              hipStream_t s) {
+  const int lead = prev ? kLead : 0;
+  const Record<T> rec = prev ? *prev : Record<T>{};
+  dim3 grid(lead + ((p.nx + BX - 1) / BX) * ((p.ny + TY * RG - 1) / (TY * RG))), block(BX, TY);
+  if (order == 2) hipLaunchKernelGGL((k_stress2d<T, 2, TY, RG, NT>), grid, block, 0, s, p, rec, lead);
+  else if (order == 4) hipLaunchKernelGGL((k_stress2d<T, 4, TY, RG, NT>), grid, block, 0, s, p, rec, lead);
+  else hipLaunchKernelGGL((k_stress2d<T, 8, TY, RG, NT>), grid, block, 0, s, p, rec, lead);
   return hipGetLastError();
 }
 
 template <typename T, int TY, int RG>
-static hipError_t stress2d_ty(int order, const Step2D<T> &p, hipStream_t s) {
-  return p.streaming ? stress2d_nt<T, TY, RG, true>(order, p, s)
-                     : stress2d_nt<T, TY, RG, false>(order, p, s);
+static hipError_t stress2d_ty(int order, const Step2D<T> &p, const Record<T> *prev,
+                              hipStream_t s) {
+  return p.streaming ? stress2d_nt<T, TY, RG, true>(order, p, prev, s)
+                     : stress2d_nt<T, TY, RG, false>(order, p, prev, s);
 }
 
 template <typename T, int TY, int RG, bool NT>
-static hipError_t velocity2d_nt(int order, const Step2D<T> &p, hipStream_t s) {
+static hipError_t velocity2d_nt(int order, const Step2D<T> &p, const EnergyFold<T> &ef,
+                                hipStream_t s) {
   dim3 grid(((p.nx + BX - 1) / BX) * ((p.ny + TY * RG - 1) / (TY * RG))), block(BX, TY);
-  if (order == 2) hipLaunchKernelGGL((k_velocity2d<T, 2, TY, RG, NT>), grid, block, 0, s, p);
-  else if (order == 4) hipLaunchKernelGGL((k_velocity2d<T, 4, TY, RG, NT>), grid, block, 0, s, p);
-  else hipLaunchKernelGGL((k_velocity2d<T, 8, TY, RG, NT>), grid, block, 0, s, p);
+  if (order == 2) hipLaunchKernelGGL((k_velocity2d<T, 2, TY, RG, NT>), grid, block, 0, s, p, ef);
+  else if (order == 4) hipLaunchKernelGGL((k_velocity2d<T, 4, TY, RG, NT>), grid, block, 0, s, p, ef);
+  else hipLaunchKernelGGL((k_velocity2d<T, 8, TY, RG, NT>), grid, block, 0, s, p, ef);
   return hipGetLastError();
 }
 
 template <typename T, int TY, int RG>
-static hipError_t velocity2d_ty(int order, const Step2D<T> &p, hipStream_t s) {
-  return p.streaming ? velocity2d_nt<T, TY, RG, true>(order, p, s)
-                     : velocity2d_nt<T, TY, RG, false>(order, p, s);
+static hipError_t velocity2d_ty(int order, const Step2D<T> &p, const EnergyFold<T> &ef,
+                              hipStream_t s) {
+  return p.streaming ? velocity2d_nt<T, TY, RG, true>(order, p, ef, s)
+                     : velocity2d_nt<T, TY, RG, false>(order, p, ef, s);
 }
 
 // p.tile_y: rows per tile, 4, 8, 16, or 32 / 64 walked by 16-row blocks
 template <typename T>
-hipError_t launch_stress2d(int order, const Step2D<T> &p, hipStream_t s) {
+hipError_t launch_stress2d(int order, const Step2D<T> &p, const Record<T> *prev, hipStream_t s) {
   switch (p.tile_y) {
-    case 64: return stress2d_ty<T, 16, 4>(order, p, s);
-    case 32: return stress2d_ty<T, 16, 2>(order, p, s);
-    case 16: return stress2d_ty<T, 16, 1>(order, p, s);
-    case 8: return stress2d_ty<T, 8, 1>(order, p, s);
-    default: return stress2d_ty<T, 4, 1>(order, p, s);
+    case 64: return stress2d_ty<T, 16, 4>(order, p, prev, s);
+    case 32: return stress2d_ty<T, 16, 2>(order, p, prev, s);
+    case 16: return stress2d_ty<T, 16, 1>(order, p, prev, s);
+    case 8: return stress2d_ty<T, 8, 1>(order, p, prev, s);
+    default: return stress2d_ty<T, 4, 1>(order, p, prev, s);
   }
 }
 
 template <typename T>
-hipError_t launch_velocity2d(int order, const Step2D<T> &p, hipStream_t s) {
+hipError_t launch_velocity2d(int order, const Step2D<T> &p, const EnergyFold<T> &ef, hipStream_t s) {
   switch (p.tile_y) {
-    case 64: return velocity2d_ty<T, 16, 4>(order, p, s);
-    case 32: return velocity2d_ty<T, 16, 2>(order, p, s);
-    case 16: return velocity2d_ty<T, 16, 1>(order, p, s);
-    case 8: return velocity2d_ty<T, 8, 1>(order, p, s);
-    default: return velocity2d_ty<T, 4, 1>(order, p, s);
+    case 64: return velocity2d_ty<T, 16, 4>(order, p, ef, s);
+    case 32: return velocity2d_ty<T, 16, 2>(order, p, ef, s);
+    case 16: return velocity2d_ty<T, 16, 1>(order, p, ef, s);
+    case 8: return velocity2d_ty<T, 8, 1>(order, p, ef, s);
+    default: return velocity2d_ty<T, 4, 1>(order, p, ef, s);
   }
 }
 
@@ -585,37 +632,46 @@ unsigned ntiles3(const Step3D<T> &p, int ty) {
 // p.tile_y selects the tile height (4, 8 or 16 rows of 64 points; double: at
 // most 8, whose two planes of values fit in registers)
 template <typename T, bool NT>
-static hipError_t stress3d_nt(const Step3D<T> &p, hipStream_t s) {
+static hipError_t stress3d_nt(const Step3D<T> &p, const Record<T> *prev, hipStream_t s) {
+  const int lead = prev ? kLead : 0;
+  const Record<T> rec = prev ? *prev : Record<T>{};
   if (p.tile_y >= 8) {
     if (p.tile_y == 16 && sizeof(T) == 4)
-      hipLaunchKernelGGL((k_stress3d<T, 16, NT>), dim3(ntiles3(p, 16)), dim3(BX, 16), 0, s, p);
+      hipLaunchKernelGGL((k_stress3d<T, 16, NT>), dim3(lead + ntiles3(p, 16)), dim3(BX, 16), 0, s, p,
+                       rec, lead);
     else
-      hipLaunchKernelGGL((k_stress3d<T, 8, NT>), dim3(ntiles3(p, 8)), dim3(BX, 8), 0, s, p);
+      hipLaunchKernelGGL((k_stress3d<T, 8, NT>), dim3(lead + ntiles3(p, 8)), dim3(BX, 8), 0, s, p,
+                       rec, lead);
   } else
-    hipLaunchKernelGGL((k_stress3d<T, 4, NT>), dim3(ntiles3(p, 4)), dim3(BX, 4), 0, s, p);
+    hipLaunchKernelGGL((k_stress3d<T, 4, NT>), dim3(lead + ntiles3(p, 4)), dim3(BX, 4), 0, s, p,
+                       rec, lead);
   return hipGetLastError();
 }
 
 template <typename T>
-hipError_t launch_stress3d(const Step3D<T> &p, hipStream_t s) {
-  return p.streaming ? stress3d_nt<T, true>(p, s) : stress3d_nt<T, false>(p, s);
+hipError_t launch_stress3d(const Step3D<T> &p, const Record<T> *prev, hipStream_t s) {
+  return p.streaming ? stress3d_nt<T, true>(p, prev, s) : stress3d_nt<T, false>(p, prev, s);
 }
 
-template <typename T, bool NT>
-static hipError_t velocity3d_nt(const Step3D<T> &p, hipStream_t s) {
+template <typename T, bool NT, bool EN>
+static hipError_t velocity3d_nt(const Step3D<T> &p, const EnergyFold<T> &ef, hipStream_t s) {
   if (p.tile_y >= 8) {
     if (p.tile_y == 16 && sizeof(T) == 4)
-      hipLaunchKernelGGL((k_velocity3d<T, 16, NT>), dim3(ntiles3(p, 16)), dim3(BX, 16), 0, s, p);
+      hipLaunchKernelGGL((k_velocity3d<T, 16, NT, EN>), dim3(ntiles3(p, 16)), dim3(BX, 16), 0, s, p, ef);
     else
-      hipLaunchKernelGGL((k_velocity3d<T, 8, NT>), dim3(ntiles3(p, 8)), dim3(BX, 8), 0, s, p);
+      hipLaunchKernelGGL((k_velocity3d<T, 8, NT, EN>), dim3(ntiles3(p, 8)), dim3(BX, 8), 0, s, p, ef);
   } else
-    hipLaunchKernelGGL((k_velocity3d<T, 4, NT>), dim3(ntiles3(p, 4)), dim3(BX, 4), 0, s, p);
+    hipLaunchKernelGGL((k_velocity3d<T, 4, NT, EN>), dim3(ntiles3(p, 4)), dim3(BX, 4), 0, s, p, ef);
   return hipGetLastError();
 }
 
 template <typename T>
-hipError_t launch_velocity3d(const Step3D<T> &p, hipStream_t s) {
-  return p.streaming ? velocity3d_nt<T, true>(p, s) : velocity3d_nt<T, false>(p, s);
+hipError_t launch_velocity3d(const Step3D<T> &p, const EnergyFold<T> &ef, hipStream_t s) {
+  if (ef.partial)
+    return p.streaming ? velocity3d_nt<T, true, true>(p, ef, s)
+                       : velocity3d_nt<T, false, true>(p, ef, s);
+  return p.streaming ? velocity3d_nt<T, true, false>(p, ef, s)
+                     : velocity3d_nt<T, false, false>(p, ef, s);
 }
 
 template <typename T>
@@ -633,9 +689,34 @@ int energy_blocks(const Energy<T> &p) {
 }
 
 template <typename T>
-hipError_t launch_energy(const Energy<T> &p, int nblocks, hipStream_t s) {
+int energy_tiles(const Step2D<T> &p) {
+  return (p.nx + BX - 1) / BX * ((p.ny + p.tile_y - 1) / p.tile_y);
+}
+template <typename T>
+int energy_tiles(const Step3D<T> &p) {
+  return (int)ntiles3(p, p.tile_y == 16 && sizeof(T) == 4 ? 16 : p.tile_y >= 8 ? 8 : 4);
+}
+
+template <typename T>
+hipError_t launch_energy_partial(const Energy<T> &p, int nblocks, hipStream_t s) {
   hipLaunchKernelGGL(k_energy_partial<T>, dim3(nblocks), dim3(EB), 0, s, p);
-  hipLaunchKernelGGL(k_energy_final<T>, dim3(1), dim3(EB), 0, s, p, nblocks);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_energy_tiles(const Step3D<T> &p, const EnergyFold<T> &ef, int offset,
+                               hipStream_t s) {
+  const int ty = p.tile_y == 16 && sizeof(T) == 4 ? 16 : p.tile_y >= 8 ? 8 : 4;
+  const dim3 grid(ntiles3(p, ty)), block(BX, ty);
+  if (ty == 16) hipLaunchKernelGGL((k_energy_tile3d<T, 16>), grid, block, 0, s, p, ef, offset);
+  else if (ty == 8) hipLaunchKernelGGL((k_energy_tile3d<T, 8>), grid, block, 0, s, p, ef, offset);
+  else hipLaunchKernelGGL((k_energy_tile3d<T, 4>), grid, block, 0, s, p, ef, offset);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_energy_final(const Energy<T> &p, int nparts, hipStream_t s) {
+  hipLaunchKernelGGL(k_energy_final<T>, dim3(1), dim3(EB), 0, s, p, nparts);
   return hipGetLastError();
 }
 
@@ -738,12 +819,17 @@ hipError_t launch_color_image(const T *f, int nx, int ny, long ld, unsigned long
 }
 
 #define CPML_INSTANTIATE(T)                                                                     \
-  template hipError_t launch_stress2d<T>(int, const Step2D<T> &, hipStream_t);                \
-  template hipError_t launch_velocity2d<T>(int, const Step2D<T> &, hipStream_t);              \
-  template hipError_t launch_stress3d<T>(const Step3D<T> &, hipStream_t);                     \
-  template hipError_t launch_velocity3d<T>(const Step3D<T> &, hipStream_t);                   \
+  template hipError_t launch_stress2d<T>(int, const Step2D<T> &, const Record<T> *, hipStream_t);                \
+  template hipError_t launch_velocity2d<T>(int, const Step2D<T> &, const EnergyFold<T> &, hipStream_t);              \
+  template hipError_t launch_stress3d<T>(const Step3D<T> &, const Record<T> *, hipStream_t);                     \
+  template hipError_t launch_velocity3d<T>(const Step3D<T> &, const EnergyFold<T> &, hipStream_t);                   \
   template hipError_t launch_record<T>(const Record<T> &, hipStream_t);                       \
-  template hipError_t launch_energy<T>(const Energy<T> &, int, hipStream_t);                  \
+  template hipError_t launch_energy_tiles<T>(const Step3D<T> &, const EnergyFold<T> &, int,   \
+                                             hipStream_t);                                    \
+  template hipError_t launch_energy_final<T>(const Energy<T> &, int, hipStream_t);            \
+  template hipError_t launch_energy_partial<T>(const Energy<T> &, int, hipStream_t);          \
+  template int energy_tiles<T>(const Step2D<T> &);                                            \
+  template int energy_tiles<T>(const Step3D<T> &);                                            \
   template int energy_blocks<T>(const Energy<T> &);                                           \
   template hipError_t launch_vmax<T>(const T *, const T *, const T *, int, int, int, long, long, \
                                      unsigned long long *, hipStream_t);                      \

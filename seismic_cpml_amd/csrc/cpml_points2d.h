@@ -71,8 +71,9 @@ __device__ __forceinline__ void stress2d_point(const Step2D<T> &p, int i, int j)
 
 // velocity + C-PML, source and rigid edges at grid point (i, j):
 // 2D2:606-680 (2D4:607-681)
-template <typename T, int ORDER, bool NT>
-__device__ __forceinline__ void velocity2d_point(const Step2D<T> &p, int i, int j) {
+// `done` gets the new velocities and the point's offset.
+template <typename T, int ORDER, bool NT, typename F>
+__device__ __forceinline__ void velocity2d_point(const Step2D<T> &p, int i, int j, F &&done) {
   const long ld = p.ld;
   const long c = i + j * ld;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
@@ -110,6 +111,11 @@ __device__ __forceinline__ void velocity2d_point(const Step2D<T> &p, int i, int 
   }
   st_once<NT>(p.vx + c, vxn);
   st_once<NT>(p.vy + c, vyn);
+  done(vxn, vyn, c);
+}
+template <typename T, int ORDER, bool NT>
+__device__ __forceinline__ void velocity2d_point(const Step2D<T> &p, int i, int j) {
+  velocity2d_point<T, ORDER, NT>(p, i, j, [](T, T, long) {});
 }
 
 }  // namespace cpml
