@@ -126,7 +126,10 @@ long round_up(long v, long m) { return (v + m - 1) / m * m; }
 
 }  // namespace
 
-constexpr size_t kStageBytes = 4 << 20;
+// Pinned staging buffers: an eighth of the field between these, since pinning
+// costs 0.3 ms per MiB, once per handle (the first copy of 1013 x 1187 floats 1.4 ms
+// with 1 MiB and 2.1 with 4; a later one of 4096 x 4096 5.4 and 2.4).
+constexpr size_t kStageMin = 1 << 20, kStageMax = 4 << 20;
 
 struct cpml_solver {
   int ndim = 2, order = 2, prec = 8, nx = 0, ny = 0, nz = 1, npml = 0, nstep = 0;
@@ -356,14 +359,15 @@ int stage_rows(cpml_solver *h, bool pack, void *grid_alloc, void *dense, int row
 // Copy the interior of a host grid array into / out of a padded device array
 // (ghost cells of the host array are neither read nor written).  The device
 // packs stretches of rows straight into (or unpacks them from) one of two
-// pinned buffers of 4 MiB while the host copies the other: a pitched copy to
+// pinned buffers while the host copies the other: a pitched copy to
 // ordinary memory costs the runtime 6 us per row and 500 us per plane (50 float steps
 // at 96 x 80 x 72 and three fields read: 123 -> 3.8 ms; 100 at 1013 x 1187 and
 // two fields: 20.3 -> 3.3 ms).
 int copy_padded(cpml_solver *h, bool download, void *grid_alloc, char *host) {
   const size_t row = h->nx * h->esize;
   const int rows = h->ny * (h->ndim == 3 ? h->nz : 1);
-  const int per = (int)std::clamp<size_t>(kStageBytes / row, 1, rows);
+  const size_t bytes = std::clamp(rows * row / 8, kStageMin, kStageMax);
+  const int per = (int)std::clamp<size_t>(bytes / row, 1, rows);
   for (int q = 0; q < 2; ++q) {
     if (!h->stage_ev[q])
       HIPCHK(h, hipEventCreateWithFlags(&h->stage_ev[q], hipEventDisableTiming));

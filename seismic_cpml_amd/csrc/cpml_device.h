@@ -142,6 +142,21 @@ __device__ __forceinline__ int first_from(const int *a, int lo, int hi, int v) {
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
+// Loads and stores through a scalar base and a 32-bit byte offset of the lane
+// (explicitly global memory: the batch reads the bases from a table, where the
+// compiler would otherwise emit flat accesses).
+template <typename T>
+using Glb = __attribute__((address_space(1))) T;
+template <typename T>
+__device__ __forceinline__ T ld_at(const T *base, unsigned byte_off) {
+  return *reinterpret_cast<const Glb<T> *>(
+      reinterpret_cast<const Glb<char> *>((const Glb<T> *)base) + byte_off);
+}
+template <typename T>
+__device__ __forceinline__ void st_at(T *base, unsigned byte_off, T x) {
+  *reinterpret_cast<Glb<T> *>(reinterpret_cast<Glb<char> *>((Glb<T> *)base) + byte_off) = x;
+}
+
 // Raw buffer resource over `bytes` bytes at p (gfx9 family word 3).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes,

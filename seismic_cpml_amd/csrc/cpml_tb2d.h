@@ -94,21 +94,6 @@ struct Int {
   static constexpr int value = V;
 };
 
-// Loads and stores through a scalar base and a 32-bit byte offset of the lane
-// (explicitly global memory: the batch reads the bases from a table, where the
-// compiler would otherwise emit flat accesses).
-template <typename T>
-using Glb = __attribute__((address_space(1))) T;
-template <typename T>
-__device__ __forceinline__ T ld_at(const T *base, unsigned byte_off) {
-  return *reinterpret_cast<const Glb<T> *>(
-      reinterpret_cast<const Glb<char> *>((const Glb<T> *)base) + byte_off);
-}
-template <typename T>
-__device__ __forceinline__ void st_at(T *base, unsigned byte_off, T x) {
-  *reinterpret_cast<Glb<T> *>(reinterpret_cast<Glb<char> *>((Glb<T> *)base) + byte_off) = x;
-}
-
 template <typename T>
 __device__ __forceinline__ T ld_el(const T *base, long element) {
   return *((const Glb<T> *)base + element);
