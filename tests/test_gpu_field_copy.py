@@ -1,10 +1,11 @@
 """set_field / field through the pinned staging buffers: one and several
-buffers' worth, an odd number of buffers, rows that do not fill a wavefront,
-and fields whose host arrays carry ghost cells.
+buffers' worth, an odd number of buffers, rows that do not fill a wavefront, and
+arrays that the caller has pinned.
 
 Bar: the values come back bit for bit, and other fields keep theirs."""
 import numpy as np
 import pytest
+import torch
 
 from seismic_cpml_amd import CpmlGpu
 
@@ -24,6 +25,11 @@ def test_field_round_trip(ndim, order, n, prec):
         a = {k: rng.standard_normal(shape).astype(real) for k in ("vx", "sigmaxy")}
         for k, v in a.items():
             s.set_field(k, v)
+        pinned = torch.empty(shape, dtype=torch.float32 if prec == 4 else torch.float64,
+                             pin_memory=True)
+        a["sigmaxx"] = pinned.numpy()
+        a["sigmaxx"][:] = a["vx"][::-1]
+        s.set_field("sigmaxx", a["sigmaxx"])
         for k, v in a.items():
             np.testing.assert_array_equal(s.field(k), v)
         assert not s.field("vy").any()
