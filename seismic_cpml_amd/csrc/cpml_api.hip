@@ -363,22 +363,25 @@ int stage_rows(cpml_solver *h, bool pack, void *grid_alloc, void *dense, int row
 // ordinary memory costs the runtime 6 us per row and 500 us per plane (50 float steps
 // at 96 x 80 x 72 and three fields read: 123 -> 3.8 ms; 100 at 1013 x 1187 and
 // two fields: 20.3 -> 3.3 ms).
-// 2D arrays that the caller has pinned are copied as they are (4096^2 float set in
-// 1.2 ms; through the buffers 2.4).
+// Arrays that the caller has pinned are copied as they are, plane by plane, where
+// the planes are worth a copy each (4096^2 float set in 1.2 ms, through the
+// buffers 2.4; 96 x 80 x 72 through the buffers 0.09).
 int copy_padded(cpml_solver *h, bool download, void *grid_alloc, char *host) {
   const size_t row = h->nx * h->esize;
   hipPointerAttribute_t attr{};
   const bool pinned = hipPointerGetAttributes(&attr, host) == hipSuccess &&
                       attr.type == hipMemoryTypeHost;
   (void)hipGetLastError();  // ordinary memory is an error to some runtimes
-  if (pinned && h->ndim == 2) {
-    char *g = static_cast<char *>(grid_alloc) + h->base * h->esize;
-    char *p = host + host_at(h, 0, 0, 0) * h->esize;
+  if (pinned && (h->ndim == 2 || row * h->ny >= kStageMin)) {
     const size_t gp = h->ld * h->esize, hp = host_x(h) * h->esize;
-    HIPCHK(h, hipMemcpy2DAsync(download ? p : g, download ? hp : gp, download ? g : p,
-                               download ? gp : hp, row, h->ny,
-                               download ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice,
-                               h->stream));
+    for (int k = 0; k < (h->ndim == 3 ? h->nz : 1); ++k) {
+      char *g = static_cast<char *>(grid_alloc) + (h->base + k * h->ps) * h->esize;
+      char *p = host + host_at(h, 0, 0, k) * h->esize;
+      HIPCHK(h, hipMemcpy2DAsync(download ? p : g, download ? hp : gp, download ? g : p,
+                                 download ? gp : hp, row, h->ny,
+                                 download ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice,
+                                 h->stream));
+    }
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return CPML_OK;
   }

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("ndim,order,n", [(2, 2, (61, 50, 1)), (2, 4, (1301, 1403, 1)),
                                           (2, 8, (4000, 1100, 1)), (3, 2, (96, 80, 72)),
-                                          (3, 2, (30, 257, 300)), (3, 4, (191, 203, 131))])
+                                          (3, 2, (30, 257, 300)), (3, 4, (191, 203, 131)),
+                                          (3, 2, (640, 610, 45))])
 @pytest.mark.parametrize("prec", [4, 8])
 def test_field_round_trip(ndim, order, n, prec):
     nx, ny, nz = n
