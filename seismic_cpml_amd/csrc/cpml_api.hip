@@ -242,9 +242,9 @@ bool chunk_fits(const cpml_solver *h, int kchunk) {
 // halo planes again, so deep chunks read less, but the machine wants about four
 // blocks per CU: 8 planes (order 4, whose halo is deeper, 32 where that leaves
 // four rounds of blocks: 210 x 800 x 220 float 1442 and 1382 us per step, 256^3
-// 583 with 8 and 605 with 16), halved for small grids (96 x 80 x 72 float 45 us
-// with 8 planes, 41 with 2; the fused kernel, which recomputes its halo
-// planes, keeps 8), and less where a chunk's buffer would pass 4 GiB.
+// 583 with 8 and 605 with 16), halved for small grids (96 x 80 x 72 float 47 us
+// with 8 planes, 30 with 2; order 4, 100 x 90 x 80, 62 with 8, 47 with 4 and 50 with
+// 2; the fused kernel, which recomputes its halo planes, keeps 8), and less where a chunk's buffer would pass 4 GiB.
 int kchunk_of(const cpml_solver *h, bool fused) {
   if (h->kchunk > 0) return h->kchunk;
   const long tiles = (long)((h->nx + 63) / 64) * ((h->ny + h->tile_y - 1) / h->tile_y);
@@ -252,7 +252,7 @@ int kchunk_of(const cpml_solver *h, bool fused) {
   int k = 8;
   if (!fused) {
     if (h->order == 4 && blocks(32) >= 4096) k = 32;
-    while (k > 2 && blocks(k) < 1024) k /= 2;
+    while (k > (h->order == 4 ? 4 : 2) && blocks(k) < 1024) k /= 2;
   }
   while (k > 1 && !chunk_fits(h, k)) --k;
   return k;

@@ -113,7 +113,8 @@ __global__ __launch_bounds__(BX *TY) void k_velocity2d(Step2D<T> p, EnergyFold<T
 // variables included, are issued before the arithmetic and stores of plane k
 // into the other of two register sets.  Bound by HBM latency and rate: with one
 // set copied at each plane's end the copies waited for those loads and stores
-// (200^3 float 317 us per step, now 273; 96 x 80 x 72 66, now 45).
+// (200^3 float 317 us per step, now 276; 96 x 80 x 72 66, now 47, both with 8
+// planes per chunk; 768^3 11.29 and 11.27 ms).
 
 // Geometry of the rebased chunk buffers of one tile.
 template <typename T>
@@ -243,7 +244,7 @@ __global__ __launch_bounds__(BX *TY3) void k_stress3d(Step3D<T> p, Record<T> pre
   auto plane = [&](int k, const SPlane<T> &L, SPlane<T> &N) {
     const auto Q = kernarg<Step3D<T>>();
     const int kk = k - t.kb + 1;  // buffer plane of k
-    load(N, min(k + 1, t.ke - 1));
+    if (k + 1 < t.ke) load(N, k + 1);
     const bool inz = p.sz.in(k);
     const unsigned mzk = mzo + (unsigned)p.sz.s(k) * mzs;
     const T cl = L.cl, cm = L.cm;
@@ -387,7 +388,7 @@ __device__ __forceinline__ void velocity3d_tile(const Step3D<T> &p, const Tile3 
   auto plane = [&](int k, const VPlane<T> &L, VPlane<T> &N) {
     const auto Q = kernarg<Step3D<T>>();
     const int kk = k - t.kb + 1;  // buffer plane of k
-    load(N, min(k + 1, t.ke - 1));
+    if (k + 1 < t.ke) load(N, k + 1);
     const bool inz = p.sz.in(k);
     const unsigned mzk = mzo + (unsigned)p.sz.s(k) * mzs;
     const T cb = L.cb;
