@@ -40,7 +40,7 @@
 // LDS, and the owned columns are whole 64-byte sectors (a store of part of one
 // reads it back).  Per launch of 2 steps, before and after: 4096^2 order 4
 // float 410 -> 280 us; 1701 x 1403 order 2 double with the energy curve 207 ->
-// 101; 32 shots of 320 to 560 points a side, order 4 float, 1577 -> 990.
+// 101; 32 uneven shots of up to 2048 points a side, order 4 float, 1577 -> 990.
 #pragma once
 
 #include <algorithm>
