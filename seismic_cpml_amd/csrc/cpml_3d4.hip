@@ -407,8 +407,8 @@ hipError_t launch_stress3d4(const Step3D<T> &p, const Record<T> *prev, hipStream
   const Record<T> rec = prev ? *prev : Record<T>{};
   if (p.tile_y >= 8) {
     if (p.tile_y == 16 && sizeof(T) == 4)
-      hipLaunchKernelGGL((k_stress3d4<T, 16>), dim3(lead + ntiles4(p, 16)), dim3(BX, 16), 0, s, p, rec,
-                       lead);
+      hipLaunchKernelGGL((k_stress3d4<T, 16>), dim3(lead + ntiles4(p, 16)), dim3(BX, 16), 0, s,
+                         p, rec, lead);
     else
       hipLaunchKernelGGL((k_stress3d4<T, 8>), dim3(lead + ntiles4(p, 8)), dim3(BX, 8), 0, s, p, rec,
                        lead);

@@ -37,9 +37,9 @@ inline __host__ __device__ int plane_tiles3(int nx, int ny, int ty) {
   return FLAT ? (int)(((long)nx * groups + BX - 1) / BX) : (nx + BX - 1) / BX * groups;
 }
 // Tile number h of the launch.  Workgroups are dispatched round-robin over the
-// 8 XCDs; each XCD gets one contiguous band of tiles (x fastest, then y, then z chunk) so the tiles that
-// read each other's halo rows share its L2; the z chunks are interleaved over
-// the bands (zchunk_of).
+// 8 XCDs; each XCD gets one contiguous band of tiles (x fastest, then y, then z
+// chunk) so the tiles that read each other's halo rows share its L2; the z chunks
+// are interleaved over the bands (zchunk_of).
 template <int TY, bool FLAT, typename P>
 __device__ __forceinline__ Tile3 tile3(const P &p, int h) {
   const int nxy = plane_tiles3<FLAT>(p.nx, p.ny, TY);
