@@ -40,6 +40,7 @@
 #include "cpml_energy.h"
 #include "cpml_internal.h"
 #include "cpml_points2d.h"
+#include "cpml_tb_geom.h"
 
 namespace cpml {
 namespace {
@@ -594,20 +595,12 @@ int upload_tables(cpml_batch *b) {
       P.a.sx = s.sx;
       P.a.sy = s.sy;
       P.ow = b->tb_ow;
+      P.jc = b->tb_jc;
+      P.js = b->tb_js;
       cpml::tb2d_split(b->order, b->tb, P);
-      auto rows = [&](int cls, int j0, int j1, int step, int t0, int t1) {
-        for (int r = j0; r < j1; r += step)
-          for (int t = t0; t < t1; ++t)
-            it[cls].push_back(make_int4(q, t, r, std::min(r + step, j1)));
-      };
-      rows(0, P.y0, P.y1, b->tb_jc, P.sx0, P.sx1);
-      for (int r = 0; r < s.ny; r += b->tb_js) {  // strips at the x slabs
-        const int e = std::min(r + b->tb_js, s.ny), cls = r >= P.y0 && e <= P.y1 ? 1 : 3;
-        rows(cls, r, e, b->tb_js, 0, P.sx0);
-        rows(cls, r, e, b->tb_js, P.sx1, P.nstrips);
-      }
-      rows(2, 0, P.y0, b->tb_js, P.sx0, P.sx1);
-      rows(2, P.y1, s.ny, b->tb_js, P.sx0, P.sx1);
+      cpml::tb2d_list(P, [&](const cpml::Tb2dItem &i) {
+        it[i.cls].push_back(make_int4(q, i.ts, i.jb, i.je));
+      });
     }
     int n = 0;
     for (int k = 0; k < 4; ++k) n += b->nitems[k] = (int)it[k].size();

@@ -48,6 +48,7 @@
 #include "cpml_device.h"
 #include "cpml_energy.h"
 #include "cpml_internal.h"
+#include "cpml_tb_geom.h"
 
 namespace cpml {
 namespace {
@@ -189,23 +190,12 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
   auto ylo = [&](int j) { return !SY || (j >= 1 && j < ny); };
   auto yhi = [&](int j) { return !SY || (j >= 0 && j <= ny - 2); };
 
-  // byte offsets from the ghost corner (-1, rl) of each array
   const int s0 = jb - (2 * NT - 1) * r, s1 = je - 1 + (2 * NT - 1) * r;
-  const int rl = max(s0 - r, -1);
-  const int ic = min(max(i, -1), nx);
-  constexpr unsigned es = sizeof(T);
-  const unsigned vo = (unsigned)(ic + 1) * es, ldb = (unsigned)P->a.ld * es;
-  const long corner = (long)rl * P->a.ld - 1;
-  auto at = [&](int j) -> unsigned {
-    const int jj = SY ? min(max(j, -1), ny) : j;
-    return (unsigned)(jj - rl) * ldb + vo;
-  };
-  const bool inx = SX && sx.in(i);
-  const bool kx1 = sx.k1, ky1 = sy.k1;
-  // x-slab arrays: byte offset of this column's row rl and the row pitch there
-  const unsigned sxw = i < sx.wl ? sx.wl : sx.wr;
-  const long sxb = inx ? sx.at(i, 0, ny) : 0;
-  auto ox = [&](int j) { return sxb + (long)(sxw * (unsigned)j); };
+  const Tb2dLane<T, SX, SY> L(i, s0 - r, nx, ny, P->a.ld, sx);
+  const long corner = L.corner;
+  const bool inx = L.inx, kx1 = sx.k1, ky1 = sy.k1;
+  auto at = [&](int j) { return L.at(j); };
+  auto ox = [&](int j) { return L.ox(j); };
   T pxa = T(0), pxb = T(0), pxah = T(0), pxbh = T(0);
   if (SX && inx) pxa = P->a.px.a[i], pxb = P->a.px.b[i], pxah = P->a.px.ah[i], pxbh = P->a.px.bh[i];
 
@@ -286,8 +276,8 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
       ly[F] = ly[F + 1] = T(0);
       if (col_in && sy.in(j)) {
         const long b = Q->a.mld * sy.s(j);
-        ly[F] = ld_at(Q->a.my[F] + b, (unsigned)ic * es);
-        ly[F + 1] = ld_at(Q->a.my[F + 1] + b, (unsigned)ic * es);
+        ly[F] = ld_at(Q->a.my[F] + b, L.mo);
+        ly[F + 1] = ld_at(Q->a.my[F + 1] + b, L.mo);
       }
     }
   };
@@ -444,8 +434,8 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
         }
         if (SY && sy.in(pr)) {
           const long b = Q->a.mld * sy.s(pr);
-          st_at(Q->my[0] + b, (unsigned)ic * es, npy0);
-          st_at(Q->my[1] + b, (unsigned)ic * es, npy1);
+          st_at(Q->my[0] + b, L.mo, npy0);
+          st_at(Q->my[1] + b, L.mo, npy1);
         }
       }
       if (m == 1 && s < s1) {
@@ -533,8 +523,8 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
         }
         if (SY && sy.in(qr)) {
           const long b = Q->a.mld * sy.s(qr);
-          st_at(Q->my[2] + b, (unsigned)ic * es, npy2);
-          st_at(Q->my[3] + b, (unsigned)ic * es, npy3);
+          st_at(Q->my[2] + b, L.mo, npy2);
+          st_at(Q->my[3] + b, L.mo, npy3);
         }
       }
       if ((SX || SY) && m == 1 && s < s1) load_m(Q, Int<2>{}, s + 1 - r);

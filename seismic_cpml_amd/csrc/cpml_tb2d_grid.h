@@ -7,41 +7,18 @@
 namespace cpml {
 namespace {
 
-// One grid.  Items with C-PML code in chunks of js rows: those of the x slabs'
-// strips (all rows), then those of the other strips (rows below y0, then from
-// y1); they are few, with more code each, and shorter chunks end sooner.  Then
-// the slab-free ones: strips [sx0, sx1) x chunks of jc rows of [y0, y1).
+// One grid: an item (tb2d_item_at) per wavefront.
 template <typename T, int ORDER, int NT, bool EN>
 __global__ __launch_bounds__(64 * WPB, (min_waves<T, ORDER, NT>())) void k_tb2d(TB2D<T> P) {
   __shared__ T delay[WPB][tb2d_delay_words<ORDER, NT, 3>() * 64 + 1];
   const int wv = threadIdx.x >> 6;
   const Tb2dItems n = tb2d_items(P);
-  const int nslab = n.edge + n.cap;
   const int item = __builtin_amdgcn_readfirstlane(
-      xcd_item(blockIdx.x & 7, (blockIdx.x >> 3) * WPB + wv, nslab, n.clean));
+      xcd_item(blockIdx.x & 7, (blockIdx.x >> 3) * WPB + wv, n.edge + n.cap, n.clean));
   if (item < 0) return;
-  const int bx = P.sx1 - P.sx0;
-  int ts, jb, je, cls;
-  if (item < n.edge) {
-    const int wx = P.nstrips - bx, u = item % wx;
-    ts = u < P.sx0 ? u : u + bx;
-    jb = item / wx * P.js;
-    je = min(jb + P.js, P.a.ny);
-    cls = jb >= P.y0 && je <= P.y1 ? 1 : 3;
-  } else if (item < nslab) {
-    const int u = item - n.edge, c = u / bx, low = (P.y0 + P.js - 1) / P.js;
-    ts = P.sx0 + u % bx;
-    jb = c < low ? c * P.js : P.y1 + (c - low) * P.js;
-    je = min(jb + P.js, c < low ? P.y0 : P.a.ny);
-    cls = 2;
-  } else {
-    const int u = item - nslab;
-    ts = P.sx0 + u % bx;
-    jb = P.y0 + u / bx * P.jc;
-    je = min(jb + P.jc, P.y1);
-    cls = 0;
-  }
-  tb2d_any<T, ORDER, NT, EN>(kernarg<TB2D<T>>(), cls, ts, jb, je, delay[wv], P.ahead, item);
+  const Tb2dItem it = tb2d_item_at(P, n, item);
+  tb2d_any<T, ORDER, NT, EN>(kernarg<TB2D<T>>(), it.cls, it.ts, it.jb, it.je, delay[wv], P.ahead,
+                           item);
 }
 
 // Energy of the levels of some launches: level b = blockIdx.x, step

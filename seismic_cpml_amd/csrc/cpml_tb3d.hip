@@ -32,10 +32,9 @@
 // and the predicates of those axes.  All are one kernel, the classes with the
 // most of them first: a launch per class on streams of their own cost 20 us per
 // launch and 768^3 12.5 ms against 12.3.
-#include <algorithm>
-
 #include "cpml_device.h"
 #include "cpml_internal.h"
+#include "cpml_tb_geom.h"
 
 namespace cpml {
 namespace {
@@ -50,50 +49,6 @@ __device__ __forceinline__ T pml(bool slab, bool k1, T d, T old, T &out, T a, T 
   out = b * old + a * d;
   if (!k1) d = over_k(d, *K);
   return d + out;
-}
-
-struct Tile {
-  int i0, j0, kb, ke, tx, ty;
-};
-
-// Index of the u-th tile of one axis' class: the clean tiles [c0, c1) when
-// S is false, else the tiles outside them (below c0, then from c1).
-template <bool S>
-__device__ __forceinline__ int axis_tile(int u, int c0, int c1) {
-  if (!S) return c0 + u;
-  return u < c0 ? u : c1 + (u - c0);
-}
-template <bool S>
-__device__ __forceinline__ int axis_count(int n, int c0, int c1) {
-  return S ? n - (c1 - c0) : c1 - c0;
-}
-
-// Tile t of class (SX, SY, SZ).  Along each axis the tiles (z: chunks) whose
-// points and ring avoid that axis' slabs form a range [cl[2a], cl[2a+1]); the
-// class covers the product of the clean (flag false) or slab (flag true) tiles
-// of each axis, x fastest, then y, then z.
-template <bool SX, bool SY, bool SZ, typename P>
-__device__ __forceinline__ Tile tb_tile(const P &Q, int t, int nx, int ny, int nz, int kchunk) {
-  const int ntx = (nx + Q.ow - 1) / Q.ow, nty = (ny + Q.ty - 1) / Q.ty;
-  const int cx = axis_count<SX>(ntx, Q.box[0], Q.box[1]);
-  const int cy = axis_count<SY>(nty, Q.box[2], Q.box[3]);
-  Tile f;
-  f.tx = axis_tile<SX>(t % cx, Q.box[0], Q.box[1]);
-  f.ty = axis_tile<SY>((t / cx) % cy, Q.box[2], Q.box[3]);
-  const int tz = axis_tile<SZ>(t / (cx * cy), Q.zn[0], Q.zn[0] + Q.zn[1]);
-  f.i0 = f.tx * Q.ow;
-  f.j0 = f.ty * Q.ty;
-  if (tz < Q.zn[0]) {
-    f.kb = tz * kchunk;
-    f.ke = min(f.kb + kchunk, Q.z0);
-  } else if (tz < Q.zn[0] + Q.zn[1]) {
-    f.kb = Q.z0 + (tz - Q.zn[0]) * kchunk;
-    f.ke = min(f.kb + kchunk, Q.z1);
-  } else {
-    f.kb = Q.z1 + (tz - Q.zn[0] - Q.zn[1]) * kchunk;
-    f.ke = min(f.kb + kchunk, nz);
-  }
-  return f;
 }
 
 // Plane slot of a 3-plane window in the iteration of phase PH (the march is
@@ -153,7 +108,7 @@ __device__ __forceinline__ void tb3d_tile(const TB3D<T> &P, int t, T *xl) {
   constexpr int NS = 6 * NT;                   // LDS slots per buffer
   const Step3D<T> &p = P.a;
   const int nx = p.nx, ny = p.ny, nz = p.nz;
-  const Tile ft = tb_tile<SX, SY, SZ>(P, t, nx, ny, nz, p.kchunk);
+  const Tb3dTile ft = tb3d_tile_at<SX, SY, SZ>(P, t, nx, ny, nz, p.kchunk);
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = ft.i0 - NT + lane, j = ft.j0 - NT + w;
@@ -167,18 +122,10 @@ __device__ __forceinline__ void tb3d_tile(const TB3D<T> &P, int t, T *xl) {
   auto zlo = [&](int k) { return !SZ || (k >= 1 && k < nz); };
   auto zhi = [&](int k) { return !SZ || (k >= 0 && k <= nz - 2); };
 
-  // Offsets from the ghost corner (-1, -1, kl) of each array: clamped
-  // coordinates read a zero ghost point.
   const int s0 = kb - (2 * NT - 1), s1 = ke - 1 + (2 * NT - 1);
-  const int kl = max(s0 - 1, -1);
-  const int ic = min(max(i, -1), nx), jc = min(max(j, -1), ny);
-  const unsigned vo = (unsigned)(((long)(jc + 1) * p.ld + (ic + 1)) * (long)sizeof(T));
-  const unsigned psb = (unsigned)(p.ps * (long)sizeof(T));
-  const long corner = (long)kl * p.ps - p.ld - 1;
-  auto pl = [&](int k) -> unsigned {
-    const int kk = SZ ? min(max(k, -1), nz) : k;
-    return (unsigned)(kk - kl) * psb + vo;
-  };
+  const Tb3dLane<T, SX, SY, SZ> L(i, j, s0 - 1, p);
+  const long corner = L.corner;
+  auto pl = [&](int k) { return L.at(k); };
   const T *const ivx = p.vx + corner, *const ivy = p.vy + corner, *const ivz = p.vz + corner;
   const T *const ixx = p.sxx + corner, *const iyy = p.syy + corner, *const izz = p.szz + corner;
   const T *const ixy = p.sxy + corner, *const ixz = p.sxz + corner, *const iyz = p.syz + corner;
@@ -187,18 +134,14 @@ __device__ __forceinline__ void tb3d_tile(const TB3D<T> &P, int t, T *xl) {
   auto args = [&]() -> KArgs { return kernarg<TB3D<T>>(); };
 
   // x/y slab membership and profiles (loop invariant)
-  const bool inx = SX && p.sx.in(i), iny = SY && p.sy.in(j);
+  const bool inx = L.inx, iny = L.iny;
   T X[4] = {T(0), T(0), T(0), T(0)}, Y[4] = {T(0), T(0), T(0), T(0)};  // a, b, a_half, b_half
   if (SX && inx) X[0] = p.px.a[i], X[1] = p.px.b[i], X[2] = p.px.ah[i], X[3] = p.px.bh[i];
   if (SY && iny) Y[0] = p.py.a[j], Y[1] = p.py.b[j], Y[2] = p.py.ah[j], Y[3] = p.py.bh[j];
   const bool kx1 = p.sx.k1, ky1 = p.sy.k1, kz1 = p.sz.k1;
-  // byte offsets inside one plane of the memory variables
-  constexpr unsigned es = sizeof(T);
-  const unsigned mxo = inx ? (unsigned)p.sx.at(i, jc, ny) * es : 0u;
-  const unsigned myo = iny ? ((unsigned)ic + (unsigned)p.mld * (unsigned)p.sy.s(j)) * es : 0u;
-  const unsigned mzo = ((unsigned)ic + (unsigned)p.mld * (unsigned)jc) * es;
+  const unsigned mxo = L.mxo, myo = L.myo, mzo = L.mzo;
   const bool mx_on = SX && inx && row_in, my_on = SY && iny && col_in, mz_on = col_in && row_in;
-  const long mxs = (long)p.sx.w * ny, mys = p.mld * p.sy.w, mzs = p.mld * ny;
+  const long mxs = L.mxs, mys = L.mys, mzs = L.mzs;
 
   // ---- column windows by plane (slot_of)
   T V[NT][3][3];    // v^m (m = 0..NT-1): vx vy vz
@@ -603,52 +546,11 @@ __global__ __launch_bounds__(64 * NW) void k_tb3d(TB3D<T> P) {
   }
 }
 
-// Tiles along one axis (size B, extent n, slab widths wl, wr) whose points and
-// ring of g avoid both slabs: [t0, t1), empty when t1 <= t0.
-void clean_tiles(int n, int B, int g, int wl, int wr, int &t0, int &t1) {
-  const int nt = (n + B - 1) / B;
-  t0 = t1 = 0;
-  bool seen = false;
-  for (int t = 0; t < nt; ++t) {
-    const int lo = t * B - g, hi = t * B + B - 1 + g;
-    const bool clean = lo >= wl && hi < n - wr;
-    if (clean && !seen) t0 = t, seen = true;
-    if (clean) t1 = t + 1;
-    else if (seen) break;
-  }
-}
-
 template <typename T, int NT, int NW>
 hipError_t tb3d_launch(const TB3D<T> &P0, hipStream_t s) {
   TB3D<T> P = P0;
-  const Step3D<T> &p = P.a;
-  P.ty = NW - 2 * NT;
   if (P.ow < 1 || P.ow > 64 - 2 * NT) return hipErrorInvalidValue;
-  // z regions: planes whose march (2NT - 1 planes of ring) avoids the z slabs
-  // and the first and last plane
-  const int g = 2 * NT - 1, nz = p.nz, kc = p.kchunk;
-  int z0 = std::max(p.sz.wl, 1) + g;
-  int z1 = nz - std::max(p.sz.wr, 1) - g;
-  if (z1 <= z0) z0 = z1 = 0;
-  P.z0 = z0;
-  P.z1 = z1;
-  P.zn[0] = (z0 + kc - 1) / kc;
-  P.zn[1] = (z1 - z0 + kc - 1) / kc;
-  P.zn[2] = (nz - z1 + kc - 1) / kc;
-  clean_tiles(p.nx, P.ow, NT, std::max(p.sx.wl, 1), std::max(p.sx.wr, 1), P.box[0], P.box[1]);
-  clean_tiles(p.ny, P.ty, NT, std::max(p.sy.wl, 1), std::max(p.sy.wr, 1), P.box[2], P.box[3]);
-  if (P.box[1] < P.box[0]) P.box[0] = P.box[1] = 0;
-  if (P.box[3] < P.box[2]) P.box[2] = P.box[3] = 0;
-  const int n[3] = {(p.nx + P.ow - 1) / P.ow, (p.ny + P.ty - 1) / P.ty,
-                    P.zn[0] + P.zn[1] + P.zn[2]};
-  long most = 0;  // tiles of the XCD that gets most
-  for (int c = 0; c < 8; ++c) {
-    const int cx = c & 1 ? n[0] - (P.box[1] - P.box[0]) : P.box[1] - P.box[0];
-    const int cy = c & 2 ? n[1] - (P.box[3] - P.box[2]) : P.box[3] - P.box[2];
-    const int cz = c & 4 ? n[2] - P.zn[1] : P.zn[1];
-    P.ncls[c] = cx * cy * cz;
-    most += (P.ncls[c] + 7) / 8;
-  }
+  const long most = tb3d_split(NT, NW, P);
   hipLaunchKernelGGL((k_tb3d<T, NT, NW>), dim3((unsigned)(8 * most)), dim3(64 * NW), 0, s, P);
   return hipGetLastError();
 }
