@@ -30,50 +30,13 @@
 // per side (the second one's stencil), and a small launch the second.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
+#include "cpml_ade8_split.h"
 #include "cpml_constdiv.h"
 #include "cpml_device.h"
 #include "cpml_internal.h"
 
 namespace cpml {
 namespace {
-
-// rows per 64-column block; measured at 4096^2 (float, full step): 1 row
-// 8.84, 2 rows 9.00, 4 rows 8.91, 8 rows 8.32, 16 rows 8.13 Gcell/s
-constexpr int ATY = 2;
-
-// Points [x0, x1) x [y0, y1) of the grid.
-struct Box {
-  int x0, x1, y0, y1;
-  __host__ __device__ bool in(int i, int j) const {
-    return i >= x0 && i < x1 && j >= y0 && j < y1;
-  }
-};
-// The same with `by` fewer points on each side (none if it is empty).
-inline __host__ __device__ Box shrink(Box b, int by) {
-  return b.x1 > b.x0 ? Box{b.x0 + by, b.x1 - by, b.y0 + by, b.y1 - by} : b;
-}
-
-// Tiles of 64 x ATY points over the grid but for a box: below it, above it (whole
-// rows), left and right of it.  An empty box leaves the whole grid.
-struct FrameTiles {
-  Box below, above, left, right;
-  static __host__ __device__ int count(Box b) {
-    return (b.x1 - b.x0 + BX - 1) / BX * ((b.y1 - b.y0 + ATY - 1) / ATY);
-  }
-  __host__ __device__ FrameTiles(int nx, int ny, Box b) {
-    const bool none = b.x1 <= b.x0;
-    if (none) b = Box{0, nx, 0, 0};
-    below = Box{0, nx, 0, b.y0};
-    above = Box{0, nx, b.y1, ny};
-    left = Box{0, b.x0, b.y0, b.y1};
-    right = Box{b.x1, nx, b.y0, b.y1};
-  }
-  __host__ __device__ int tiles() const {
-    return count(below) + count(above) + count(left) + count(right);
-  }
-};
 
 // Tile h of nt in XCD-aware order: the hardware hands workgroup h to XCD h % 8;
 // each XCD gets one contiguous band of tiles (x fastest), so the halo columns and
@@ -83,27 +46,22 @@ __device__ __forceinline__ int xcd_tile(int h, int nt) {
   return xcd * q + min(xcd, r) + loc;
 }
 // Point of this thread in tile t of a box: false outside.
-__device__ __forceinline__ bool tile_point(Box b, int t, int &i, int &j) {
-  const int ntx = (b.x1 - b.x0 + BX - 1) / BX;
-  i = b.x0 + (t % ntx) * BX + threadIdx.x;
+__device__ __forceinline__ bool tile_point(AdeBox b, int t, int &i, int &j) {
+  const int ntx = (b.x1 - b.x0 + AdeFrame::TX - 1) / AdeFrame::TX;
+  i = b.x0 + (t % ntx) * AdeFrame::TX + threadIdx.x;
   j = b.y0 + (t / ntx) * ATY + threadIdx.y;
   return i < b.x1 && j < b.y1;
 }
-__device__ __forceinline__ bool frame_point(const FrameTiles &f, int h, int &i, int &j) {
-  const int n0 = f.count(f.below), n1 = n0 + f.count(f.left), n2 = n1 + f.count(f.right);
-  const int t = xcd_tile(h, f.tiles());
-  const Box b = t < n0 ? f.below : t < n1 ? f.left : t < n2 ? f.right : f.above;
-  return tile_point(b, t - (t < n0 ? 0 : t < n1 ? n0 : t < n2 ? n1 : n2), i, j);
+__device__ __forceinline__ bool frame_point(const AdeFrame &f, int h, int &i, int &j) {
+  int t = xcd_tile(h, f.tiles());
+  const AdeBox b = f.part(t);
+  return tile_point(b, t, i, j);
 }
 
 // (c1 d1 + c2 d2 + c3 d3 + c4 d4) / delta, ADE8:263-266, 720-723
 template <typename T>
 __device__ __forceinline__ T h8(T d1, T d2, T d3, T d4, T del) {
   return (((T(kHolberg1) * d1 + T(kHolberg2) * d2) + T(kHolberg3) * d3) + T(kHolberg4) * d4) / del;
-}
-
-__device__ __forceinline__ bool band(int I, int J, int nx, int ny, int npml) {  // Fortran indices
-  return I <= npml + 2 || I >= nx - npml - 2 || J <= npml + 2 || J >= ny - npml - 2;
 }
 
 template <typename T>
@@ -136,7 +94,7 @@ __device__ __forceinline__ void ade_point(const Ade8<T> &a, int inc, int in, int
   const Step2D<T> &p = a.s;
   const long ld = p.ld, c = i + j * ld;
   const int nx = p.nx, ny = p.ny, I = i + 1, J = j + 1;
-  const bool bd = band(I, J, nx, ny, a.npml);
+  const bool bd = ade_band(I, J, nx, ny, a.npml);
   const bool edge = i == 0 || i == nx - 1 || j == 0 || j == ny - 1;
   const T *const X0[5] = {p.vx, p.vy, p.sxx, p.syy, p.sxy};
   const T *const *st = inc == 0 ? X0 : a.d[in];
@@ -246,24 +204,21 @@ __device__ __forceinline__ void ade_point(const Ade8<T> &a, int inc, int in, int
 
 // Stage inc on the grid but for `skip`; X is accumulated outside `box`.
 template <typename T>
-__device__ __forceinline__ void ade_frame(const Ade8<T> &a, int inc, Box box, Box skip, int h) {
+__device__ __forceinline__ void ade_frame(const Ade8<T> &a, int inc, AdeBox box, AdeBox skip, int h) {
   int i, j;
-  if (frame_point(FrameTiles(a.s.nx, a.s.ny, skip), h, i, j))
+  if (frame_point(AdeFrame(a.s.nx, a.s.ny, skip), h, i, j))
     ade_point(a, inc, inc & 1, (inc & 1) ^ 1, i, j, !box.in(i, j));
 }
 template <typename T, bool WHOLE>
-__global__ __launch_bounds__(BX *ATY) void k_ade_stage(Ade8<T> a, int inc, Box box) {
+__global__ __launch_bounds__(BX *ATY) void k_ade_stage(Ade8<T> a, int inc, AdeBox box) {
   if (!WHOLE) {
     ade_frame(a, inc, box, box, blockIdx.x);
     return;
   }
   int i, j;
-  if (tile_point(Box{0, a.s.nx, 0, a.s.ny}, xcd_tile(blockIdx.x, gridDim.x), i, j))
+  if (tile_point(AdeBox{0, a.s.nx, 0, a.s.ny}, xcd_tile(blockIdx.x, gridDim.x), i, j))
     ade_point(a, inc, inc & 1, (inc & 1) ^ 1, i, j, true);
 }
-
-constexpr int PG = 8;    // ring columns of a pair's strip (4 per stage)
-constexpr int PW = 48;   // columns it owns
 
 // Media of one row of a strip: values at the points and at their neighbours.
 template <typename T>
@@ -329,13 +284,13 @@ __device__ __forceinline__ void ade_rates(const Step2D<T> &p, const AdeMedia<T> 
 // of the box.  Iteration p takes row p of the first stage and row p - 4 of the
 // second.
 template <typename T, bool FIRST>
-__device__ __forceinline__ void ade_pair(const Ade8<T> &a, Box box, int c0, int jb, int je,
+__device__ __forceinline__ void ade_pair(const Ade8<T> &a, AdeBox box, int c0, int jb, int je,
                                          T (*delay)[4][BX]) {
   const Step2D<T> &p = a.s;
   const long ld = p.ld;
   const int lane = threadIdx.x, i = c0 - PG + lane;
   const bool own = lane >= PG && lane < PG + PW && i < box.x1;
-  const unsigned o = (unsigned)(min(i, p.nx - 1) * (int)sizeof(T));
+  const unsigned o = ade_pair_offset<T>(i, p.nx);
   constexpr int inc = FIRST ? 0 : 2;
   const T r1 = rk42<T>(inc), r2 = rk42<T>(inc + 1);
   const T n1 = rk41<T>(inc + 1), n2 = FIRST ? rk41<T>(inc + 2) : T(0);
@@ -434,64 +389,41 @@ __device__ __forceinline__ void ade_pair(const Ade8<T> &a, Box box, int c0, int 
 
 // The pair's items (one wavefront each), then the frame's first stage.
 template <typename T, bool FIRST>
-__global__ __launch_bounds__(BX *ATY) void k_ade_pair(Ade8<T> a, Box box, int jc, int nblocks) {
+__global__ __launch_bounds__(BX *ATY) void k_ade_pair(Ade8<T> a, AdePairs pairs, int nblocks) {
   __shared__ T delay[ATY][FIRST ? 7 : 6][4][BX];
   const int h = blockIdx.x;
   if (h >= nblocks) {
-    ade_frame(a, FIRST ? 0 : 2, box, shrink(box, 4), h - nblocks);
+    ade_frame(a, FIRST ? 0 : 2, pairs.box, shrink(pairs.box, 4), h - nblocks);
     return;
   }
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
-  const int ns = (box.x1 - box.x0 + PW - 1) / PW, nc = (box.y1 - box.y0 + jc - 1) / jc;
   // each XCD gets one contiguous band of items (strips fastest)
   const int t = xcd_tile(h, nblocks) * ATY + w;
-  if (t >= ns * nc) return;
-  const int jb = box.y0 + t / ns * jc;
-  ade_pair<T, FIRST>(a, box, box.x0 + t % ns * PW, jb, min(jb + jc, box.y1), delay[w]);
-}
-
-// The points whose two stages see neither band nor edges: the first stage's
-// points (4 around them) lie outside the band, its stencil (8 around) off the
-// edges; whole 64-byte sectors from the left.  Empty for grids whose step a
-// march's length sets: 500 x 600 float 57 us with single stages, 96 with pairs,
-// 1000 x 1200 135 and 127, 4096^2 1847 and 907; double 500 x 600 97 and 115, 1000 x
-// 900 203 and 171, 2800^2 1960 and 943.
-template <typename T>
-Box pair_box(const Ade8<T> &a) {
-  const int lo = std::max(a.npml + 6, 9), sector = 64 / (int)sizeof(T);
-  Box b{(lo + sector - 1) / sector * sector, std::min(a.s.nx - a.npml - 7, a.s.nx - 9), lo,
-        std::min(a.s.ny - a.npml - 7, a.s.ny - 9)};
-  if (b.x1 - b.x0 < 64 || b.y1 - b.y0 < 64 ||
-      (double)(b.x1 - b.x0) * (b.y1 - b.y0) * sizeof(T) < 4e6)
-    return Box{0, 0, 0, 0};
-  return b;
+  if (t >= pairs.count()) return;
+  int c0, jb, je;
+  pairs.item(t, c0, jb, je);
+  ade_pair<T, FIRST>(a, pairs.box, c0, jb, je, delay[w]);
 }
 
 }  // namespace
 
 template <typename T>
 hipError_t launch_ade8_step(const Ade8<T> &a, hipStream_t s) {
-  const Box box = pair_box(a);
+  const AdeBox box = ade_pair_box<T>(a.s.nx, a.s.ny, a.npml);
   const dim3 block(BX, ATY);
-  const int frame = FrameTiles(a.s.nx, a.s.ny, box).tiles();
+  const int frame = AdeFrame(a.s.nx, a.s.ny, box).tiles();
   if (box.x1 == 0) {
     // stage 1 reads X0; the states of stages 2..4 alternate between d[1] and d[0]
     for (int inc = 0; inc < 4; ++inc)
       hipLaunchKernelGGL((k_ade_stage<T, true>), dim3(frame), block, 0, s, a, inc, box);
     return hipGetLastError();
   }
-  // rows of an item: as many items as fit in flight, 16 (its 16 ring rows cost as
-  // much) to 64 (4096^2 float 16, 32, 64 and 128 rows 1013, 951, 923 and 942 us per
-  // step; 2000 x 2400 365, 341, 350 and 570; 1000 x 900 double 203, 182, 292, 521)
-  const int strips = (box.x1 - box.x0 + PW - 1) / PW;
-  const int jc = std::clamp(
-      (int)((double)strips * (box.y1 - box.y0) / (sizeof(T) == 4 ? 3000 : 600)), 16, 64);
-  const int items = strips * ((box.y1 - box.y0 + jc - 1) / jc);
-  const int nblocks = (items + ATY - 1) / ATY;
-  const int first = FrameTiles(a.s.nx, a.s.ny, shrink(box, 4)).tiles();
-  hipLaunchKernelGGL((k_ade_pair<T, true>), dim3(nblocks + first), block, 0, s, a, box, jc, nblocks);
+  const AdePairs pairs = ade_pairs<T>(box);
+  const int nblocks = (pairs.count() + ATY - 1) / ATY;
+  const int first = AdeFrame(a.s.nx, a.s.ny, shrink(box, 4)).tiles();
+  hipLaunchKernelGGL((k_ade_pair<T, true>), dim3(nblocks + first), block, 0, s, a, pairs, nblocks);
   hipLaunchKernelGGL((k_ade_stage<T, false>), dim3(frame), block, 0, s, a, 1, box);
-  hipLaunchKernelGGL((k_ade_pair<T, false>), dim3(nblocks + first), block, 0, s, a, box, jc, nblocks);
+  hipLaunchKernelGGL((k_ade_pair<T, false>), dim3(nblocks + first), block, 0, s, a, pairs, nblocks);
   hipLaunchKernelGGL((k_ade_stage<T, false>), dim3(frame), block, 0, s, a, 3, box);
   return hipGetLastError();
 }

@@ -1,9 +1,14 @@
-// Addresses of the time-blocked marches (cpml_tb_geom.h: the kernels' own code)
-// over random grids, slabs, strips and chunks, every item and every lane:
+// Addresses of the marches that read through plain pointers, over random grids,
+// slabs, strips and chunks, every item and every lane: time-blocked 2D and 3D
+// (cpml_tb_geom.h) and the ADE-RK4 pairs of stages (cpml_ade8_split.h), the code that
+// the kernels compile themselves:
 //   * each point of the grid is stored by exactly one lane, at its own address;
 //   * each field load lies in its padded array, without a wrap of the 32-bit offset;
 //   * each load and store of a memory variable lies in its array (they are made
-//     where the kernels' predicates say so), along y and z inside its row.
+//     where the kernels' predicates say so), along y and z inside its row;
+//   * Slab::at numbers an x slab's points without gaps;
+//   * a pair's points and the first stage's points around them lie outside the band
+//     and off the edges.
 // usage: address_audit grids [ghost]   (ghost: the columns of the y and z memory
 // variables clamped like the fields', to the ghost column nx: must be found)
 // Prints the number of addresses checked; exit code 1 if one is out of bounds.
@@ -15,6 +20,7 @@
 #include <string>
 #include <vector>
 
+#include "../../seismic_cpml_amd/csrc/cpml_ade8_split.h"
 #include "../../seismic_cpml_amd/csrc/cpml_tb_geom.h"
 
 using namespace cpml;
@@ -197,6 +203,74 @@ static void grid3() {
   once(owned);
 }
 
+// x-slab arrays: every point of the slab has its own element of [0, w * rows).
+static void slab_layout() {
+  const Slab s = slab(pick(2, 90));
+  const int rows = pick(1, 50);
+  std::vector<int> hit((size_t)s.w * rows);
+  for (int i = 0; i < s.n; ++i)
+    for (int j = 0; j < rows && s.in(i); ++j) {
+      const long q = s.at(i, j, rows);
+      expect(q >= 0 && q < (long)hit.size(), "slab layout", i, j, rows);
+      if (q >= 0 && q < (long)hit.size()) ++hit[q];
+    }
+  once(hit);
+}
+
+// Points of the frame's tiles, each counted in `owned`.
+static void frame(const AdeFrame &f, int nx, std::vector<int> &owned) {
+  for (int h = 0; h < f.tiles(); ++h) {
+    int t = h;
+    const AdeBox b = f.part(t);
+    const int ntx = (b.x1 - b.x0 + AdeFrame::TX - 1) / AdeFrame::TX;
+    for (int y = 0; y < ATY; ++y)
+      for (int x = 0; x < AdeFrame::TX; ++x) {
+        const int i = b.x0 + (t % ntx) * AdeFrame::TX + x, j = b.y0 + (t / ntx) * ATY + y;
+        if (i < b.x1 && j < b.y1) ++owned[i + (size_t)nx * j];
+      }
+  }
+}
+
+template <typename T>
+static void ade() {
+  const int npml = pick(0, 30), nx = extent(1100, 1500), ny = pick(1000, 1400);
+  const long align = 256 / sizeof(T), ld = round_up(align + nx + 4, align);
+  const long base = align + 4 * ld, total = ld * (ny + 8);
+  const AdeBox box = ade_pair_box<T>(nx, ny, npml);
+  std::vector<int> owned((size_t)nx * ny), first((size_t)nx * ny);
+  frame(AdeFrame(nx, ny, box), nx, owned);
+  if (box.x1 > 0) {
+    const AdePairs pairs = ade_pairs<T>(box);
+    for (int t = 0; t < pairs.count(); ++t) {
+      int c0, jb, je;
+      pairs.item(t, c0, jb, je);
+      expect(jb - 8 >= 1 && je + 7 <= ny - 2, "pair rows", jb, je, npml);
+      for (int lane = 0; lane < 64; ++lane) {
+        const int i = c0 - PG + lane;
+        const long o = ade_pair_offset<T>(i, nx) / sizeof(T);
+        for (int j : {jb - 8, je + 7})
+          expect(o < nx && base + j * ld + o >= 0 && base + j * ld + o < total, "pair load", i, j, npml);
+        if (lane < PG || lane >= PG + PW || i >= box.x1) continue;
+        expect(i - 8 >= 1 && i + 8 <= nx - 2, "pair columns", i, c0, npml);
+        for (int j = jb; j < je; ++j) {
+          ++owned[i + (size_t)nx * j];
+          if (j > box.y0 && j < box.y1 - 1 && i > box.x0 && i < box.x1 - 1) continue;
+          for (int di : {-4, 4})
+            for (int dj : {-4, 4})
+              expect(!ade_band(i + di + 1, j + dj + 1, nx, ny, npml), "pair in the band", i, j, npml);
+        }
+      }
+    }
+    // the first stage of the frame: all but the box less 4 points on each side
+    const AdeBox in = shrink(box, 4);
+    frame(AdeFrame(nx, ny, in), nx, first);
+    for (int j = 0; j < ny; ++j)
+      for (int i = 0; i < nx; ++i)
+        expect(first[i + (size_t)nx * j] == (in.in(i, j) ? 0 : 1), "first stage", i, j, npml);
+  }
+  once(owned);
+}
+
 int main(int argc, char **argv) {
   const int grids = argc > 1 ? std::atoi(argv[1]) : 40;
   ghost = argc > 2 && std::strcmp(argv[2], "ghost") == 0;
@@ -207,6 +281,8 @@ int main(int argc, char **argv) {
     grid3<float, 2>();
     grid3<double, 1>();
     grid3<double, 2>();
+    slab_layout();
+    if (g % 20 == 0) ade<float>(), ade<double>();
   }
   std::printf("%ld addresses checked, %ld out of bounds\n", checked, bad);
   return bad ? 1 : 0;

@@ -1,7 +1,8 @@
-"""Items and addresses of the time-blocked marches (cpml_tb_geom.h, the code that
-the kernels compile) on the CPU, over random grids, slabs, strip widths and chunk
-depths: what is loaded and stored lies inside its array, and each point of the
-grid is stored once.  The memory variables have no ghost points: with the
+"""Items and addresses of the marches without a hardware range check -- time-blocked
+2D, batch and 3D (cpml_tb_geom.h) and the ADE-RK4 pairs (cpml_ade8_split.h) -- on the
+CPU, through the code that the kernels compile, over random grids, slabs, strip
+widths and chunk depths: what is loaded and stored lies inside its array, and
+each point of the grid is stored once.  The memory variables have no ghost points: with the
 fields' clamp (to the ghost column nx) narrow strips read past their rows, and
 the audit has to say so."""
 import subprocess
