@@ -71,10 +71,20 @@ __device__ __forceinline__ void tile_energy(const EnergyFold<T> &ef, int tile, d
   }
 }
 
+// Waves per SIMD the 2D kernels are built for: all that the vector registers leave
+// room for.  Without the bound they take more than 80 scalar registers, and the
+// SIMD holds 7 waves instead of 8 and half as many blocks of 16: at 2900^2 float
+// in 64-row tiles 190 us per step and 149 with it, with the energy curve 217 and 169 (16
+// rows 225 and 183); double 280 and 260.
+template <typename T, int ORDER>
+constexpr int min_waves2d() {
+  return sizeof(T) == 4 || ORDER < 8 ? 8 : 1;
+}
+
 // A tile is 64 points by TY*RG rows; the block (64 x TY threads) walks its RG
 // row groups, so each wavefront lives for several rows.
 template <typename T, int ORDER, int TY, int RG, bool NT>
-__global__ __launch_bounds__(BX *TY) void k_stress2d(Step2D<T> p, Record<T> prev, int lead) {
+__global__ __launch_bounds__(BX *TY, (min_waves2d<T, ORDER>())) void k_stress2d(Step2D<T> p, Record<T> prev, int lead) {
   int h, i, j;
   if (lead_block(prev, lead, h)) return;
   tile2d<TY, RG>(h, p.nx, p.ny, i, j);
@@ -83,23 +93,25 @@ __global__ __launch_bounds__(BX *TY) void k_stress2d(Step2D<T> p, Record<T> prev
     if (i < p.nx && j + r * TY < p.ny) stress2d_point<T, ORDER, NT>(p, i, j + r * TY);
 }
 
-template <typename T, int ORDER, int TY, int RG, bool NT>
-__global__ __launch_bounds__(BX *TY) void k_velocity2d(Step2D<T> p, EnergyFold<T> ef) {
+// EN: the energy of the points it computes, summed over the tile.  Steps without it
+// have a kernel without its registers: 4096^2 float 137 -> 125 us.
+template <typename T, int ORDER, int TY, int RG, bool NT, bool EN>
+__global__ __launch_bounds__(BX *TY, (min_waves2d<T, ORDER>())) void k_velocity2d(Step2D<T> p, EnergyFold<T> ef) {
   int i, j;
   tile2d<TY, RG>(blockIdx.x, p.nx, p.ny, i, j);
-  const bool en = ef.partial && *p.step % ef.cadence == 0;
+  const bool en = EN && *p.step % ef.cadence == 0;
   double kin = 0.0, pot = 0.0;
 #pragma unroll
   for (int r = 0; r < RG; ++r)
     if (i < p.nx && j + r * TY < p.ny) {
       const int jr = j + r * TY;
       velocity2d_point<T, ORDER, NT>(p, i, jr, [&](T vx, T vy, long c) {
-        if (en && i >= ef.i0 && i <= ef.i1 && jr >= ef.j0 && jr <= ef.j1)
+        if (EN && en && i >= ef.i0 && i <= ef.i1 && jr >= ef.j0 && jr <= ef.j1)
           point_energy2d(vx, vy, p.sxx[c], p.syy[c], p.sxy[c], p.lam[c], p.mu[c], p.rho[c], kin,
                          pot);
       });
     }
-  if (en) tile_energy<TY>(ef, blockIdx.x, kin, pot);
+  if (EN && en) tile_energy<TY>(ef, blockIdx.x, kin, pot);
 }
 
 // ---------------------------------------------------------------- 3D ----
@@ -585,21 +597,24 @@ static hipError_t stress2d_ty(int order, const Step2D<T> &p, const Record<T> *pr
                      : stress2d_nt<T, TY, RG, false>(order, p, prev, s);
 }
 
-template <typename T, int TY, int RG, bool NT>
+template <typename T, int TY, int RG, bool NT, bool EN>
 static hipError_t velocity2d_nt(int order, const Step2D<T> &p, const EnergyFold<T> &ef,
                                 hipStream_t s) {
   dim3 grid(((p.nx + BX - 1) / BX) * ((p.ny + TY * RG - 1) / (TY * RG))), block(BX, TY);
-  if (order == 2) hipLaunchKernelGGL((k_velocity2d<T, 2, TY, RG, NT>), grid, block, 0, s, p, ef);
-  else if (order == 4) hipLaunchKernelGGL((k_velocity2d<T, 4, TY, RG, NT>), grid, block, 0, s, p, ef);
-  else hipLaunchKernelGGL((k_velocity2d<T, 8, TY, RG, NT>), grid, block, 0, s, p, ef);
+  if (order == 2) hipLaunchKernelGGL((k_velocity2d<T, 2, TY, RG, NT, EN>), grid, block, 0, s, p, ef);
+  else if (order == 4) hipLaunchKernelGGL((k_velocity2d<T, 4, TY, RG, NT, EN>), grid, block, 0, s, p, ef);
+  else hipLaunchKernelGGL((k_velocity2d<T, 8, TY, RG, NT, EN>), grid, block, 0, s, p, ef);
   return hipGetLastError();
 }
 
 template <typename T, int TY, int RG>
 static hipError_t velocity2d_ty(int order, const Step2D<T> &p, const EnergyFold<T> &ef,
-                              hipStream_t s) {
-  return p.streaming ? velocity2d_nt<T, TY, RG, true>(order, p, ef, s)
-                     : velocity2d_nt<T, TY, RG, false>(order, p, ef, s);
+                                hipStream_t s) {
+  if (ef.partial)
+    return p.streaming ? velocity2d_nt<T, TY, RG, true, true>(order, p, ef, s)
+                       : velocity2d_nt<T, TY, RG, false, true>(order, p, ef, s);
+  return p.streaming ? velocity2d_nt<T, TY, RG, true, false>(order, p, ef, s)
+                     : velocity2d_nt<T, TY, RG, false, false>(order, p, ef, s);
 }
 
 // p.tile_y: rows per tile, 4, 8, 16, or 32 / 64 walked by 16-row blocks
