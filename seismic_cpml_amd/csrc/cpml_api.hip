@@ -202,7 +202,7 @@ struct cpml_solver {
   // 2D viscoelastic attenuation (cpml_gpu_set_attenuation)
   int nsls = 0;                 // 0: elastic
   double tau[4][cpml::kMaxSls] = {};  // tau_epsilon_nu1, tau_sigma_nu1, _nu2, _nu2
-  void *re[3] = {};             // R_e1, R_e11, R_e13: nsls dense nx*ny planes each
+  void *re[3] = {};             // R_e1, R_e11, R_e13: nsls planes of ny rows of mld each
   // ADE-PML RK4 step of the 8th-order program (cpml_gpu_set_ade_rk4)
   bool ade = false;
   void *ade_d[10] = {};         // stage states [2][field], padded like the fields
@@ -499,7 +499,7 @@ cpml::Visco2D<T> visco2d(cpml_solver *h) {
   v.re1 = static_cast<T *>(h->re[0]);
   v.re11 = static_cast<T *>(h->re[1]);
   v.re13 = static_cast<T *>(h->re[2]);
-  v.nn = (long)h->nx * h->ny;
+  v.nn = h->mld * h->ny;
   v.nsls = h->nsls;
   const T dt = T(h->dt);
   T s1 = 0, s2 = 0;
@@ -2098,7 +2098,7 @@ int cpml_gpu_set_attenuation(cpml_solver *h, int N_SLS, const double *tau_epsilo
   h->nsls = N_SLS;
   for (int q = 0; q < 4; ++q)
     for (int l = 0; l < N_SLS; ++l) h->tau[q][l] = t[q][l];
-  const size_t bytes = (size_t)N_SLS * h->nx * h->ny * h->esize;
+  const size_t bytes = (size_t)N_SLS * h->mld * h->ny * h->esize;
   for (int k = 0; k < 3 && N_SLS > 0; ++k) {
     if ((rc = dev_alloc(h, &h->re[k], bytes))) return rc;
     HIPCHK(h, hipMemsetAsync(h->re[k], 0, bytes, h->stream));
@@ -2167,8 +2167,11 @@ int cpml_gpu_get_attenuation_memory(cpml_solver *h, int which, void *out) {
   if (which < 0 || which > 2) return fail(h, CPML_ERR_ARG, "which must be 0, 1 or 2");
   int rc = set_device(h);
   if (rc) return rc;
-  HIPCHK(h, hipMemcpy(out, h->re[which], (size_t)h->nsls * h->nx * h->ny * h->esize,
-                      hipMemcpyDeviceToHost));
+  const size_t rows = (size_t)h->nsls * h->ny, pitch = h->mld * h->esize, row = h->nx * h->esize;
+  std::vector<char> tmp(rows * pitch);
+  HIPCHK(h, hipMemcpy(tmp.data(), h->re[which], tmp.size(), hipMemcpyDeviceToHost));
+  for (size_t r = 0; r < rows; ++r)
+    std::memcpy(static_cast<char *>(out) + r * row, tmp.data() + r * pitch, row);
   return CPML_OK;
 }
 

@@ -366,13 +366,13 @@ template <typename T>
 hipError_t launch_ade8_step(const Ade8<T> &a, hipStream_t s);
 
 // 2D viscoelastic step: the 2D step plus the attenuation memory variables
-// (dense nx*ny per SLS plane) and their per-SLS coefficients.
+// (ny rows of mld per SLS plane) and their per-SLS coefficients.
 constexpr int kMaxSls = 8;
 template <typename T>
 struct Visco2D {
   Step2D<T> s;
   T *re1, *re11, *re13;
-  long nn;   // nx * ny
+  long nn;   // elements of an SLS plane: mld * ny
   int nsls;
   T P1[kMaxSls], P2[kMaxSls];  // DELTAT_phi_nu1, _nu2
   T H1[kMaxSls], H2[kMaxSls];  // HALF_DELTAT_over_tau_sigma_nu1, _nu2

@@ -19,9 +19,11 @@
 // only its own old value, so R is updated in place (the reference keeps an
 // _old copy of every array and copies it each step, 2D-visco2:736-738).
 //
-// One point per thread, 64 x 4 blocks; R is stored dense (nx * ny per SLS
-// plane) next to the padded wavefields.  Bound by HBM: 36 words per point and step
-// with three solids, 4096^2 float 489 us, 4.9 TB/s.
+// One point per thread, 64 x 4 blocks; R is stored in rows of whole cache lines
+// (mld) per SLS plane: its accesses stream past the caches, and parts of a line are
+// then merged nowhere (dense rows, 2900^2 double 547 us per step, 497 now; 4001^2 float
+// 549 and 487; 2001 x 2200 142 and 127).  Bound by HBM: 36 words per point and step with
+// three solids, 4096^2 float 489 us, 4.9 TB/s.
 #include <hip/hip_runtime.h>
 
 #include "cpml_device.h"
@@ -62,7 +64,7 @@ __global__ __launch_bounds__(BX *VTY) void k_stress2dve(Visco2D<T> v) {
   if (!point2(v, i, j)) return;
   const Step2D<T> &p = v.s;
   const long ld = p.ld, c = i + j * ld;
-  const long r = i + (long)j * p.nx;  // dense index of the memory variables
+  const long r = i + (long)j * p.mld;  // index of the memory variables
   // the kernel reads v and writes sigma and R: restrict lets the reads of a
   // point issue together instead of waiting behind its stores
   const T *__restrict__ vx = p.vx;
