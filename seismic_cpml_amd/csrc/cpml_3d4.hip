@@ -23,11 +23,13 @@
 // read from global memory and come from the same or adjacent rows of the
 // block, so they hit in L1/L2.  Profile values of the column are loaded once.
 //
-// Bound by HBM: 30 words per point and step at 3.3 TB/s (210 x 800 x 220, float),
-// a rate that the loads in flight set.  So the loads of the next plane, memory
-// variables included, go into a second register set before this plane's
-// arithmetic and stores, through buffers whose offsets the scalar unit adds:
-// 1536 -> 1382 us per step, double 3203 -> 2746, 256^3 float 627 -> 583.
+// Bound by HBM, at a rate that the wavefronts in flight set: 6 per SIMD in float
+// (79 registers), 3 in double (141).  A plane's loads, memory variables included,
+// are issued together through buffers whose offsets the scalar unit adds.
+// Loading the next plane ahead into a second register set leaves 4 and 2
+// wavefronts and is slower: float 210 x 800 x 220 1606 us per step and 1531 without,
+// 512^3 4353 and 4004, 768^3 13572 and 12794; double 512^3 9134 and 8773 (128^3 189 and
+// 196).
 #include <hip/hip_runtime.h>
 
 #include "cpml_constdiv.h"
@@ -76,8 +78,8 @@ struct Chunk4 {
   }
 };
 
-// C-PML of one axis on three derivatives of a point inside its slab, with the
-// memory variables m read a plane ahead: psi <- b*psi + a*d ; d <- d/K + psi
+// C-PML of one derivative of a point inside the axis' slab, with its memory
+// variable m read with the plane: psi <- b*psi + a*d ; d <- d/K + psi
 // where `in` (the update's loop range).
 template <typename T>
 __device__ __forceinline__ void pml4(bool in, T &d, T m, T *psi, T a, T b, T K) {
@@ -97,10 +99,8 @@ struct SPlane4 {
   T px[3], py[3], pz[3];  // memory variables, where the point lies in the axis' slab
 };
 
-// Float: at least 4 waves per SIMD (128 VGPRs against 132 unbounded, which
-// leave 3); more would spill.
 template <typename T, int TY4>
-__global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_stress3d4(Step3D<T> p,
+__global__ __launch_bounds__(BX *TY4) void k_stress3d4(Step3D<T> p,
     Record<T> prev, int lead) {
   int h;
   if (lead_block(prev, lead, h)) return;
@@ -174,14 +174,11 @@ __global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_stress3d4(S
   T vy_zm = g.ld(rvy, 0, 0, -1, k0), vy0 = g.ld(rvy, 0, 0, 0, k0), vy_zp = g.ld(rvy, 0, 0, 1, k0);
   T vz_zmm = g.ld(rvz, 0, 0, -2, k0), vz_zm = g.ld(rvz, 0, 0, -1, k0);
   T vz0 = g.ld(rvz, 0, 0, 0, k0);
-  // one plane: L holds its values, N receives the next one's.  The caller
-  // alternates two sets, so no copy waits for the loads in flight, and they are
-  // issued before this plane's stores, so waiting for them does not wait for
-  // those.
-  auto plane = [&](int k, const SPlane4<T> &L, SPlane4<T> &N) {
+  for (int k = c.kb; k < c.ke; ++k) {
     const auto Q = kernarg<Step3D<T>>();
     const int kk = k - c.kb + 2;
-    load(N, min(k + 1, c.ke - 1));
+    SPlane4<T> L;
+    load(L, k);
     const T mu = L.mu, lam = L.lam;
     const bool inz = p.sz.in(k);
     const bool r_k1 = k >= 1, r_kn = k <= nz - 2;
@@ -229,12 +226,6 @@ __global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_stress3d4(S
     vx_zm = vx0, vx0 = vx_zp, vx_zp = L.vx_zpp;
     vy_zm = vy0, vy0 = vy_zp, vy_zp = L.vy_zpp;
     vz_zmm = vz_zm, vz_zm = vz0, vz0 = L.vz_zp;
-  };
-  SPlane4<T> A, B;
-  load(A, c.kb);
-  for (int k = c.kb; k < c.ke; k += 2) {
-    plane(k, A, B);
-    if (k + 1 < c.ke) plane(k + 1, B, A);
   }
 }
 
@@ -248,7 +239,7 @@ struct VPlane4 {
 };
 
 template <typename T, int TY4>
-__global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_velocity3d4(Step3D<T> p) {
+__global__ __launch_bounds__(BX *TY4) void k_velocity3d4(Step3D<T> p) {
   const Tile3 c = tile3<TY4, kFlat4<T>>(p, blockIdx.x);
   if (!c.ok) return;
   const int i = c.i, j = c.j, nx = p.nx, ny = p.ny, nz = p.nz;
@@ -317,14 +308,11 @@ __global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_velocity3d4
   T syz0 = g.ld(ryz, 0, 0, 0, k0);
   T szz_zm = g.ld(rzz, 0, 0, -1, k0), szz0 = g.ld(rzz, 0, 0, 0, k0);
   T szz_zp = g.ld(rzz, 0, 0, 1, k0);
-  // one plane: L holds its values, N receives the next one's.  The caller
-  // alternates two sets, so no copy waits for the loads in flight, and they are
-  // issued before this plane's stores, so waiting for them does not wait for
-  // those.
-  auto plane = [&](int k, const VPlane4<T> &L, VPlane4<T> &N) {
+  for (int k = c.kb; k < c.ke; ++k) {
     const auto Q = kernarg<Step3D<T>>();
     const int kk = k - c.kb + 2;
-    load(N, min(k + 1, c.ke - 1));
+    VPlane4<T> L;
+    load(L, k);
     const T cb = L.cb;
     T vxn = L.vx, vyn = L.vy, vzn = L.vz;
     const bool inz = p.sz.in(k);
@@ -382,12 +370,6 @@ __global__ __launch_bounds__(BX *TY4, sizeof(T) == 4 ? 4 : 1) void k_velocity3d4
     sxz_zmm = sxz_zm, sxz_zm = sxz0, sxz0 = L.xz_zp;
     syz_zmm = syz_zm, syz_zm = syz0, syz0 = L.yz_zp;
     szz_zm = szz0, szz0 = szz_zp, szz_zp = L.zz_zpp;
-  };
-  VPlane4<T> A, B;
-  load(A, c.kb);
-  for (int k = c.kb; k < c.ke; k += 2) {
-    plane(k, A, B);
-    if (k + 1 < c.ke) plane(k + 1, B, A);
   }
 }
 
@@ -399,8 +381,8 @@ unsigned ntiles4(const Step3D<T> &p, int ty) {
 
 }  // namespace
 
-// p.tile_y selects the rows per block (4, 8 or 16; double: at most 8, whose two
-// planes of values fit in registers)
+// p.tile_y selects the rows per block (4, 8 or 16; double: at most 8, since the
+// 128 registers that blocks of 16 wavefronts leave would spill)
 template <typename T>
 hipError_t launch_stress3d4(const Step3D<T> &p, const Record<T> *prev, hipStream_t s) {
   const int lead = prev ? kLead : 0;

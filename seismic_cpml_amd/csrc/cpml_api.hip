@@ -239,20 +239,24 @@ bool chunk_fits(const cpml_solver *h, int kchunk) {
   } while (0)
 
 // Planes per block of the 3D two-phase and fused kernels.  Each block reads its
-// halo planes again, so deep chunks read less, but the machine wants about four
-// blocks per CU: 8 planes (order 4, whose halo is deeper, 32 where that leaves
-// four rounds of blocks: 210 x 800 x 220 float 1442 and 1382 us per step, 256^3
-// 583 with 8 and 605 with 16), halved for small grids (96 x 80 x 72 float 47 us
-// with 8 planes, 30 with 2; order 4, 100 x 90 x 80, 62 with 8, 47 with 4 and 50 with
-// 2; the fused kernel, which recomputes its halo planes, keeps 8), and less where a chunk's buffer would pass 4 GiB.
+// halo planes again, so deep chunks read less, but neighbouring tiles drift apart
+// in them and fetch the rows they share twice, and the machine wants rounds of blocks.
+// 8 planes (the fused kernel, which recomputes its halo planes, always); order 2:
+// halved to 2 while that leaves less than four blocks per CU (96 x 80 x 72 float 47 us
+// with 8 planes, 30 with 2); order 4, whose kernels hold 3 (double) to 6 blocks per CU:
+// 4 planes below 24 blocks per CU and 2 below 18 (float 256^3 600 us with 8, 657 with
+// 16 and 743 with 32, 200^3 397 with 8 and 380 with 4, 150 x 250 x 80 165, 150 and 138
+// with 8, 4 and 2; double 200^3 706 with 8 and 692 with 4, 100 x 320 x 60 245, 210 and 205).
+// Less where a chunk's buffer would pass 4 GiB.
 int kchunk_of(const cpml_solver *h, bool fused) {
   if (h->kchunk > 0) return h->kchunk;
   const long tiles = (long)((h->nx + 63) / 64) * ((h->ny + h->tile_y - 1) / h->tile_y);
   auto blocks = [&](int k) { return tiles * ((h->nz + k - 1) / k); };
   int k = 8;
-  if (!fused) {
-    if (h->order == 4 && blocks(32) >= 4096) k = 32;
-    while (k > (h->order == 4 ? 4 : 2) && blocks(k) < 1024) k /= 2;
+  if (!fused && h->order == 4) {
+    if (blocks(8) < 24 * 256) k = blocks(4) < 18 * 256 ? 2 : 4;
+  } else if (!fused) {
+    while (k > 2 && blocks(k) < 1024) k /= 2;
   }
   while (k > 1 && !chunk_fits(h, k)) --k;
   return k;

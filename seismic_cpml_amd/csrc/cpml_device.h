@@ -27,10 +27,12 @@ struct Tile3 {
 // FLAT numbers the columns through the TY-row groups of a plane, one group after
 // the other, and cuts them into wavefronts of 64, so that only a plane's last
 // tile has idle lanes; otherwise each group of rows is cut by itself, so that
-// every wavefront but a row's last stores whole cache lines.  Double, order 4,
-// 210 columns: FLAT 2746 us per step, by rows 3020; elsewhere the whole lines
-// count for more (float, order 4: 1505 and 1382; double, order 2, 101 columns:
-// 3068 and 2827).
+// every wavefront but a row's last stores whole cache lines.  Double, order 4: FLAT
+// 3103 us per step at 210 x 800 x 220, by rows 3494; 65 x 300 x 300 578 and 862,
+// 250 x 300 x 280 1680 and 1713, 700 x 500 x 100 2953 and 2912, alike where the
+// columns are whole wavefronts.  Elsewhere the whole lines count for more: float,
+// order 4, 210 x 800 x 220 1592 and 1531, 250 x 300 x 280 854 and 768; double, order 2,
+// 101 columns 3068 and 2827.
 template <bool FLAT>
 inline __host__ __device__ int plane_tiles3(int nx, int ny, int ty) {
   const int groups = (ny + ty - 1) / ty;
