@@ -51,8 +51,11 @@ struct Slab {
   // Element of (i, j) in one plane of an x-slab memory array of `rows` rows:
   // the rows of the min side, then those of the max side, so each side's rows
   // are contiguous (a tile touches one side, and whole cache lines of it).
-  __host__ __device__ long at(int i, long j, long rows) const {
-    return i < wl ? i + wl * j : wl * rows + (i - (n - wr)) + wr * j;
+  __host__ __device__ long at(int i, int j, int rows) const {
+    const bool lo = i < wl;
+    const unsigned pitch = lo ? wl : wr;  // 32 x 32 bits: one multiply-add
+    return (lo ? (long)i : (long)wl * rows + (i - (n - wr))) +
+           (long)((unsigned long)pitch * (unsigned)j);
   }
 };
 

@@ -40,7 +40,7 @@ __device__ __forceinline__ void stress2d_point(const Step2D<T> &p, int i, int j)
   const long ld = p.ld;
   const long c = i + j * ld;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const long mxo = p.sx.at(i, j, p.ny);
+  auto mxo = [&] { return p.sx.at(i, j, p.ny); };  // inside the slab only
   const long myo = i + p.mld * p.sy.s(j);
   // sigma_xx, sigma_yy at (i+1/2, j), Fortran i=1..NX-1, j=2..NY
   if (i <= p.nx - 2 && j >= 1) {
@@ -49,7 +49,7 @@ __device__ __forceinline__ void stress2d_point(const Step2D<T> &p, int i, int j)
     const T lp2m = lhx + T(2) * mhx;
     T dvx_dx = Op<T, ORDER>::d(p.vx, c, 1) / p.den_x;
     T dvy_dy = Op<T, ORDER>::d(p.vy, c - ld, ld) / p.den_y;
-    if (inx) dvx_dx = cpml(dvx_dx, p.mx[0] + mxo, p.px.ah[i], p.px.bh[i], p.px.Kh[i]);
+    if (inx) dvx_dx = cpml(dvx_dx, p.mx[0] + mxo(), p.px.ah[i], p.px.bh[i], p.px.Kh[i]);
     if (iny) dvy_dy = cpml(dvy_dy, p.my[0] + myo, p.py.a[j], p.py.b[j], p.py.K[j]);
     // own-point values (ld_once / st_once: streamed past the L2 when NT)
     st_once<NT>(p.sxx + c, ld_once<NT>(p.sxx + c) + (lp2m * dvx_dx + lhx * dvy_dy) * p.dt);
@@ -60,7 +60,7 @@ __device__ __forceinline__ void stress2d_point(const Step2D<T> &p, int i, int j)
     const T mhy = T(0.5) * (p.mu[c + ld] + p.mu[c]);
     T dvy_dx = Op<T, ORDER>::d(p.vy, c - 1, 1) / p.den_x;
     T dvx_dy = Op<T, ORDER>::d(p.vx, c, ld) / p.den_y;
-    if (inx) dvy_dx = cpml(dvy_dx, p.mx[1] + mxo, p.px.a[i], p.px.b[i], p.px.K[i]);
+    if (inx) dvy_dx = cpml(dvy_dx, p.mx[1] + mxo(), p.px.a[i], p.px.b[i], p.px.K[i]);
     // 2D4:596 divides by K_y(j) where 2D2:595 uses K_y_half(j)
     if (iny)
       dvx_dy = cpml(dvx_dy, p.my[1] + myo, p.py.ah[j], p.py.bh[j],
@@ -77,14 +77,14 @@ __device__ __forceinline__ void velocity2d_point(const Step2D<T> &p, int i, int 
   const long ld = p.ld;
   const long c = i + j * ld;
   const bool inx = p.sx.in(i), iny = p.sy.in(j);
-  const long mxo = p.sx.at(i, j, p.ny);
+  auto mxo = [&] { return p.sx.at(i, j, p.ny); };  // inside the slab only
   const long myo = i + p.mld * p.sy.s(j);
   T vxn = ld_once<NT>(p.vx + c), vyn = ld_once<NT>(p.vy + c);
   // vx at (i, j), Fortran i=2..NX, j=2..NY
   if (i >= 1 && j >= 1) {
     T dsxx_dx = Op<T, ORDER>::d(p.sxx, c - 1, 1) / p.den_x;
     T dsxy_dy = Op<T, ORDER>::d(p.sxy, c - ld, ld) / p.den_y;
-    if (inx) dsxx_dx = cpml(dsxx_dx, p.mx[2] + mxo, p.px.a[i], p.px.b[i], p.px.K[i]);
+    if (inx) dsxx_dx = cpml(dsxx_dx, p.mx[2] + mxo(), p.px.a[i], p.px.b[i], p.px.K[i]);
     if (iny) dsxy_dy = cpml(dsxy_dy, p.my[2] + myo, p.py.a[j], p.py.b[j], p.py.K[j]);
     vxn = vxn + (dsxx_dx + dsxy_dy) * p.dt / p.rho[c];
   }
@@ -93,7 +93,7 @@ __device__ __forceinline__ void velocity2d_point(const Step2D<T> &p, int i, int 
     const T rhh = T(0.25) * (p.rho[c] + p.rho[c + 1] + p.rho[c + 1 + ld] + p.rho[c + ld]);
     T dsxy_dx = Op<T, ORDER>::d(p.sxy, c, 1) / p.den_x;
     T dsyy_dy = Op<T, ORDER>::d(p.syy, c, ld) / p.den_y;
-    if (inx) dsxy_dx = cpml(dsxy_dx, p.mx[3] + mxo, p.px.ah[i], p.px.bh[i], p.px.Kh[i]);
+    if (inx) dsxy_dx = cpml(dsxy_dx, p.mx[3] + mxo(), p.px.ah[i], p.px.bh[i], p.px.Kh[i]);
     if (iny) dsyy_dy = cpml(dsyy_dy, p.my[3] + myo, p.py.ah[j], p.py.bh[j], p.py.Kh[j]);
     vyn = vyn + (dsxy_dx + dsyy_dy) * p.dt / rhh;
   }
