@@ -710,7 +710,8 @@ cpml::EnergyFold<T> fold_of(cpml_solver *h) {
 // Room for the partial sums of the tiles (allocated before any capture).
 int ensure_parts(cpml_solver *h) {
   if (h->cadence == 0) return CPML_OK;
-  const size_t n = 2 * (size_t)(h->prec == 4 ? energy_parts<float>(h) : energy_parts<double>(h));
+  const int parts = h->prec == 4 ? energy_parts<float>(h) : energy_parts<double>(h);
+  const size_t n = 2 * ((size_t)parts + (parts > cpml::kEnergyGroups ? cpml::kEnergyGroups : 0));
   if (n <= h->epart_cap) return CPML_OK;
   HIPCHK(h, hipStreamSynchronize(h->stream));
   dev_free(h, *(void **)&h->epart);
@@ -730,6 +731,18 @@ hipError_t enqueue_energy(cpml_solver *h, int offset) {
   cpml::Energy<T> e = energy_of<T>(h);
   e.offset = offset;
   return cpml::launch_energy_partial<T>(e, h->eblocks, h->stream);
+}
+// Where many partial sums are to be added and nothing runs beside that: their
+// groups first, behind them in epart; p and n then say where and how many.
+template <typename P>
+hipError_t enqueue_groups(cpml_solver *h, int offset, P &p, int &n) {
+  if (n <= cpml::kEnergyGroups) return hipSuccess;
+  double *groups = h->epart + 2 * (size_t)n;
+  const hipError_t e = cpml::launch_energy_groups(h->epart, n, groups, h->step, offset, h->cadence,
+                                                  h->stream);
+  p.partial = groups;
+  n = cpml::kEnergyGroups;
+  return e;
 }
 // Receivers, energy sum and counter of a single step.
 template <typename T>
@@ -768,7 +781,9 @@ hipError_t enqueue_velocity(cpml_solver *h) {
 template <typename T>
 hipError_t enqueue_finish(cpml_solver *h) {
   h->rec_pending = false;
-  return cpml::launch_record<T>(finish_of<T>(h), h->stream);
+  cpml::Record<T> r = finish_of<T>(h);
+  const hipError_t e = enqueue_groups(h, r.skip, r, r.nparts);
+  return e == hipSuccess ? cpml::launch_record<T>(r, h->stream) : e;
 }
 template <typename T>
 hipError_t enqueue_tail(cpml_solver *h) {
@@ -980,8 +995,9 @@ hipError_t enqueue_tb(cpml_solver *h) {
     e = enqueue_energy<T>(h, offset);
     cpml::Energy<T> en = energy_of<T>(h);
     en.offset = offset;
-    if (e == hipSuccess)
-      e = cpml::launch_energy_final<T>(en, energy_parts<T>(h), h->stream);
+    int parts = energy_parts<T>(h);
+    if (e == hipSuccess) e = enqueue_groups(h, offset, en, parts);
+    if (e == hipSuccess) e = cpml::launch_energy_final<T>(en, parts, h->stream);
   }
   ++h->tb_pending;
   return e;

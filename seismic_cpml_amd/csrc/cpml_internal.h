@@ -310,6 +310,12 @@ struct Energy {
   int offset;  // the state is that of step *step + offset (time blocks: NT - 1)
 };
 
+// Partial sums of the energy are added in this many groups.  Where nothing else
+// runs beside their sum (time blocks, the last step of a graph), a launch of that many
+// threads adds each group first: one block alone took 365 us for the 221184 tiles of
+// 768^3, 8 and 6 us so.
+constexpr int kEnergyGroups = 2048;
+
 // Energy of the step that a velocity launch computes: a pair of partial sums per
 // tile, for the steps of the cadence (partial null: off).
 template <typename T>
@@ -425,6 +431,9 @@ hipError_t launch_tb2d_multi(int order, int nt, const TB2D<T> *grids, const int4
                              const int (&n)[4], int waves, int ahead, hipStream_t s);
 template <typename T>
 hipError_t launch_energy_final(const Energy<T> &p, int nparts, hipStream_t s);
+// Sums of the groups of nparts pairs for step *step + offset, if the cadence asks for it
+hipError_t launch_energy_groups(const double *partial, int nparts, double *groups, const int *step,
+                                int offset, int cadence, hipStream_t s);
 template <typename T>
 hipError_t launch_energy_tiles(const Step3D<T> &p, const EnergyFold<T> &ef, int offset,
                                hipStream_t s);

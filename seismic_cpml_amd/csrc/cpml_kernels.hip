@@ -530,6 +530,17 @@ __global__ __launch_bounds__(BX *TY3) void k_energy_tile3d(Step3D<T> p, EnergyFo
   tile_energy<TY3>(ef, blockIdx.x, kin, pot);
 }
 
+__global__ __launch_bounds__(EB) void k_energy_groups(const double *partial, int nparts,
+                                                      double *groups, const int *step, int offset,
+                                                      int cadence) {
+  if ((*step + offset) % cadence != 0) return;
+  const int g = blockIdx.x * EB + threadIdx.x;
+  double kin, pot;
+  group_sum(partial, nparts, g, kin, pot);
+  groups[2 * g] = kin;
+  groups[2 * g + 1] = pot;
+}
+
 template <typename T>
 __global__ __launch_bounds__(EB) void k_energy_final(Energy<T> p, int nblocks) {
   const int it = *p.step + p.offset;
@@ -727,6 +738,13 @@ hipError_t launch_energy_tiles(const Step3D<T> &p, const EnergyFold<T> &ef, int 
   if (ty == 16) hipLaunchKernelGGL((k_energy_tile3d<T, 16>), grid, block, 0, s, p, ef, offset);
   else if (ty == 8) hipLaunchKernelGGL((k_energy_tile3d<T, 8>), grid, block, 0, s, p, ef, offset);
   else hipLaunchKernelGGL((k_energy_tile3d<T, 4>), grid, block, 0, s, p, ef, offset);
+  return hipGetLastError();
+}
+
+hipError_t launch_energy_groups(const double *partial, int nparts, double *groups, const int *step,
+                                int offset, int cadence, hipStream_t s) {
+  hipLaunchKernelGGL(k_energy_groups, dim3(kEnergyGroups / EB), dim3(EB), 0, s, partial, nparts,
+                     groups, step, offset, cadence);
   return hipGetLastError();
 }
 

@@ -36,15 +36,29 @@ __device__ __forceinline__ void block_sum2(int tid, double &a, double &b) {
   b = sb[0];
 }
 
+// Sums of the partial pairs g, g + kEnergyGroups, ...
+__device__ __forceinline__ void group_sum(const double *partial, int nparts, int g, double &kin,
+                                          double &pot) {
+  kin = pot = 0.0;
+#pragma unroll 8
+  for (int b = g; b < nparts; b += kEnergyGroups) {
+    kin += partial[2 * b];
+    pot += partial[2 * b + 1];
+  }
+}
+
 // The kinetic and potential energy of step it from nparts partial sums, by the
-// first 256 threads of a block.
+// first 256 threads of a block, group by group (so that the sums of the groups can
+// be formed by a launch of their own before).
 template <typename E>
 __device__ __forceinline__ void energy_final(const E &e, int tid, int it, int nparts, bool half) {
   double kin = 0.0, pot = 0.0;
   if (tid < 256)
-    for (int b = tid; b < nparts; b += 256) {
-      kin += e.partial[2 * b];
-      pot += e.partial[2 * b + 1];
+    for (int g = tid; g < min(nparts, kEnergyGroups); g += 256) {
+      double a, b;
+      group_sum(e.partial, nparts, g, a, b);
+      kin += a;
+      pot += b;
     }
   block_sum2(tid, kin, pot);
   if (tid == 0) {
