@@ -369,14 +369,29 @@ int stage_rows(cpml_solver *h, bool pack, void *grid_alloc, void *dense, int row
 // two fields: 20.3 -> 3.3 ms).
 // Arrays that the caller has pinned are copied as they are, plane by plane, where
 // the planes are worth a copy each (4096^2 float set in 1.2 ms, through the
-// buffers 2.4; 96 x 80 x 72 through the buffers 0.09).
+// buffers 2.4; 96 x 80 x 72 through the buffers 0.09).  So are arrays in device memory,
+// which the host must not touch, and any array if there is no memory to pin.
 int copy_padded(cpml_solver *h, bool download, void *grid_alloc, char *host) {
   const size_t row = h->nx * h->esize;
+  const int rows = h->ny * (h->ndim == 3 ? h->nz : 1);
+  const size_t bytes = std::clamp(rows * row / 8, kStageMin, kStageMax);
+  const int per = (int)std::clamp<size_t>(bytes / row, 1, rows);
   hipPointerAttribute_t attr{};
-  const bool pinned = hipPointerGetAttributes(&attr, host) == hipSuccess &&
-                      attr.type == hipMemoryTypeHost;
-  (void)hipGetLastError();  // ordinary memory is an error to some runtimes
-  if (pinned && (h->ndim == 2 || row * h->ny >= kStageMin)) {
+  const bool known = hipPointerGetAttributes(&attr, host) == hipSuccess;
+  bool direct = known && (attr.type == hipMemoryTypeDevice ||
+                          (attr.type == hipMemoryTypeHost &&
+                           (h->ndim == 2 || row * h->ny >= kStageMin)));
+  for (int q = 0; q < 2 && !direct; ++q) {
+    if (!h->stage_ev[q])
+      HIPCHK(h, hipEventCreateWithFlags(&h->stage_ev[q], hipEventDisableTiming));
+    if (!h->stage[q] &&
+        hipHostMalloc(&h->stage[q], per * row, hipHostMallocDefault) != hipSuccess) {
+      h->stage[q] = nullptr;
+      direct = true;
+    }
+  }
+  (void)hipGetLastError();  // of pointers that the runtime does not know, and of the pinning
+  if (direct) {
     const size_t gp = h->ld * h->esize, hp = host_x(h) * h->esize;
     for (int k = 0; k < (h->ndim == 3 ? h->nz : 1); ++k) {
       char *g = static_cast<char *>(grid_alloc) + (h->base + k * h->ps) * h->esize;
@@ -388,15 +403,6 @@ int copy_padded(cpml_solver *h, bool download, void *grid_alloc, char *host) {
     }
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return CPML_OK;
-  }
-  const int rows = h->ny * (h->ndim == 3 ? h->nz : 1);
-  const size_t bytes = std::clamp(rows * row / 8, kStageMin, kStageMax);
-  const int per = (int)std::clamp<size_t>(bytes / row, 1, rows);
-  for (int q = 0; q < 2; ++q) {
-    if (!h->stage_ev[q])
-      HIPCHK(h, hipEventCreateWithFlags(&h->stage_ev[q], hipEventDisableTiming));
-    if (!h->stage[q])
-      HIPCHK(h, hipHostMalloc(&h->stage[q], per * row, hipHostMallocDefault));
   }
   auto host_rows = [&](int row0, int n, char *dense) {
     for (int r = 0; r < n; ++r) {
