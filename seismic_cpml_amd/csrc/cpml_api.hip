@@ -2339,17 +2339,10 @@ int cpml_gpu_set_time_block(cpml_solver *h, int steps, int strip_width, int chun
     return fail(h, CPML_ERR_ARG, "strip width must be 0 (default) or 1.." +
                                      std::to_string(64 - 2 * g) + " for this order and step count");
   if (chunk_rows < 0) return fail(h, CPML_ERR_ARG, "chunk rows must be >= 0");
-  // default strip: whole 64-byte sectors of the lanes the ring leaves, so no tile
-  // stores part of one (order 4, 2 steps, float, 64-row chunks of 4096^2: 48
-  // columns 286 us, 52 columns 295; the batch of 32 shots 908 and 967)
-  const int widest = 64 - 2 * g, sector = 64 / (int)h->esize;
-  const int ow = strip_width > 0 ? strip_width
-                                 : (widest >= sector ? widest / sector * sector : widest);
-  int jc = chunk_rows;
-  if (jc == 0)
-    jc = h->ndim == 3 ? cpml::tb3d_default_planes(h->nx, h->ny, h->nz, ow,
-                                                  (h->esize == 4 ? 16 : 8) - 2 * steps)
-                      : cpml::tb2d_default_rows(h->nx, h->ny, ow);
+  const int es = (int)h->esize;
+  const int ow = strip_width > 0 ? strip_width : cpml::tb_default_strip(g, es);
+  int jc = chunk_rows > 0 ? chunk_rows
+                          : cpml::tb_default_chunk(h->ndim, h->nx, h->ny, h->nz, es, steps, ow);
   if (h->ndim == 2) jc = std::min(jc, cpml::tb2d_max_rows(h->ld, h->esize));
   if (chunk_rows == 0)
     while (jc > 1 && !chunk_fits(h, jc)) --jc;
@@ -2391,11 +2384,10 @@ int cpml_gpu_autotune(cpml_solver *h, int trial_steps, int *steps_per_launch, in
   if (blockable) {
     const int nmax = h->ndim == 3 ? cpml::tb3d_max_nt((int)h->esize)
                                   : cpml::tb2d_max_nt(h->order, (int)h->esize);
-    const std::vector<int> depths =
-        h->ndim == 3 ? std::vector<int>{32, 64} : std::vector<int>{16, 24, 40, 64};
     for (int nt = 1; nt <= nmax; ++nt)
       if (h->ndim == 2 || h->cadence == 0 || h->cadence % nt == 0)  // 3D energy: block ends
-        for (int jc : depths)
+        for (int jc : cpml::tb_autotune_chunks(h->ndim, h->nx, h->ny, h->nz, (int)h->esize,
+                                               h->order, nt))
           if (chunk_fits(h, jc)) cands.push_back({nt, jc});
   }
   auto report = [&](int nt, int jc, double ms) {

@@ -1263,10 +1263,7 @@ int cpml_batch_set_time_block(cpml_batch *b, int steps, int strip_width, int chu
     b->cur = 0;
   }
   b->tb = steps;
-  // whole 64-byte sectors of the lanes the ring leaves, as cpml_gpu_set_time_block
-  const int widest = 64 - 2 * g, sector = 64 / b->esize;
-  b->tb_ow = strip_width > 0 ? strip_width
-                             : (widest >= sector ? widest / sector * sector : widest);
+  b->tb_ow = strip_width > 0 ? strip_width : cpml::tb_default_strip(g, (int)b->esize);
   b->tb_jc = chunk_rows > 0 ? chunk_rows : 40;
   for (const Shot &s : b->shots)
     b->tb_jc = std::min(b->tb_jc, cpml::tb2d_max_rows(s.ld, b->esize));

@@ -18,8 +18,10 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
+#include <vector>
 
 #include "../../include/cpml_gpu.h"
 #include "cpml_constdiv.h"
@@ -258,6 +260,31 @@ inline int tb3d_default_planes(int nx, int ny, int nz, int ow, int rows) {
   const double tiles = (double)((nx + ow - 1) / ow) * ((ny + rows - 1) / rows);
   const double planes = tiles * nz / (3.0 * 256.0);
   return planes > 64.0 ? 64 : planes < 8.0 ? 8 : (int)planes;
+}
+
+// Default strip of a time-blocked tile: whole 64-byte sectors of the lanes that the
+// ring of g columns on each side leaves, so no tile stores part of one (order 4, 2
+// steps, float, 64-row chunks of 4096^2: 48 columns 286 us, 52 columns 295; the batch
+// of 32 shots 908 and 967).
+inline int tb_default_strip(int g, int esize) {
+  const int widest = 64 - 2 * g, sector = 64 / esize;
+  return widest >= sector ? widest / sector * sector : widest;
+}
+// Default chunk (2D: rows, 3D: planes) of time blocks of `steps` steps in strips of ow.
+inline int tb_default_chunk(int ndim, int nx, int ny, int nz, int esize, int steps, int ow) {
+  return ndim == 3 ? tb3d_default_planes(nx, ny, nz, ow, (esize == 4 ? 16 : 8) - 2 * steps)
+                   : tb2d_default_rows(nx, ny, ow);
+}
+// Chunks that the autotuner times for such blocks, shallowest first: the default
+// among them, so that it never ends with a slower shape than the default.
+inline std::vector<int> tb_autotune_chunks(int ndim, int nx, int ny, int nz, int esize, int order,
+                                           int steps) {
+  std::vector<int> c = ndim == 3 ? std::vector<int>{8, 16, 32, 64} : std::vector<int>{16, 24, 40, 64};
+  c.push_back(tb_default_chunk(ndim, nx, ny, nz, esize, steps,
+                               tb_default_strip(steps * (order - 1), esize)));
+  std::sort(c.begin(), c.end());
+  c.erase(std::unique(c.begin(), c.end()), c.end());
+  return c;
 }
 
 // Items of one grid by kind: slab-free; of the strips that touch an x slab or
