@@ -165,7 +165,8 @@ int cpml_gpu_set_graph_steps(cpml_solver *h, int steps);
  * the grid and the order) and rows of 64 points per
  * tile (4, 8 or 16; default 4; 2D also 32 or 64, walked by 16-row blocks; the
  * fused 3D step owns 62-point rows, 6 of them per block for 4 or 8 and 14 for
- * 16).  Results do not depend on either. */
+ * 16).  Fields, memory variables and seismograms do not depend on either; the
+ * energy curve, whose terms are summed by tiles, agrees to the rounding of its sums. */
 int cpml_gpu_set_kchunk(cpml_solver *h, int kchunk);
 int cpml_gpu_set_tile(cpml_solver *h, int tile_y);
 /* 3D only: run each time step as ONE fused kernel (stress and velocity in a
