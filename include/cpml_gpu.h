@@ -161,11 +161,11 @@ int cpml_velocity_norm_noalloc(int prec, int ndim, int NX, int NY, int NZ, const
 
 /* Steps captured per HIP graph replay (default 16; 0 = launch eagerly). */
 int cpml_gpu_set_graph_steps(cpml_solver *h, int steps);
-/* Tiling: planes per block along z (3D; default 2 to 32 by
- * the grid and the order) and rows of 64 points per
- * tile (4, 8 or 16; default 4; 2D also 32 or 64, walked by 16-row blocks; the
- * fused 3D step owns 62-point rows, 6 of them per block for 4 or 8 and 14 for
- * 16).  Fields, memory variables and seismograms do not depend on either; the
+/* Tiling: planes per block along z (3D; default 2 to 8 by the grid and the order)
+ * and rows of 64 points per tile (4, 8 or 16; default 4; 2D also 32 or 64, walked by
+ * 16-row blocks; the two-phase 3D steps in double take 16 as 8, since blocks of 16
+ * wavefronts leave them too few registers; the fused 3D step owns 62-point rows, 6 of
+ * them per block for 4 or 8 and 14 for 16).  Fields, memory variables and seismograms do not depend on either; the
  * energy curve, whose terms are summed by tiles, agrees to the rounding of its sums. */
 int cpml_gpu_set_kchunk(cpml_solver *h, int kchunk);
 int cpml_gpu_set_tile(cpml_solver *h, int tile_y);
