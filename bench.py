@@ -542,19 +542,14 @@ def bench_ade8(args):
     # copy and first stage state 20; per stage velocity rates 6, stress
     # rates 7, accumulation with the next stage's state 25 (the last one 15)
     words = 20 + 4 * (6 + 7) + 3 * 25 + 15
-    # this build's own compulsory words (X ping-pongs, no copy): stage 1
-    # reads X0 5 (its state) and media 3 and writes X 5 and the next state
-    # 5; stages 2-3 read the state 5, media 3, X 5, X0 5 and write X 5 and the
-    # next state 5; stage 4 reads 13 and writes 5 (band memory variables not
-    # counted)
-    own_words = 18 + 2 * 28 + 18
+    own = workloads.ade8_own_bytes(w)  # of the step as it is built
     step_gbs = 4 * words * w.cells / (wall / steps) / 1e9
-    own_gbs = 4 * own_words * w.cells / (wall / steps) / 1e9
+    own_gbs = own / (wall / steps) / 1e9
     config = {
         "workload": f"2D ADE-PML RK4 {n}^2, 8th order (Holberg), NPML 20, 12 seeded layers, "
                     "Ricker 10 Hz at the centre, 256 receivers",
         "grid": [w.nx, w.ny], "npml": w.npml, "deltat": w.dt,
-        "bytes_per_cell_update": 4 * words, "own_bytes_per_cell_update": 4 * own_words,
+        "bytes_per_cell_update": 4 * words, "own_bytes_per_cell_update": round(own / w.cells, 1),
         "step_hbm_gbs": round(step_gbs, 1), "step_hbm_frac": round(step_gbs / HBM_PEAK_GBS, 4),
         "launches_per_step": 4,
     }
@@ -562,7 +557,7 @@ def bench_ade8(args):
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(step_gbs / HBM_PEAK_GBS, 4),
             "traffic": None, "algorithmic_bytes": 4 * words * w.cells,
             "bytes_model": "the program's array structure (rates stored between phases)",
-            "own_algorithmic_bytes": 4 * own_words * w.cells, "own_achieved": round(own_gbs, 1),
+            "own_algorithmic_bytes": own, "own_achieved": round(own_gbs, 1),
             "own_frac": round(own_gbs / HBM_PEAK_GBS, 4)}
     cpu = None if args.no_cpu_baseline else cpu_baseline_ade8(w, tab, seconds=args.cpu_seconds)
     return _line("Gcell-updates/s (2D 4096^2 ADE-PML RK4 8th-order FP32 time loop)", value, args,

@@ -236,6 +236,30 @@ def bytes_per_step(w: Workload, slabs, fused: bool = False, nsls: int = 0,
     return {"stress": stress, "velocity": vel, "step": stress + vel}
 
 
+def ade8_pair_box(nx, ny, npml, prec):
+    """Points [x0, x1) x [y0, y1) whose Runge-Kutta stages the ADE-RK4 step takes two
+    per pass (ade_pair_box of csrc/cpml_ade8_split.h); zeros: none."""
+    lo, sector = max(npml + 6, 9), 64 // prec
+    x0, x1 = -(-lo // sector) * sector, min(nx - npml - 7, nx - 9)
+    y0, y1 = lo, min(ny - npml - 7, ny - 9)
+    if x1 - x0 < 64 or y1 - y0 < 64 or (x1 - x0) * (y1 - y0) * prec < 4e6:
+        return 0, 0, 0, 0
+    return x0, x1, y0, y1
+
+
+def ade8_own_bytes(w: Workload) -> int:
+    """Bytes that the ADE-RK4 step cannot do without as it is built, per step, every
+    array touched once per pass (band memory variables not counted).  Stage by
+    stage (the frame): stage 1 reads X0 5 and media 3 and writes X 5 and the next
+    state 5; stages 2-3 read the state 5, media 3, X 5, X0 5 and write X 5 and the
+    next state 5; stage 4 reads 13 and writes 5 -- 92 words.
+    Two stages per pass (the box): 1-2 read X0 5 and media 3 and write X 5 and the
+    next state 5; 3-4 read the state 5, media 3, X 5 and X0 5 and write X 5 -- 41."""
+    x0, x1, y0, y1 = ade8_pair_box(w.nx, w.ny, w.npml, w.prec)
+    box = (x1 - x0) * (y1 - y0)
+    return w.prec * (41 * box + (18 + 2 * 28 + 18) * (w.cells - box))
+
+
 @dataclass
 class BatchWorkload:
     """Per-shot inputs of a batched 2D run (host arrays)."""
