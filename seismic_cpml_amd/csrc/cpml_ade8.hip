@@ -58,10 +58,15 @@ __device__ __forceinline__ bool frame_point(const AdeFrame &f, int h, int &i, in
   return tile_point(b, t, i, j);
 }
 
-// (c1 d1 + c2 d2 + c3 d3 + c4 d4) / delta, ADE8:263-266, 720-723
+// c1 d1 + c2 d2 + c3 d3 + c4 d4, ADE8:263-266
+template <typename T>
+__device__ __forceinline__ T sum8(T d1, T d2, T d3, T d4) {
+  return ((T(kHolberg1) * d1 + T(kHolberg2) * d2) + T(kHolberg3) * d3) + T(kHolberg4) * d4;
+}
+// the same over delta, ADE8:720-723
 template <typename T>
 __device__ __forceinline__ T h8(T d1, T d2, T d3, T d4, T del) {
-  return (((T(kHolberg1) * d1 + T(kHolberg2) * d2) + T(kHolberg3) * d3) + T(kHolberg4) * d4) / del;
+  return sum8(d1, d2, d3, d4) / del;
 }
 
 template <typename T>
@@ -236,10 +241,6 @@ struct AdeMedia {
 
 // 8th-order sums along x of f at this lane: between columns i - 1 and i (back) and
 // between i and i + 1 (forward).
-template <typename T>
-__device__ __forceinline__ T sum8(T d1, T d2, T d3, T d4) {
-  return ((T(kHolberg1) * d1 + T(kHolberg2) * d2) + T(kHolberg3) * d3) + T(kHolberg4) * d4;
-}
 template <typename T>
 __device__ __forceinline__ T x_back(T f) {
   const T m1 = lane_prev(f), m2 = lane_prev(m1), m3 = lane_prev(m2), m4 = lane_prev(m3);

@@ -97,7 +97,7 @@ __device__ __forceinline__ void const_divide(T &a, const ConstDiv<T> &A, T &b,
     a = qa, b = qb, c = qc, d = qd;
   }
 }
-// The same of up to three numbers and one divisor.
+// The same of three numbers and one divisor.
 template <typename T>
 __device__ __forceinline__ void const_divide(const ConstDiv<T> &D, T &a, T &b, T &c) {
   const T m = fmax(fmax(fabs(a), fabs(b)), fabs(c));
@@ -110,11 +110,6 @@ __device__ __forceinline__ void const_divide(const ConstDiv<T> &D, T &a, T &b, T
   } else {
     a = qa, b = qb, c = qc;
   }
-}
-template <typename T>
-__device__ __forceinline__ void const_divide(const ConstDiv<T> &D, T &a, T &b) {
-  T c = b;
-  const_divide(D, a, c, b);
 }
 #endif
 

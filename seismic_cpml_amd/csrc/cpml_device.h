@@ -144,6 +144,18 @@ __device__ __forceinline__ int first_from(const int *a, int lo, int hi, int v) {
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
+// psi <- b*psi + a*d ; d <- d/K + psi in an absorbing slab, with the old psi
+// given and the new one returned through `out`.  k1: K is 1 all along the axis,
+// so d / K == d; K: where to read it otherwise.
+template <typename T>
+__device__ __forceinline__ T pml(bool slab, bool k1, T d, T old, T &out, T a, T b, const T *K) {
+  out = old;
+  if (!slab) return d;
+  out = b * old + a * d;
+  if (!k1) d = over_k(d, *K);
+  return d + out;
+}
+
 // Loads and stores through a scalar base and a 32-bit byte offset of the lane
 // (explicitly global memory: the batch reads the bases from a table, where the
 // compiler would otherwise emit flat accesses).
@@ -158,6 +170,21 @@ template <typename T>
 __device__ __forceinline__ void st_at(T *base, unsigned byte_off, T x) {
   *reinterpret_cast<Glb<T> *>(reinterpret_cast<Glb<char> *>((Glb<T> *)base) + byte_off) = x;
 }
+
+// The same store streamed past the caches: state that the next launch reads a
+// whole grid later.  (Memory variables, whose rows are shorter than a cache line, merge
+// in the L2 and take st_at.)
+template <typename T>
+__device__ __forceinline__ void st_stream_at(T *base, unsigned byte_off, T x) {
+  __builtin_nontemporal_store(
+      x, reinterpret_cast<Glb<T> *>(reinterpret_cast<Glb<char> *>((Glb<T> *)base) + byte_off));
+}
+
+// A number as a type, for phases and levels that the compiler has to know.
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
 
 // Raw buffer resource over `bytes` bytes at p (gfx9 family word 3).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, unsigned bytes) {

@@ -545,7 +545,7 @@ template <typename T>
 __global__ __launch_bounds__(EB) void k_energy_final(Energy<T> p, int nblocks) {
   const int it = *p.step + p.offset;
   if (it % p.cadence != 0) return;
-  energy_final(p, threadIdx.x, it, nblocks, p.ndim == 2);
+  energy_final(p, threadIdx.x, it, nblocks, false);
 }
 
 // ------------------------------------------------- max |v| (stability) --

@@ -53,18 +53,6 @@
 namespace cpml {
 namespace {
 
-// psi <- b*psi + a*d ; d <- d/K + psi in an absorbing slab, with the old psi
-// given and the new one returned through `out`.  k1: K is 1 all along the axis,
-// so d / K == d; K: where to read it otherwise.
-template <typename T>
-__device__ __forceinline__ T pml(bool slab, bool k1, T d, T old, T &out, T a, T b, const T *K) {
-  out = old;
-  if (!slab) return d;
-  out = b * old + a * d;
-  if (!k1) d = over_k(d, *K);
-  return d + out;
-}
-
 // The description of the grid an item works on, in memory that no kernel
 // writes while it runs: the kernel's argument block, or one entry of the
 // batch's table.
@@ -89,11 +77,6 @@ __device__ __forceinline__ ConstDiv<T> div_copy(
   o.d = s.d, o.c = s.c, o.cl = s.cl, o.ch = s.ch, o.hi = s.hi, o.lo = s.lo;
   return o;
 }
-
-template <int V>
-struct Int {
-  static constexpr int value = V;
-};
 
 template <typename T>
 __device__ __forceinline__ T ld_el(const T *base, long element) {
@@ -212,10 +195,9 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
   // 4) and as many moves per row.
   T *const dl = delay + lane;
   auto coef = [&](int q, int pos) -> T & { return dl[(q * DC + pos) * 64]; };
-  auto memx = [&](int m, int q, int pos) -> T & {
+  auto slab_mem = [&](int m, int q, int pos) -> T & {
     return dl[(5 * DC + ((m - 1) * 4 + q) * DM + pos) * 64];
   };
-  auto memy = [&](int m, int q, int pos) -> T & { return memx(m, q, pos); };
   // corner items (both slabs): their y memory variables wait in registers, so
   // that all classes fit the same LDS
   T wy[NL][4][DM];
@@ -228,7 +210,7 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
         for (int k = 0; k < DM; ++k) wy[m][q][k] = T(0);
   auto old_y = [&](int m, int q, int pos) -> T {
     if constexpr (SX) return wy[m - 1][q][0];
-    else return memy(m, q, pos);
+    else return slab_mem(m, q, pos);
   };
   for (int q = 0; q < tb2d_delay_words<ORDER, NT, CLS>(); ++q) dl[q * 64] = T(1);
   int pc = 0, pm = 0;   // this row's places in the rings (DC and DM rows long)
@@ -380,7 +362,7 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
       T syy = m == 1 ? nyy : S[mb][1][wi(0)];
       T sxy = m == 1 ? nxy : S[mb][2][wi(0)];
       T ox0 = lx[0], ox1 = lx[1], oy0 = ly[0], oy1 = ly[1];
-      if (SX && m > 1) ox0 = memx(m - 1, 0, pm), ox1 = memx(m - 1, 1, pm);
+      if (SX && m > 1) ox0 = slab_mem(m - 1, 0, pm), ox1 = slab_mem(m - 1, 1, pm);
       if (SY && m > 1) oy0 = old_y(m - 1, 0, pm), oy1 = old_y(m - 1, 1, pm);
       T npx0 = ox0, npx1 = ox1, npy0 = oy0, npy1 = oy1;
       {
@@ -446,7 +428,7 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
       // ---------------- v^m at row qr: 2D2:606-680 (2D4:607-681)
       T vxn = V[m - 1][0][wi(0)], vyn = V[m - 1][1][wi(0)];
       T ox2 = lx[2], ox3 = lx[3], oy2 = ly[2], oy3 = ly[3];
-      if (SX && m > 1) ox2 = memx(m - 1, 2, pm), ox3 = memx(m - 1, 3, pm);
+      if (SX && m > 1) ox2 = slab_mem(m - 1, 2, pm), ox3 = slab_mem(m - 1, 3, pm);
       if (SY && m > 1) oy2 = old_y(m - 1, 2, pm), oy3 = old_y(m - 1, 3, pm);
       T npx2 = ox2, npx3 = ox3, npy2 = oy2, npy3 = oy3;
       const T rho = cf[m - 1][3], rhh = cf[m - 1][4];
@@ -538,13 +520,13 @@ __device__ __forceinline__ void tb2d_item(GridPtr<T> P, int ts, int jb, int je, 
       for (int m = 1; m < NT; ++m)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          if (SX) memx(m, q, pm) = px[m - 1][q];
+          if (SX) slab_mem(m, q, pm) = px[m - 1][q];
           if constexpr (SX && SY) {
 #pragma unroll
             for (int k = 0; k < DM - 1; ++k) wy[m - 1][q][k] = wy[m - 1][q][k + 1];
             wy[m - 1][q][DM - 1] = py[m - 1][q];
           } else if (SY) {
-            memy(m, q, pm) = py[m - 1][q];
+            slab_mem(m, q, pm) = py[m - 1][q];
           }
         }
     }

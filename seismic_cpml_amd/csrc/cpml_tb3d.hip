@@ -39,46 +39,12 @@
 namespace cpml {
 namespace {
 
-// psi <- b*psi + a*d ; d <- d/K + psi (old psi given, new one in `out`) where
-// `slab`: the point lies in this axis' slab.  k1: K is 1 all along the axis, so
-// d / K == d; K: where to read it otherwise.
-template <typename T>
-__device__ __forceinline__ T pml(bool slab, bool k1, T d, T old, T &out, T a, T b, const T *K) {
-  out = old;
-  if (!slab) return d;
-  out = b * old + a * d;
-  if (!k1) d = over_k(d, *K);
-  return d + out;
-}
-
 // Plane slot of a 3-plane window in the iteration of phase PH (the march is
 // unrolled by 3, so slots are compile-time constants and no window moves).
 template <int PH, int K>
 constexpr int slot_of() {
   return ((PH + K) % 3 + 3) % 3;
 }
-template <int V>
-struct Int {
-  static constexpr int value = V;
-};
-
-template <typename T>
-__device__ __forceinline__ T ld_at(const T *base, unsigned byte_off) {
-  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + byte_off);
-}
-// State stores are streamed past the caches (the next launch reads them a
-// whole grid later); those of the memory variables, whose rows are shorter
-// than a cache line, merge in the L2.
-template <typename T>
-__device__ __forceinline__ void st_at(T *base, unsigned byte_off, T x) {
-  __builtin_nontemporal_store(x,
-                              reinterpret_cast<T *>(reinterpret_cast<char *>(base) + byte_off));
-}
-template <typename T>
-__device__ __forceinline__ void st_mem(T *base, unsigned byte_off, T x) {
-  *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + byte_off) = x;
-}
-
 // What bounds the march (float, 2 steps, 768^3, milliseconds per launch; boxes
 // differ by a few percent, pairs are from one box):
 //  * stores of part of a cache line.  A copy of 12 arrays read and 9 written
@@ -357,22 +323,22 @@ __device__ __forceinline__ void tb3d_tile(const TB3D<T> &P, int t, T *xl) {
       wr[(ss + 2) * SLOT] = sn[1];
       if (m == NT && pk >= kb && pk < ke && own) {
         const unsigned o = pl(pk);
-        st_at(P.sxx + corner, o, sn[0]);
-        st_at(P.syy + corner, o, sn[1]);
-        st_at(P.szz + corner, o, sn[2]);
-        st_at(P.sxy + corner, o, sn[3]);
-        st_at(P.sxz + corner, o, sn[4]);
-        st_at(P.syz + corner, o, sn[5]);
+        st_stream_at(P.sxx + corner, o, sn[0]);
+        st_stream_at(P.syy + corner, o, sn[1]);
+        st_stream_at(P.szz + corner, o, sn[2]);
+        st_stream_at(P.sxy + corner, o, sn[3]);
+        st_stream_at(P.sxz + corner, o, sn[4]);
+        st_stream_at(P.syz + corner, o, sn[5]);
         const KArgs Q = args();
         if (SX && inx)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) st_mem(Q->mx[f] + mxs * pk, mxo, nm[f]);
+          for (int f = 0; f < 3; ++f) st_at(Q->mx[f] + mxs * pk, mxo, nm[f]);
         if (SY && iny)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) st_mem(Q->my[f] + mys * pk, myo, nm[3 + f]);
+          for (int f = 0; f < 3; ++f) st_at(Q->my[f] + mys * pk, myo, nm[3 + f]);
         if (SZ && p.sz.in(pk))
 #pragma unroll
-          for (int f = 0; f < 3; ++f) st_mem(Q->mz[f] + mzs * p.sz.s(pk), mzo, nm[6 + f]);
+          for (int f = 0; f < 3; ++f) st_at(Q->mz[f] + mzs * p.sz.s(pk), mzo, nm[6 + f]);
       }
       if (m == 1 && s < s1) {  // sigma and the coefficients of the next plane
         load_s(s + 1);
@@ -478,19 +444,19 @@ __device__ __forceinline__ void tb3d_tile(const TB3D<T> &P, int t, T *xl) {
         wr[(ss + 5) * SLOT] = vn[2];
       } else if (qk >= kb && qk < ke && own) {
         const unsigned o = pl(qk);
-        st_at(P.vx + corner, o, vn[0]);
-        st_at(P.vy + corner, o, vn[1]);
-        st_at(P.vz + corner, o, vn[2]);
+        st_stream_at(P.vx + corner, o, vn[0]);
+        st_stream_at(P.vy + corner, o, vn[1]);
+        st_stream_at(P.vz + corner, o, vn[2]);
         const KArgs Q = args();
         if (SX && inx)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) st_mem(Q->mx[3 + f] + mxs * qk, mxo, nv[f]);
+          for (int f = 0; f < 3; ++f) st_at(Q->mx[3 + f] + mxs * qk, mxo, nv[f]);
         if (SY && iny)
 #pragma unroll
-          for (int f = 0; f < 3; ++f) st_mem(Q->my[3 + f] + mys * qk, myo, nv[3 + f]);
+          for (int f = 0; f < 3; ++f) st_at(Q->my[3 + f] + mys * qk, myo, nv[3 + f]);
         if (SZ && p.sz.in(qk))
 #pragma unroll
-          for (int f = 0; f < 3; ++f) st_mem(Q->mz[3 + f] + mzs * p.sz.s(qk), mzo, nv[6 + f]);
+          for (int f = 0; f < 3; ++f) st_at(Q->mz[3 + f] + mzs * p.sz.s(qk), mzo, nv[6 + f]);
       }
       if (m == 1 && s < s1) {  // v of the plane after the next, buoyancy of this one
         load_v(s + 2);
