@@ -149,9 +149,8 @@ struct cpml_solver {
   void *field2[9] = {}; // second state buffer of the fused 3D step
   int cur = 0;          // 1: the state lives in field2 / mem2
   bool fused = false;   // 3D: one fused kernel per step (ping-pong state)
-  // 2D time blocking: tb steps per launch (0: off), strips of tb_ow columns
-  // (0: every lane the ring leaves; 3D: a multiple of 8), chunks of tb_jc rows
-  // (2D items with C-PML code: tb_js)
+  // time blocking: tb steps per launch (0: off), strips of tb_ow columns, chunks of
+  // tb_jc rows (3D: planes; 2D items with C-PML code: tb_js rows)
   int tb = 0, tb_ow = 0, tb_jc = 40, tb_js = 16;
   int *tb_rec = nullptr;        // per-strip receiver lists (device)
   bool rec_pending = false;     // a single step whose receivers are not recorded yet

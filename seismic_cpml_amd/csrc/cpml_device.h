@@ -94,7 +94,7 @@ __device__ __forceinline__ T cpml2(T d, const T *psi_old, T *psi_new, T a, T b, 
   return over_k(d, K) + m;
 }
 
-// The kernel's only argument, read through the kernel-argument segment with a
+// The kernel's first argument, read through the kernel-argument segment with a
 // pointer the compiler cannot prove loop-invariant.  Kernels whose argument
 // block holds more pointers than fit in scalar registers re-read the ones
 // they need inside their z loop (scalar loads, cached) instead of keeping

@@ -140,8 +140,8 @@ constexpr int tb2d_delay_words() {
 // The march is bound by instruction issue (4096^2, order 4, 2 steps per
 // launch, float: 600 vector instructions per row before, 121 of them IEEE
 // divisions by 24 DELTA and density and 129 register moves).  So: division by
-// the launch constants in 6 instructions (cpml_constdiv.h); 27 f formed once
-// per value and carried to the next row; half-point coefficients formed once
+// the launch constants in 4 instructions and a range test (cpml_constdiv.h); 27 f
+// formed once per value and carried to the next row; half-point coefficients formed once
 // and carried to the later levels; x neighbours by DPP, folded into the
 // arithmetic; no predicates along an axis whose slabs and faces the class
 // does not touch; unconditional loads (coordinates clamped to the zero ghost
