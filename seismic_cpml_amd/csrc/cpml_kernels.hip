@@ -71,20 +71,22 @@ __device__ __forceinline__ void tile_energy(const EnergyFold<T> &ef, int tile, d
   }
 }
 
-// Waves per SIMD the 2D kernels are built for: all that the vector registers leave
-// room for.  Without the bound they take more than 80 scalar registers, and the
-// SIMD holds 7 waves instead of 8 and half as many blocks of 16: at 2900^2 float
-// in 64-row tiles 190 us per step and 149 with it, with the energy curve 217 and 169 (16
-// rows 225 and 183); double 280 and 260.
-template <typename T, int ORDER>
+// Waves per SIMD the 2D kernels in blocks of 16 wavefronts are built for: all that
+// the vector registers leave room for.  Without the bound they take more than 80 scalar
+// registers, and the SIMD holds 7 waves instead of 8 and half as many of these blocks:
+// at 2900^2 float in 64-row tiles 190 us per step and 149 with it, with the energy
+// curve 217 and 169 (16 rows 225 and 183); double 280 and 260.  Smaller blocks lose
+// nothing to speak of, and small grids would pay for the spilled scalars (300 x 200 with
+// the curve 8.5 us per step and 8.8).
+template <typename T, int ORDER, int TY>
 constexpr int min_waves2d() {
-  return sizeof(T) == 4 || ORDER < 8 ? 8 : 1;
+  return TY == 16 && (sizeof(T) == 4 || ORDER < 8) ? 8 : 1;
 }
 
 // A tile is 64 points by TY*RG rows; the block (64 x TY threads) walks its RG
 // row groups, so each wavefront lives for several rows.
 template <typename T, int ORDER, int TY, int RG, bool NT>
-__global__ __launch_bounds__(BX *TY, (min_waves2d<T, ORDER>())) void k_stress2d(Step2D<T> p, Record<T> prev, int lead) {
+__global__ __launch_bounds__(BX *TY, (min_waves2d<T, ORDER, TY>())) void k_stress2d(Step2D<T> p, Record<T> prev, int lead) {
   int h, i, j;
   if (lead_block(prev, lead, h)) return;
   tile2d<TY, RG>(h, p.nx, p.ny, i, j);
@@ -96,7 +98,7 @@ __global__ __launch_bounds__(BX *TY, (min_waves2d<T, ORDER>())) void k_stress2d(
 // EN: the energy of the points it computes, summed over the tile.  Steps without it
 // have a kernel without its registers: 4096^2 float 137 -> 125 us.
 template <typename T, int ORDER, int TY, int RG, bool NT, bool EN>
-__global__ __launch_bounds__(BX *TY, (min_waves2d<T, ORDER>())) void k_velocity2d(Step2D<T> p, EnergyFold<T> ef) {
+__global__ __launch_bounds__(BX *TY, (min_waves2d<T, ORDER, TY>())) void k_velocity2d(Step2D<T> p, EnergyFold<T> ef) {
   int i, j;
   tile2d<TY, RG>(blockIdx.x, p.nx, p.ny, i, j);
   const bool en = EN && *p.step % ef.cadence == 0;
